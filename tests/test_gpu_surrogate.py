@@ -180,6 +180,33 @@ def test_training_gradient_vs_oracle(orc, gpu_engine_factory):
             assert np.linalg.norm(g[a:b] - go[a:b]) <= 3e-2 * np.linalg.norm(go[a:b]) + 1e-6, (a, b)
 
 
+@pytest.mark.parametrize("bsize", [1, 15, 17, 1000, 4096, 4320])
+def test_training_gradient_tile_remainders(orc, gpu_engine_factory, bsize):
+    """Batches that end inside a 16-sample tile, that fill fewer tiles than
+    the partial rows (256) and that need a second tile per workgroup: the
+    summed gradient and loss against FP64.  Bound: BF16 operands (2^-9 each)
+    through four products, as in the test above; a single sample has no
+    averaging, so its gradient takes twice that."""
+    say(f"surrogate training gradient, batch {bsize}")
+    box = systems.tip4p2005_box(216, seed=13, min_sep=1.8)
+    e, _ = water_md_engine(gpu_engine_factory, box, np.zeros_like(box["x"]), rc=7.0, skin=1.0,
+                           sz=(32, 32, 32), order=5, e3b=True, dt=1.0)
+    nm, frames = len(box["mol"]), 20
+    p = random_model(2, S.features(S.descriptors(box["mol"], box["x"], box["L"])))
+    e.surrogate_set(p)
+    for k in range(frames):
+        e.surrogate_record(reset=k == 0, capacity=frames * nm)
+    target = np.tile(e.e3b_molecule_energies(nm).astype(np.float64), frames)
+    feat = np.tile(e.surrogate_eval(nm)[1].astype(np.float64), (frames, 1))
+    g = e.surrogate_grad(5, bsize, 11, 4)
+    rows = ((5 + np.arange(bsize)) * 11 + 4) % (nm * frames)
+    lo, go = S.loss_grad(p.astype(np.float64), feat[rows], target[rows])
+    rel = np.linalg.norm(g[:-1] - go) / np.linalg.norm(go)
+    say(f"loss {g[-1]:.5f} vs {lo:.5f}, gradient rel err {rel:.2e}")
+    assert g[-1] == pytest.approx(lo, rel=4e-2 if bsize < 16 else 2e-2)
+    assert rel < (4e-2 if bsize < 16 else 2e-2)
+
+
 @pytest.mark.parametrize("graph", [0, 1])
 def test_e3b_judge_and_fallback(orc, gpu_engine_factory, graph):
     """E3B judges the learned term every 100 steps: the checks are counted,
