@@ -402,7 +402,10 @@ void captured_step(Ctx &c, int fflags) {
     const bool allRigid = c.rigid.on && c.rigid.nsites == c.n && !c.nh.on;
     c.fuseMolVirial = c.baro.on && allRigid;
     c.fuseThermo = c.thermoOn && allRigid;
-    c.fuseCheck = c.rigid.on && c.rigid.nsites == c.n;
+    // all-rigid systems and free atoms: the first half refreshes the positions
+    // of the force evaluation and measures the displacements for the binning
+    // (flexible molecules place their M sites between the drift and the refresh)
+    c.fuseCheck = c.fuseStep && !c.flex.on && (!c.rigid.on || c.rigid.nsites == c.n);
     integrate_first_half(c);
     decide_step(c);
     nlist_rebuild_async(c);  // every kernel gated by dFlags[3]
@@ -1032,6 +1035,7 @@ void run_captured(const std::vector<Ctx *> &cs, int nsteps, int flags, const Rin
                 }
                 // chunk state: displacement slots, running row maxima, counters, turn
                 fill_int(c, (int *)c.dMax, 4, 0);
+                fill_int(c, (int *)c.dispSlots, kDispSlots * kDispStride, 0);
                 fill_int(c, c.dFlags + 1, 5, 0);
                 // device turn counter: the thermostat and barostat gates take it
                 // modulo their intervals
@@ -1308,6 +1312,7 @@ int mdx_create(int device, mdx_ctx **out) {
         c.acc = dalloc<unsigned long long>(c, kAccTotal);
         c.dFlags = dalloc<int>(c, 12);
         c.dMax = dalloc<unsigned>(c, 4);
+        c.dispSlots = dalloc<unsigned>(c, kDispSlots * kDispStride);
         c.checkPart = dalloc<float>(c, 2 * kCheckBlocks);
         c.thermo = dalloc<unsigned long long>(c, 2);
         MDX_HIP(hipHostMalloc((void **)&c.pinned, sizeof(int) * 8, hipHostMallocDefault));

@@ -38,9 +38,8 @@ __device__ __forceinline__ void fadd(unsigned long long *f, int i, v3 v) {
     fx_add(&f[3 * i + 2], v.z);
 }
 
-__device__ __forceinline__ void flex_map_body(int blk, int nblk, const int *__restrict__ gate, int nmol, const int4 *__restrict__ ids,
+__device__ __forceinline__ void flex_map_body(int blk, int nblk, int nmol, const int4 *__restrict__ ids,
                            const int *__restrict__ idToIdx, int4 *__restrict__ atoms) {
-    if (gate && *gate == 0) return;
     const int m = blk * blockDim.x + threadIdx.x;
     if (m >= nmol) return;
     const int4 d = ids[m];
@@ -167,9 +166,10 @@ FlexArgs make_args(const Ctx &c) {
 
 }  // namespace
 
+// the map of a new set-up (list rebuilds map the molecules in the build's launch)
 void flex_map(Ctx &c) {
     if (!c.flex.on) return;
-    launch<flex_map_body, 256>(c, cdiv(c.flex.nmol, 256), 0, rebuild_gate(c), c.flex.nmol, c.flex.ids, c.idToIdx, c.flex.atoms);
+    launch<flex_map_body, 256>(c, cdiv(c.flex.nmol, 256), 0, c.flex.nmol, c.flex.ids, c.idToIdx, c.flex.atoms);
 }
 
 void flex_place_m(Ctx &c) {

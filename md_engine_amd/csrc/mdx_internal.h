@@ -453,7 +453,7 @@ struct Ctx {
     bool vtrace = false;  // set by compute for the terms it launches
     bool fuseMolVirial = false;  // captured barostat steps: rigid second half sums ACC_MOL
     bool fuseThermo = false;     // captured thermostat steps: rigid second half sums m v^2
-    bool fuseCheck = false;      // captured steps: rigid first half gives the skin check's maxima
+    bool fuseCheck = false;      // captured steps: the first half gives the skin check's maxima, the binning decides
     bool deferMSpread = false;   // compute leaves the M-site forces for a later flex_spread_m (ring contraction)
     hipStream_t stream = nullptr;
     // second stream of captured steps: the P3M chain runs beside the pair and
@@ -478,7 +478,7 @@ struct Ctx {
     unsigned long long *force = nullptr;   // 3 per atom
     unsigned long long *acc = nullptr;     // kAccTotal: kAccRep replicas of ACC_N slots
     BoxDev *box = nullptr;                 // device copy of the box-dependent launch data
-    BoxDev *boxLast = nullptr;             // the box of the last list build (copied by k_scan)
+    BoxDev *boxLast = nullptr;             // the box of the last list build (copied by the sort)
     int replayChunk = 0;                   // option replay_chunk: chunk of each run replayed once
     std::vector<LaunchRec> *rec = nullptr; // set while a batch records this context's step launches
     BoxDev boxHost;                        // host mirror (last upload or read-back)
@@ -502,12 +502,13 @@ struct Ctx {
     int reach[3] = {2, 2, 4};
     int ncell = 0;
     int *colRank = nullptr;
-    int *cellCount = nullptr;
     int *cellStart = nullptr;     // 2 ncell + 1: cells of the charged atoms, then of the charge-free ones
-    int *cellFill = nullptr;
-    int *cellOf = nullptr;
-    int *perm = nullptr;
-    int *perm2 = nullptr;
+    // re-sort: per cell slot a list of its atoms (head, -1 when empty; next by
+    // atom), atoms per chunk of slots, and the sort's chunk shape
+    int *cellHead = nullptr;
+    int *cellNext = nullptr;
+    int *chunkSum = nullptr;
+    int nChunk = 0, sortCpw = 32, sortCsh = 5;
     int2 *colXY = nullptr;        // by column rank: cell (x, y)
     int cap = 0;
     uint32_t *nl = nullptr;
@@ -523,13 +524,13 @@ struct Ctx {
     int waveMaxN = 0, waveMaxA = 0, waveMaxB = 0;
     bool capture = false;         // a step is being recorded into a graph
     bool rowMaxPending = false;   // a captured build's row maxima go with the next position refresh
-    bool decided = false;         // the first half kick of this captured step took the step's decisions
     bool refreshed = false;       // ... and refreshed xq, the mesh records, forces and accumulators
     bool forked = false;          // the captured rebuild recorded the mesh stream's fork after its copy-back
     bool baroFused = false;       // the rigid second half of this captured step ran the barostat step
     bool fuseStep = true;         // option "fuse_step": captured steps fold small launches into others
     int graphSteps = 0;           // mdx_run: 1 = captured steps (option "graph")
     unsigned *dMax = nullptr;     // 2 slots x (max |x - x_last|^2, max predicted^2) as float bits
+    unsigned *dispSlots = nullptr; // captured steps: max |x - x_last|^2 as float bits, kDispSlots words a line apart
     float *checkPart = nullptr;   // per-workgroup maxima of the displacement check (2 x kCheckBlocks)
     int *pinned = nullptr;        // host-pinned: [0..1] last build's max counts, [2..5] dMax copies, [6] stream overflow
     hipEvent_t capEvent = nullptr;
@@ -558,7 +559,7 @@ struct Ctx {
     int nExclIds = 0;
     int maxExcl = 0;
     int exclSpan = 0;             // largest |id_i - id_j| over excluded pairs
-    uint32_t *exclIdx = nullptr;  // per atom: maxExcl partners as current index | tag << 30
+    uint32_t *exclIdx = nullptr;  // per atom: maxExcl partners, id | tag << 30 (team builds: index | tag << 30)
     size_t exclIdxN = 0;
 
     // LJ + Ewald real space
@@ -910,12 +911,19 @@ __device__ __forceinline__ int xcd_block(int blk, int nlogical) {
 // largest displacement since the last build exceeds skin/2 (the reference's
 // setBuildFlag test, GridGPU.cu:755-774), count it, and set the thermostat
 // and barostat gates for the steps where the turn reaches a multiple of their
-// intervals; clears the displacement slots for the next step.  The maxima
-// come from nb per-workgroup partials; the first wave of the calling
-// workgroup reduces them and its thread 0 writes.
+// intervals.
+//
+// Where the first half kick measures the displacements, its workgroups fold
+// their maxima into kDispSlots words (a cache line each, so that the atomics
+// of different workgroups do not queue on one address) and every workgroup of
+// the binning reduces the words for itself: no launch and no last-workgroup
+// ticket in between.  A ticket costs about 24 ns a workgroup (its fence and its
+// same-address atomic: 3.5 us for 128 workgroups, 11 us for 512), a launch of
+// its own 1.6 us; this costs one load.  The sort clears the words.
+constexpr int kDispSlots = 32, kDispStride = 16;
 struct DecideArgs {
-    int *ticket;                 // last-workgroup counter when fused into another launch
-    const float *part;
+    const float *part;           // decide_body: per-workgroup maxima
+    unsigned *slots;             // bin_body: the maxima words, nullptr when decide_body took the decisions
     unsigned *dmax;
     int *flags;
     float half2;
@@ -937,13 +945,10 @@ __device__ __forceinline__ void part_max(int nb, const float *__restrict__ part,
     }
 }
 
-__device__ __forceinline__ void decide_wg(int nb, const DecideArgs &d) {
-    if (threadIdx.x >= 64) return;
-    float d2, p2;
-    part_max(nb, d.part, d2, p2);
-    if (threadIdx.x != 0) return;
+// one thread writes the decisions of the step
+__device__ __forceinline__ void decide_write(const DecideArgs &d, bool rebuild) {
     int *flags = d.flags;
-    const int build = d2 > d.half2 ? 1 : 0;
+    const int build = rebuild ? 1 : 0;
     flags[3] = build;
     flags[4] += build;
     const int turn = flags[6] + 1;
@@ -956,6 +961,21 @@ __device__ __forceinline__ void decide_wg(int nb, const DecideArgs &d) {
     flags[8] = (d.baroEvery > 0 && turn % d.baroEvery == 0) ? 1 : 0;
     d.dmax[0] = 0u;
     d.dmax[1] = 0u;
+}
+
+// a workgroup's largest squared displacement (a lane value per thread) into
+// its word: non-negative floats order like their bit patterns
+__device__ __forceinline__ void disp_fold(float d2, unsigned *slots, int blk) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) d2 = fmaxf(d2, __shfl_xor(d2, o, 64));
+    if ((threadIdx.x & 63) == 0)
+        atomicMax(&slots[((blk + (threadIdx.x >> 6)) & (kDispSlots - 1)) * kDispStride], __float_as_uint(d2));
+}
+__device__ __forceinline__ float disp_max(const unsigned *slots) {
+    float d2 = __uint_as_float(slots[(threadIdx.x & (kDispSlots - 1)) * kDispStride]);
+#pragma unroll
+    for (int o = kDispSlots / 2; o > 0; o >>= 1) d2 = fmaxf(d2, __shfl_xor(d2, o, 64));
+    return d2;
 }
 
 // True in the last workgroup of a launch to get here (every thread of every
@@ -974,6 +994,43 @@ __device__ __forceinline__ bool last_block(int *ticket, int nblk) {
     __syncthreads();
     if (last) __threadfence();
     return last != 0;
+}
+
+// squared minimum-image displacement, the expressions and rounding of the
+// list's skin check (dist2 of the neighbor-list code), so that the maxima of a
+// fused check agree with it bit for bit
+__device__ __forceinline__ double disp2(const double4 &a, const double4 &b, const Geometry &g) {
+#pragma clang fp contract(off)
+    double d[3] = {b.x - a.x, b.y - a.y, b.z - a.z};
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        if (g.periodic[k]) {
+            double img = rint(d[k] * g.invL[k]);
+            d[k] = d[k] - img * g.L[k];
+        }
+    return d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+}
+
+// The force evaluation's position refresh done by the first half kick of a
+// captured step (xq != nullptr): FP32 positions, the P3M mesh records of the
+// charged sites (rec != nullptr), cleared force rows and accumulators.
+struct RefreshArgs {
+    float4 *xq;
+    float4 *rec;
+    const float *q;
+    unsigned long long *force;
+    unsigned long long *acc;
+    int nacc;
+};
+RefreshArgs refresh_args(Ctx &c);  // for this context, marking the refresh as done
+__device__ __forceinline__ void refresh_site(const RefreshArgs &ra, int i, const double4 &p, const BoxDev *bx,
+                                             const Geometry &g) {
+    const float qs = ra.q[i];
+    ra.xq[i] = make_float4((float)(p.x - g.lo[0]), (float)(p.y - g.lo[1]), (float)(p.z - g.lo[2]), qs);
+    if (ra.rec && qs != 0.0f) ra.rec[i] = mesh_record(p, bx->mesh);
+    ra.force[3 * (size_t)i + 0] = 0ull;
+    ra.force[3 * (size_t)i + 1] = 0ull;
+    ra.force[3 * (size_t)i + 2] = 0ull;
 }
 
 // maximum over the 64 lanes of a wave (every lane gets it)
@@ -1274,7 +1331,6 @@ void flex_place_m(Ctx &c);
 void flex_forces(Ctx &c, bool energy, bool virial);
 void flex_spread_m(Ctx &c);
 void rigid_second_half(Ctx &c, bool kick);
-int fused_check_blocks(const Ctx &c);  // workgroups of k_rigid_vv1 when it can give the skin check, else 0
 
 // integrate.hip
 void integrate_first_half(Ctx &c);

@@ -63,223 +63,256 @@ __device__ __forceinline__ void check_body(int blk, int nblk, int n, const doubl
     if (__any(move) && (threadIdx.x & 63) == 0) flags[0] = 1;
 }
 
-// Wrap into the box (periodicWrap) and bin into cells (countNumInGridCells).
-// Charged and charge-free atoms go to two copies of the grid (slots
-// [0, ncell) and [ncell, 2 ncell)), so that after the permutation the charged
-// atoms come first, each class sorted by cell: a neighbor row then lists its
-// charged partners first, and the charge spread and gather see only charged
-// atoms.
-__device__ __forceinline__ void bin_atom(int i, double4 *__restrict__ pos, const float *__restrict__ q,
-                                         const BoxDev *__restrict__ bx, int ncell, const int *__restrict__ colRank,
-                                         int *__restrict__ cellOf, int *__restrict__ cellCount,
-                                         const double4 *__restrict__ cen, const int *__restrict__ ids) {
-    const Geometry g = bx->geo;
-    const CellGrid cg = bx->cg;
-    double4 p = pos[i];
-    double *pc = &p.x;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        if (g.periodic[a]) {
-            double img = floor((pc[a] - g.lo[a]) * g.invL[a]);
-            pc[a] = pc[a] - img * g.L[a];
-        }
+// Wrap into the box (periodicWrap) and bin into cells (countNumInGridCells),
+// the first of the two launches of a re-sort.  Charged and charge-free atoms
+// go to two copies of the grid (slots [0, ncell) and [ncell, 2 ncell)), so
+// that after the permutation the charged atoms come first, each class sorted
+// by cell: a neighbor row then lists its charged partners first, and the
+// charge spread and gather see only charged atoms.
+//
+// Each atom is pushed onto its cell's list (head, next) and its records are
+// copied to the scratch arrays pos1 ... id1, from which the second launch
+// gathers them back in the new order: the sorted records end where they were,
+// as the fixed buffers of captured steps need, without a copy-back pass.  The
+// second launch works on chunks of 2^csh cell slots; the atoms of each chunk
+// are counted here, one atomic per chunk and wave (the atoms still lie in the
+// order of the previous build, so a wave meets one or two chunks).
+__device__ __forceinline__ void bin_body(int blk, int nblk, const int *__restrict__ gate, int n,
+                                         const double4 *__restrict__ pos, const double4 *__restrict__ vel,
+                                         const float *__restrict__ q, const int *__restrict__ type,
+                                         const int *__restrict__ id, double4 *__restrict__ pos1,
+                                         double4 *__restrict__ vel1, float *__restrict__ q1, int *__restrict__ type1,
+                                         int *__restrict__ id1, const BoxDev *__restrict__ bx, int ncell,
+                                         const int *__restrict__ colRank, int *__restrict__ head,
+                                         int *__restrict__ next, int *__restrict__ chunkSum, int csh,
+                                         const double4 *__restrict__ cen, DecideArgs da) {
+    if (da.slots) {  // the step's decisions, by every workgroup for itself
+        const bool build = disp_max(da.slots) > da.half2;
+        if (blk == 0 && threadIdx.x == 0) decide_write(da, build);
+        if (!build) return;
+    } else if (gate && *gate == 0) {
+        return;
     }
-    pos[i] = p;
-    // ring centroid lists: the atom goes to the cell of its ring's centroid
-    // (already in the box)
-    if (cen) p = cen[ids[i]];
-    int cx = cell_coord(p.x, g.lo[0], cg.cellInv[0], cg.nc[0]);
-    int cy = cell_coord(p.y, g.lo[1], cg.cellInv[1], cg.nc[1]);
-    int cz = cell_coord(p.z, g.lo[2], cg.cellInv[2], cg.nc[2]);
-    int rank = colRank[cx * cg.nc[1] + cy] * cg.nc[2] + cz + (q[i] == 0.0f ? ncell : 0);
-    cellOf[i] = rank;
-    atomicAdd(&cellCount[rank], 1);
-}
-
-__device__ __forceinline__ void bin_body(int blk, int nblk, const int *__restrict__ gate, int n, double4 *__restrict__ pos, const float *__restrict__ q,
-                      const BoxDev *__restrict__ bx, int ncell, const int *__restrict__ colRank,
-                      int *__restrict__ cellOf, int *__restrict__ cellCount,
-                      const double4 *__restrict__ cen, const int *__restrict__ ids) {
-    if (gate && *gate == 0) return;
-    int i = blk * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    bin_atom(i, pos, q, bx, ncell, colRank, cellOf, cellCount, cen, ids);
-}
-
-// Exclusive scan of the cell counts by one workgroup (replaces the host
-// cumulativeSum round trip, helpers.h:15-24).  Each thread sums a contiguous
-// segment, the segment totals are scanned across the workgroup, and each
-// thread then writes its segment's prefixes.  Also seeds the fill cursors.
-// The counts are cleared as they are consumed, ready for the next binning
-// (no separate clearing launch in every captured step).
-// one workgroup of 1024 threads
-__device__ __forceinline__ void scan_wg(int ncell, int *__restrict__ count, int *__restrict__ start, int *__restrict__ fill,
-                                        const BoxDev *__restrict__ box, BoxDev *__restrict__ boxLast) {
-    // the box this build uses, kept for rebuilding the same list later
-    constexpr int kBoxWords = (int)(sizeof(BoxDev) / sizeof(int));
-    static_assert(sizeof(BoxDev) % sizeof(int) == 0, "BoxDev copied as words");
-    if (boxLast)
-        for (int k = threadIdx.x; k < kBoxWords; k += blockDim.x)
-            reinterpret_cast<int *>(boxLast)[k] = reinterpret_cast<const int *>(box)[k];
-    __shared__ int wsum[16];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int seg = (ncell + 1023) / 1024;
-    const int b0 = threadIdx.x * seg, b1 = min(b0 + seg, ncell);
-    // a thread's segment is read eight counts at a time with the loads in
-    // flight together (one dependent load per count made this kernel ~17 us)
-    constexpr int U = 8;
-    int v[U];
-    int local = 0;
-    for (int k0 = b0; k0 < b1; k0 += U) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = k0 + u < b1 ? count[k0 + u] : 0;
-#pragma unroll
-        for (int u = 0; u < U; ++u) local += v[u];
-    }
-    int x = local;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) wsum[wid] = x;
-    __syncthreads();
-    if (wid == 0) {
-        int t = lane < 16 ? wsum[lane] : 0;
-#pragma unroll
-        for (int o = 1; o < 16; o <<= 1) {
-            const int y = __shfl_up(t, o, 64);
-            if (lane >= o) t += y;
-        }
-        if (lane < 16) wsum[lane] = t;
-    }
-    __syncthreads();
-    int run = (wid > 0 ? wsum[wid - 1] : 0) + x - local;
-    for (int k0 = b0; k0 < b1; k0 += U) {
-        if (seg > U) {  // uniform; otherwise v still holds this segment
-#pragma unroll
-            for (int u = 0; u < U; ++u) v[u] = k0 + u < b1 ? count[k0 + u] : 0;
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (k0 + u < b1) {
-                start[k0 + u] = run;
-                fill[k0 + u] = run;
-                count[k0 + u] = 0;
-                run += v[u];
-            }
-        }
-    }
-    if (threadIdx.x == 1023) start[ncell] = wsum[15];
-}
-
-__device__ __forceinline__ void scan_body(int blk, int nblk, const int *__restrict__ gate, int ncell, int *__restrict__ count,
-                                          int *__restrict__ start, int *__restrict__ fill,
-                                          const BoxDev *__restrict__ box, BoxDev *__restrict__ boxLast) {
-    if (gate && *gate == 0) return;
-    scan_wg(ncell, count, start, fill, box, boxLast);
-}
-
-// Captured steps: the binning with the scan in its last workgroup (1024
-// threads a workgroup), one launch fewer on every step's path.
-__device__ __forceinline__ void bin_scan_body(int blk, int nblk, const int *__restrict__ gate, int n,
-                                              double4 *__restrict__ pos, const float *__restrict__ q,
-                                              const BoxDev *__restrict__ bx, int ncell, const int *__restrict__ colRank,
-                                              int *__restrict__ cellOf, int *__restrict__ cellCount,
-                                              const double4 *__restrict__ cen, const int *__restrict__ ids, int nslot,
-                                              int *__restrict__ start, int *__restrict__ fill,
-                                              BoxDev *__restrict__ boxLast, int *__restrict__ ticket) {
-    if (gate && *gate == 0) return;
     const int i = blk * blockDim.x + threadIdx.x;
-    if (i < n) bin_atom(i, pos, q, bx, ncell, colRank, cellOf, cellCount, cen, ids);
-    if (last_block(ticket, nblk)) scan_wg(nslot, cellCount, start, fill, bx, boxLast);
-}
-
-__device__ __forceinline__ void place_body(int blk, int nblk, const int *__restrict__ gate, int n, const int *__restrict__ cellOf, int *__restrict__ fill,
-                        int *__restrict__ perm) {
-    if (gate && *gate == 0) return;
-    int i = blk * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int slot = atomicAdd(&fill[cellOf[i]], 1);
-    perm[slot] = i;
-}
-
-// Make the order inside each cell independent of atomic slot order: one
-// workgroup per cell slot ranks its entries by atom id in LDS (ids are unique,
-// so rank = number of smaller keys) and writes them in rank order.
-__device__ __forceinline__ void cellsort_body(int blk, int nblk, const int *__restrict__ gate, int ncell,
-                                                 const int *__restrict__ start, const int *__restrict__ permIn,
-                                                 int *__restrict__ permOut, const int *__restrict__ id) {
-    if (gate && *gate == 0) return;
-    constexpr int CAP = 1024;
-    __shared__ int skey[CAP];
-    __shared__ int sperm[CAP];
-    const int c = blk;
-    const int a = start[c], b = start[c + 1], m = b - a;
-    if (m <= CAP) {
-        for (int t = threadIdx.x; t < m; t += 64) {
-            const int p = permIn[a + t];
-            sperm[t] = p;
-            skey[t] = id[p];
-        }
-        __syncthreads();
-        for (int t = threadIdx.x; t < m; t += 64) {
-            const int key = skey[t];
-            int r = 0;
-            for (int j = 0; j < m; ++j) r += skey[j] < key;
-            permOut[a + r] = sperm[t];
-        }
-    } else if (threadIdx.x == 0) {
-        // very crowded cell: serial insertion sort
-        for (int s = a; s < b; ++s) permOut[s] = permIn[s];
-        for (int s = a + 1; s < b; ++s) {
-            const int v = permOut[s];
-            const int key = id[v];
-            int t = s - 1;
-            while (t >= a && id[permOut[t]] > key) {
-                permOut[t + 1] = permOut[t];
-                --t;
+    int chunk = -1;
+    if (i < n) {
+        const Geometry g = bx->geo;
+        const CellGrid cg = bx->cg;
+        double4 p = pos[i];
+        const double4 v = vel[i];
+        const float qi = q[i];
+        const int ti = type[i], myid = id[i];
+        double *pc = &p.x;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            if (g.periodic[a]) {
+                double img = floor((pc[a] - g.lo[a]) * g.invL[a]);
+                pc[a] = pc[a] - img * g.L[a];
             }
-            permOut[t + 1] = v;
         }
+        pos1[i] = p;
+        vel1[i] = v;
+        q1[i] = qi;
+        type1[i] = ti;
+        id1[i] = myid;
+        // ring centroid lists: the atom goes to the cell of its ring's centroid
+        // (already in the box)
+        if (cen) p = cen[myid];
+        const int cx = cell_coord(p.x, g.lo[0], cg.cellInv[0], cg.nc[0]);
+        const int cy = cell_coord(p.y, g.lo[1], cg.cellInv[1], cg.nc[1]);
+        const int cz = cell_coord(p.z, g.lo[2], cg.cellInv[2], cg.nc[2]);
+        const int cell = colRank[cx * cg.nc[1] + cy] * cg.nc[2] + cz + (qi == 0.0f ? ncell : 0);
+        next[i] = atomicExch(&head[cell], i);
+        chunk = cell >> csh;
+    }
+    unsigned long long todo = __ballot(chunk >= 0);
+    while (todo) {
+        const int leader = __ffsll(todo) - 1;
+        const int k = __shfl(chunk, leader, 64);
+        const unsigned long long same = __ballot(chunk == k);
+        if ((int)(threadIdx.x & 63) == leader) atomicAdd(&chunkSum[k], __popcll(same));
+        todo &= ~same;
     }
 }
 
-// Gather the per-atom records into cell order (sortPerAtomArrays,
+// What the second launch of a re-sort reads and writes.
+struct SortArgs {
+    int n, nslot;        // atoms; cell slots (2 ncell)
+    int cpw, csh;        // cells a workgroup takes at a time (<= 256), log2 of a chunk's cells
+    int *head;           // per cell: its list of atoms (left empty for the next binning)
+    const int *next;
+    const int *chunkSum; // atoms per chunk
+    int *start;          // nslot + 1
+    const double4 *pos0, *vel0;
+    const float *q0;
+    const int *type0, *id0;
+    double4 *pos1, *vel1;
+    float *q1;
+    int *type1, *id1;
+    int *idToIdx;
+    double4 *last;       // positions of this build (wrapped)
+    float4 *xq;
+    float4 *rec;         // P3M mesh records, or nullptr
+    const double4 *cen;  // ring centroids by id, and the build positions made of them
+    double4 *bpos;
+    int *atomMolO;       // cleared for the molecule map of the build
+    int *member;
+    int maxExcl;         // exclusion rows by id (id | tag << 30, ~0u past the end)
+    const int *exclOff;
+    const uint32_t *exclIds;
+    uint32_t *exclRow;
+    unsigned *slots;     // the displacement maxima the binning decided from, cleared here
+    const BoxDev *bx;
+    BoxDev *boxLast;     // the box this build uses, kept for rebuilding the same list later
+};
+
+// Gather the record of atom o into place k (sortPerAtomArrays,
 // GridGPU.cu:253-293) and refresh idToIdx, the last-build positions and xq.
-__device__ __forceinline__ void permute_body(int blk, int nblk, const int *__restrict__ gate, int n, const int *__restrict__ perm, const double4 *__restrict__ pos0,
-                          const double4 *__restrict__ vel0, const float *__restrict__ q0,
-                          const int *__restrict__ t0, const int *__restrict__ id0,
-                          double4 *__restrict__ pos1, double4 *__restrict__ vel1,
-                          float *__restrict__ q1, int *__restrict__ t1, int *__restrict__ id1,
-                          int *__restrict__ idToIdx, double4 *__restrict__ last,
-                          float4 *__restrict__ xq, const BoxDev *__restrict__ bx, float4 *__restrict__ rec,
-                          const double4 *__restrict__ cen, double4 *__restrict__ bpos) {
-    if (gate && *gate == 0) return;
-    const Geometry g = bx->geo;
-    int k = blk * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    int o = perm[k];
-    double4 p = pos0[o];
-    pos1[k] = p;
-    vel1[k] = vel0[o];
-    float qq = q0[o];
-    q1[k] = qq;
-    t1[k] = t0[o];
-    int myid = id0[o];
-    id1[k] = myid;
-    idToIdx[myid] = k;
-    last[k] = p;
+__device__ __forceinline__ void place_atom(const SortArgs &a, int o, int k, int myid, const Geometry &g) {
+    double4 p = a.pos0[o];
+    const double4 v = a.vel0[o];
+    const float qq = a.q0[o];
+    const int tt = a.type0[o];
+    a.pos1[k] = p;
+    a.vel1[k] = v;
+    a.q1[k] = qq;
+    a.type1[k] = tt;
+    a.id1[k] = myid;
+    a.idToIdx[myid] = k;
+    a.last[k] = p;
+    if (a.atomMolO) a.atomMolO[k] = -1;
+    if (a.member) a.member[k] = 0;
+    if (a.maxExcl > 0) {
+        const int o0 = a.exclOff[myid], ne = a.exclOff[myid + 1] - o0;
+        for (int s = 0; s < a.maxExcl; ++s) a.exclRow[(size_t)k * a.maxExcl + s] = s < ne ? a.exclIds[o0 + s] : ~0u;
+    }
     // the P3M mesh records in the new order (captured steps whose first half
     // kick refreshed them before the rebuild)
-    if (rec && qq != 0.0f) rec[k] = mesh_record(p, bx->mesh);
+    if (a.rec && qq != 0.0f) a.rec[k] = mesh_record(p, a.bx->mesh);
     // ring centroid lists: the build works on the centroids (xq is written
     // again from the positions before the forces)
-    if (cen) {
-        p = cen[myid];
-        bpos[k] = p;
+    if (a.cen) {
+        p = a.cen[myid];
+        a.bpos[k] = p;
     }
-    xq[k] = make_float4((float)(p.x - g.lo[0]), (float)(p.y - g.lo[1]), (float)(p.z - g.lo[2]), qq);
+    a.xq[k] = make_float4((float)(p.x - g.lo[0]), (float)(p.y - g.lo[1]), (float)(p.z - g.lo[2]), qq);
+}
+
+// Scan, in-cell order and permutation of one chunk of cells per workgroup.
+// The workgroup's first place is the sum of the chunk counts before its own;
+// within it, one thread per cell walks the cell's list, a prefix sum over the
+// cells gives the cell starts, and one thread per atom ranks the atom by id
+// among its cell's (ids are unique, so the layout depends only on positions,
+// never on the order of the pushes) and moves its records.
+//
+// This replaces a scan of all cell counts by one workgroup (15 us at 7,200
+// cell slots, 126 us at 49,726, 2.8 ms at 828,478), a placing pass, a sort with
+// one workgroup per slot, the permutation and a copy-back: with the binning,
+// six launches of 40 us for 32,768 water sites and 3.1 ms for 500,000 LJ atoms
+// became two of 18.5 us and 70 us.
+// A cell slot holds about 0.6 (LJ) to 7 (water) atoms, so the walk is short; a
+// round whose atoms exceed the LDS buffer (crowded cells) ranks them through
+// the lists instead.
+constexpr int kSortThreads = 256;
+constexpr int kSortCap = 2048;  // atoms a round ranks in LDS
+__device__ __forceinline__ void sort_body(int blk, int nblk, const int *__restrict__ gate, SortArgs a) {
+    if (a.slots && blk == 0 && threadIdx.x < kDispSlots) a.slots[threadIdx.x * kDispStride] = 0u;
+    if (gate && *gate == 0) return;
+    __shared__ int sIdx[kSortCap], sKey[kSortCap];
+    __shared__ unsigned char sCell[kSortCap];
+    __shared__ int sStart[kSortThreads + 1], wsum[kSortThreads / 64];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    if (blk == 0) {
+        constexpr int kBoxWords = (int)(sizeof(BoxDev) / sizeof(int));
+        static_assert(sizeof(BoxDev) % sizeof(int) == 0, "BoxDev copied as words");
+        for (int k = tid; k < kBoxWords; k += kSortThreads)
+            reinterpret_cast<int *>(a.boxLast)[k] = reinterpret_cast<const int *>(a.bx)[k];
+    }
+    const Geometry g = a.bx->geo;
+    // atoms of the chunks before this one
+    int before = 0;
+    constexpr int U = 8;
+    for (int k0 = tid; k0 < blk; k0 += U * kSortThreads) {
+        int v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = k0 + u * kSortThreads < blk ? a.chunkSum[k0 + u * kSortThreads] : 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) before += v[u];
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
+    if (lane == 0) wsum[w] = before;
+    __syncthreads();
+    int base = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    const int c0 = blk << a.csh, c1 = min(c0 + (1 << a.csh), a.nslot);
+    for (int cb = c0; cb < c1; cb += a.cpw) {
+        const int c = cb + tid;
+        const bool live = tid < a.cpw && c < c1;
+        // the first entries of the cell's list stay in registers
+        constexpr int R = 8;
+        int e[R], m = 0, h = live ? a.head[c] : -1;
+        if (live) a.head[c] = -1;
+        const int first = h;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            e[r] = h;
+            if (h >= 0) {
+                h = a.next[h];
+                ++m;
+            }
+        }
+        while (h >= 0) {
+            h = a.next[h];
+            ++m;
+        }
+        int x = m;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(x, o, 64);
+            if (lane >= o) x += y;
+        }
+        __syncthreads();  // wsum and the lists' buffers of the round before are free
+        if (lane == 63) wsum[w] = x;
+        __syncthreads();
+        int pre = x - m;
+        for (int k = 0; k < w; ++k) pre += wsum[k];
+        const int total = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+        if (live) a.start[c] = base + pre;
+        sStart[tid] = pre;
+        if (tid == 0) sStart[kSortThreads] = total;
+        if (total <= kSortCap) {  // uniform
+            int k = pre;
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (r < m) {
+                    sIdx[k] = e[r];
+                    sCell[k++] = (unsigned char)tid;
+                }
+            if (m > R)
+                for (h = a.next[e[R - 1]]; h >= 0; h = a.next[h]) {
+                    sIdx[k] = h;
+                    sCell[k++] = (unsigned char)tid;
+                }
+            __syncthreads();
+            for (int t = tid; t < total; t += kSortThreads) sKey[t] = a.id0[sIdx[t]];
+            __syncthreads();
+            for (int t = tid; t < total; t += kSortThreads) {
+                const int cl = sCell[t], s0 = sStart[cl], s1 = sStart[cl + 1], key = sKey[t];
+                int r = s0;
+                for (int j = s0; j < s1; ++j) r += sKey[j] < key;
+                place_atom(a, sIdx[t], base + r, key, g);
+            }
+        } else {
+            for (int o = first; o >= 0; o = a.next[o]) {
+                const int key = a.id0[o];
+                int r = pre;
+                for (int j = first; j >= 0; j = a.next[j]) r += a.id0[j] < key;
+                place_atom(a, o, base + r, key, g);
+            }
+        }
+        base += total;
+    }
+    if (blk == nblk - 1 && tid == 0) a.start[a.nslot] = a.n;
 }
 
 __device__ __forceinline__ void xq_body(int blk, int nblk, int n, const double4 *__restrict__ pos, const float *__restrict__ q,
@@ -316,64 +349,12 @@ __device__ __forceinline__ void xq_zero_body(int blk, int nblk, int n, const dou
     if (rec && qk != 0.0f) rec[k] = mesh_record(p, bx->mesh);
 }
 
-// exclusion row of atom i (id myid) in current indices, tags kept
-__device__ __forceinline__ void excl_row(int i, int myid, const int *__restrict__ exclOff,
-                                         const uint32_t *__restrict__ exclIds, const int *__restrict__ idToIdx,
-                                         int maxExcl, uint32_t *__restrict__ exclIdx) {
-    const int e0 = exclOff[myid], e1 = exclOff[myid + 1];
-    for (int q = 0; q < maxExcl; ++q) {
-        uint32_t v = ~0u;
-        if (q < e1 - e0) {
-            const uint32_t e = exclIds[e0 + q];
-            v = (uint32_t)idToIdx[e & 0x3FFFFFFFu] | (e & 0xC0000000u);
-        }
-        exclIdx[(size_t)i * maxExcl + q] = v;
-    }
-}
-
-__device__ __forceinline__ void copy_back_body(int blk, int nblk, const int *__restrict__ gate, int n, const double4 *__restrict__ pos1,
-                            const double4 *__restrict__ vel1, const float *__restrict__ q1,
-                            const int *__restrict__ t1, const int *__restrict__ id1, double4 *__restrict__ pos0,
-                            double4 *__restrict__ vel0, float *__restrict__ q0, int *__restrict__ t0,
-                            int *__restrict__ id0, const int *__restrict__ exclOff,
-                            const uint32_t *__restrict__ exclIds, const int *__restrict__ idToIdx, int maxExcl,
-                            uint32_t *__restrict__ exclIdx, int *__restrict__ atomMolO,
-                            int *__restrict__ member) {
-    if (gate && *gate == 0) return;
-    int k = blk * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    pos0[k] = pos1[k];
-    vel0[k] = vel1[k];
-    q0[k] = q1[k];
-    t0[k] = t1[k];
-    const int myid = id1[k];
-    id0[k] = myid;
-    // the exclusion rows (k_excl_idx) and the cleared oxygen map of the new
-    // order in the same pass: one launch fewer in every captured step
-    if (maxExcl > 0) excl_row(k, myid, exclOff, exclIds, idToIdx, maxExcl, exclIdx);
-    if (atomMolO) atomMolO[k] = -1;
-    if (member) member[k] = 0;
-}
-
-// one wave: the maxima of the nb workgroups
-
-// Device-side step decisions of a captured step (one thread): rebuild the
-// list iff the largest displacement since the last build exceeds skin/2 (the
-// reference's setBuildFlag test, GridGPU.cu:755-774), count it, and set the
-// thermostat gate for the steps where the turn reaches a multiple of its
-// interval.  Clears the displacement slot for the next step.
-__device__ __forceinline__ void decide_body(int blk, int nblk, int nb, const float *__restrict__ part, unsigned *__restrict__ dmax,
-                         int *__restrict__ flags, float half2, int every, int baroEvery,
-                         unsigned long long *__restrict__ thermo) {
-    DecideArgs d{};
-    d.part = part;
-    d.dmax = dmax;
-    d.flags = flags;
-    d.half2 = half2;
-    d.every = every;
-    d.baroEvery = baroEvery;
-    d.thermo = thermo;
-    decide_wg(nb, d);
+// The step decisions as a launch of their own (one wave), from the nb
+// per-workgroup maxima of the displacement check.
+__device__ __forceinline__ void decide_body(int blk, int nblk, int nb, DecideArgs d) {
+    float d2, p2;
+    part_max(nb, d.part, d2, p2);
+    if (threadIdx.x == 0) decide_write(d, d2 > d.half2);
 }
 
 // Stencil walk without local arrays (a dynamically indexed local array would
@@ -761,6 +742,18 @@ __device__ __forceinline__ void build_body(int blk, int nblk, const int *__restr
 // a lane finds its run from the run of the chunk start (runs are rarely
 // shorter than the few lanes they straddle), so the bookkeeping is a couple
 // of LDS reads per lane and the compaction is one mbcnt on the wave ballot.
+// the exclusion rows of the sort, translated to current indices as they are
+// read (the sort has just renumbered the atoms)
+struct ExclArgs {
+    int maxExcl;
+    const uint32_t *row;
+    const int *idToIdx;
+};
+__device__ __forceinline__ uint32_t excl_entry(const ExclArgs &x, int i, int q) {
+    const uint32_t e = x.row[(size_t)i * x.maxExcl + q];
+    return e == ~0u ? e : (uint32_t)x.idToIdx[e & 0x3FFFFFFFu] | (e & 0xC0000000u);
+}
+
 struct RunEntry {
     int vend;      // end of the run in the stream
     int off;       // atom index = stream position + off
@@ -772,7 +765,7 @@ template <bool SHIFT>
 __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__restrict__ gate,
     int n, const double4 *__restrict__ pos, const float4 *__restrict__ xq, const BoxDev *__restrict__ bx,
     const int *__restrict__ colRank, const int *__restrict__ cellStart, int ncell,
-    double rlist2, const uint32_t *__restrict__ exclIdx, int maxExcl, int cap,
+    double rlist2, ExclArgs ex, int cap,
     uint32_t *__restrict__ nl, int *__restrict__ nlCount, int *__restrict__ nlCountA, int *__restrict__ flags,
     int *__restrict__ waveMax) {
     if (gate && *gate == 0) return;
@@ -783,6 +776,7 @@ __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__
     constexpr int U = 4;             // chunks of 64 candidates per load block
     constexpr int R = 4 * kMaxCols;  // 2 classes x 2 z-runs per column
     __shared__ RunEntry sRun[4][R + 1];
+    __shared__ uint32_t sEx[4][64];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int i = __builtin_amdgcn_readfirstlane(blk * 4 + (int)(threadIdx.x >> 6));
     if (i >= n) {
@@ -798,9 +792,16 @@ __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__
     const int cx = cell_coord(pi.x, g.lo[0], cg.cellInv[0], cg.nc[0]);
     const int cy = cell_coord(pi.y, g.lo[1], cg.cellInv[1], cg.nc[1]);
     const int cz = cell_coord(pi.z, g.lo[2], cg.cellInv[2], cg.nc[2]);
-    const uint32_t *exRow = exclIdx + (size_t)i * maxExcl;
-    const uint32_t ex0 = maxExcl > 0 ? exRow[0] : ~0u, ex1 = maxExcl > 1 ? exRow[1] : ~0u;
-    const uint32_t ex2 = maxExcl > 2 ? exRow[2] : ~0u, ex3 = maxExcl > 3 ? exRow[3] : ~0u;
+    // exclusion partners in current indices, one per lane: the first four are
+    // uniform, further ones go to LDS
+    uint32_t exv = ~0u;
+    if (ex.maxExcl > 0) {
+        if (lane < ex.maxExcl) exv = excl_entry(ex, i, lane);
+        if (ex.maxExcl > 4) sEx[w][lane] = exv;
+    }
+    const int maxExcl = ex.maxExcl;
+    const uint32_t ex0 = (uint32_t)__builtin_amdgcn_readlane((int)exv, 0), ex1 = (uint32_t)__builtin_amdgcn_readlane((int)exv, 1);
+    const uint32_t ex2 = (uint32_t)__builtin_amdgcn_readlane((int)exv, 2), ex3 = (uint32_t)__builtin_amdgcn_readlane((int)exv, 3);
     // ---- table: one (class, column) per lane
     const int cls = lane >> 5, col = lane & 31;
     const int *cs = cellStart + cls * ncell;
@@ -946,11 +947,12 @@ __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__
                 tag = e1 == uj ? ex1 >> 30 : tag;
                 tag = e2 == uj ? ex2 >> 30 : tag;
                 tag = e3 == uj ? ex3 >> 30 : tag;
-                if (maxExcl > 4 && hit)
+                if (maxExcl > 4 && hit) {
                     for (int qq = 4; qq < maxExcl; ++qq) {
-                        const uint32_t e = exRow[qq];
+                        const uint32_t e = qq < 64 ? sEx[w][qq] : excl_entry(ex, i, qq);
                         if ((e & 0x3FFFFFFFu) == uj) tag = e >> 30;
                     }
+                }
             }
             const unsigned long long m = __ballot(hit);
             if (hit) {
@@ -975,15 +977,13 @@ __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__
     }
 }
 
-// Exclusion partners of each atom as current indices (idx | tag << 30), one
-// row of maxExcl per atom padded with ~0u, refreshed after each permutation.
-__device__ __forceinline__ void excl_idx_body(int blk, int nblk, const int *__restrict__ gate, int n, const int *__restrict__ id, const int *__restrict__ exclOff,
-                           const uint32_t *__restrict__ exclIds, const int *__restrict__ idToIdx,
-                           int maxExcl, uint32_t *__restrict__ exclIdx) {
+// Exclusion rows from ids to current indices (idx | tag << 30), in place,
+// for the team builds, which read them lane by lane.
+__device__ __forceinline__ void excl_idx_body(int blk, int nblk, const int *__restrict__ gate, long long n,
+                                              const int *__restrict__ idToIdx, uint32_t *__restrict__ row) {
     if (gate && *gate == 0) return;
-    int i = blk * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    excl_row(i, id[i], exclOff, exclIds, idToIdx, maxExcl, exclIdx);
+    const long long k = (long long)blk * blockDim.x + threadIdx.x;
+    if (k < n && row[k] != ~0u) row[k] = (uint32_t)idToIdx[row[k] & 0x3FFFFFFFu] | (row[k] & 0xC0000000u);
 }
 
 // E3B molecule list from the atom list: for each water, the oxygens among its
@@ -1038,34 +1038,11 @@ __device__ __forceinline__ void e3b_list_body(int blk, int nblk,
     if (lane == 0) waveMax[gtid >> 6] = wmax;
 }
 
-// Captured steps also map the rigid molecules here (k_rigid_map's work, rigid
-// molecules nmolR > 0, member cleared by k_copy_back): one launch for both.
-__device__ __forceinline__ void mol_atoms_body(int blk, int nblk, const int *__restrict__ gate, int nmol, const int4 *__restrict__ molIds, const int *__restrict__ idToIdx,
-                            int4 *__restrict__ molAtoms, int *__restrict__ atomMolO, int nmolR,
-                            const int4 *__restrict__ rigidIds, int4 *__restrict__ rigidAtoms,
-                            int *__restrict__ member) {
-    if (gate && *gate == 0) return;
-    int m = blk * blockDim.x + threadIdx.x;
-    if (m < nmolR) {
-        const int4 i = rigidIds[m];
-        const int4 a = make_int4(idToIdx[i.x], idToIdx[i.y], idToIdx[i.z], i.w >= 0 ? idToIdx[i.w] : -1);
-        rigidAtoms[m] = a;
-        member[a.x] = 1;
-        member[a.y] = 1;
-        member[a.z] = 1;
-        if (a.w >= 0) member[a.w] = 1;
-    }
-    if (m >= nmol) return;
-    int4 ids = molIds[m];
-    int4 a = make_int4(idToIdx[ids.x], idToIdx[ids.y], idToIdx[ids.z], idToIdx[ids.w]);
-    molAtoms[m] = a;
-    atomMolO[a.x] = m;
-}
-
-// The list build with the molecule map of a rebuild (mol_atoms_body) as
-// extra workgroups of the same launch: the map only needs the new indices,
-// which the permutation wrote before, and the E3B list that reads it comes
-// after (one launch fewer per step).
+// Molecule to current site indices after a re-sort (E3B, rigid and flexible
+// molecules), with the oxygen map and the membership flags that the re-sort
+// cleared, and the chunk counts of the binning cleared for the next one.
+// Extra workgroups of the list build: the maps only need the new indices, and
+// what reads them comes after (one launch fewer per step).
 struct MolMapArgs {
     int blocks;
     int nmol;
@@ -1077,23 +1054,51 @@ struct MolMapArgs {
     const int4 *rigidIds;
     int4 *rigidAtoms;
     int *member;
+    int nmolF;
+    const int4 *flexIds;
+    int4 *flexAtoms;
+    int nchunk;
+    int *chunkSum;
 };
+
+__device__ __forceinline__ int4 mol_indices(const int4 &i, const int *__restrict__ idToIdx) {
+    return make_int4(idToIdx[i.x], idToIdx[i.y], idToIdx[i.z], i.w >= 0 ? idToIdx[i.w] : -1);
+}
+
+__device__ __forceinline__ void mol_map_body(int blk, int nblk, const int *__restrict__ gate, MolMapArgs mm) {
+    if (gate && *gate == 0) return;
+    const int m = blk * blockDim.x + threadIdx.x;
+    if (m < mm.nchunk) mm.chunkSum[m] = 0;
+    if (m < mm.nmolR) {
+        const int4 a = mol_indices(mm.rigidIds[m], mm.idToIdx);
+        mm.rigidAtoms[m] = a;
+        mm.member[a.x] = 1;
+        mm.member[a.y] = 1;
+        mm.member[a.z] = 1;
+        if (a.w >= 0) mm.member[a.w] = 1;
+    }
+    if (m < mm.nmolF) mm.flexAtoms[m] = mol_indices(mm.flexIds[m], mm.idToIdx);
+    if (m < mm.nmol) {
+        const int4 a = mol_indices(mm.molIds[m], mm.idToIdx);
+        mm.molAtoms[m] = a;
+        mm.atomMolO[a.x] = m;
+    }
+}
 
 template <bool SHIFT>
 __device__ __forceinline__ void build_map_body(int blk, int nblk, const int *__restrict__ gate,
     int n, const double4 *__restrict__ pos, const float4 *__restrict__ xq, const BoxDev *__restrict__ bx,
     const int *__restrict__ colRank, const int *__restrict__ cellStart, int ncell,
-    double rlist2, const uint32_t *__restrict__ exclIdx, int maxExcl, int cap,
+    double rlist2, ExclArgs ex, int cap,
     uint32_t *__restrict__ nl, int *__restrict__ nlCount, int *__restrict__ nlCountA, int *__restrict__ flags,
     int *__restrict__ waveMax, MolMapArgs mm) {
     const int nb = nblk - mm.blocks;
     if (blk >= nb) {  // uniform over the workgroup
-        mol_atoms_body(blk - nb, mm.blocks, gate, mm.nmol, mm.molIds, mm.idToIdx, mm.molAtoms, mm.atomMolO, mm.nmolR,
-                       mm.rigidIds, mm.rigidAtoms, mm.member);
+        mol_map_body(blk - nb, mm.blocks, gate, mm);
         return;
     }
-    build_wave_body<SHIFT>(blk, nb, gate, n, pos, xq, bx, colRank, cellStart, ncell, rlist2, exclIdx, maxExcl, cap, nl,
-                           nlCount, nlCountA, flags, waveMax);
+    build_wave_body<SHIFT>(blk, nb, gate, n, pos, xq, bx, colRank, cellStart, ncell, rlist2, ex, cap, nl, nlCount,
+                           nlCountA, flags, waveMax);
 }
 
 __device__ __forceinline__ void fill_int_body(int blk, int nblk, const int *__restrict__ gate, int n, int *__restrict__ p, int v) {
@@ -1131,8 +1136,9 @@ uint32_t morton2(uint32_t x, uint32_t y) {
 // slots of the pair-list waves in c.waveMax; the molecule-list slots follow
 size_t wave_slots_a(const Ctx &c) { return (size_t)c.n + 4; }
 
-// mm.blocks > 0: the molecule map of the rebuild runs in the same launch
+// with the molecule maps of the rebuild in the same launch
 void launch_build_wave(Ctx &c, int cur, const MolMapArgs &mm) {
+    const ExclArgs ex{c.exclOff ? c.maxExcl : 0, c.exclIdx, c.idToIdx};
     MDX_REQUIRE(std::min(c.nc[0], 2 * c.reach[0] + 1) * std::min(c.nc[1], 2 * c.reach[1] + 1) <= kMaxCols, 1,
                 "stencil wider than the build kernel's column table");
     const int blocks = cdiv(c.n, 4);
@@ -1141,9 +1147,9 @@ void launch_build_wave(Ctx &c, int cur, const MolMapArgs &mm) {
     for (int a = 0; a < 3; ++a)
         if (c.geo.periodic[a] && c.nc[a] < 2 * c.reach[a] + 1) shift = false;
     if (shift)
-        launch<build_map_body<true>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, c.box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, c.exclIdx, c.exclOff ? c.maxExcl : 0, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm);
+        launch<build_map_body<true>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, c.box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, ex, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm);
     else
-        launch<build_map_body<false>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, c.box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, c.exclIdx, c.exclOff ? c.maxExcl : 0, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm);
+        launch<build_map_body<false>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, c.box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, ex, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm);
     c.waveMaxA = blocks * 4;
 }
 
@@ -1193,20 +1199,30 @@ void nlist_setup(Ctx &c) {
         if (c.ncell) {
             dfree(c, c.colXY);
             dfree(c, c.colRank);
-            dfree(c, c.cellCount);
+            dfree(c, c.cellHead);
             dfree(c, c.cellStart);
-            dfree(c, c.cellFill);
         }
         c.ncell = ncell;
         c.colRank = dalloc<int>(c, (size_t)c.nc[0] * c.nc[1]);
         c.colXY = dalloc<int2>(c, (size_t)c.nc[0] * c.nc[1]);
         // two copies of the grid: charged atoms, then charge-free ones
-        c.cellCount = dalloc<int>(c, 2 * (size_t)ncell);
-        // k_scan leaves the counts at zero for the next binning
-        MDX_HIP(hipMemsetAsync(c.cellCount, 0, sizeof(int) * 2 * (size_t)ncell, c.stream));
+        c.cellHead = dalloc<int>(c, 2 * (size_t)ncell);
+        // the sort leaves the lists empty for the next binning
+        MDX_HIP(hipMemsetAsync(c.cellHead, 0xFF, sizeof(int) * 2 * (size_t)ncell, c.stream));
         c.cellStart = dalloc<int>(c, 2 * (size_t)ncell + 1);
-        c.cellFill = dalloc<int>(c, 2 * (size_t)ncell);
     }
+    // chunks of cells for the sort: at least 512 workgroups while a workgroup
+    // still has 32 cells (an 8,192-molecule box has 7,200 slots: 225 workgroups
+    // of 32), then up to 256 cells at a time, then several rounds of 256
+    // (about 2,048 workgroups: each sums the chunk counts before its own)
+    const int nslot = 2 * ncell;
+    c.sortCpw = 32;
+    while (c.sortCpw < kSortThreads && cdiv(nslot, c.sortCpw) > 512) c.sortCpw *= 2;
+    int chunk = c.sortCpw;
+    while (cdiv(nslot, chunk) > 2048) chunk *= 2;
+    c.sortCsh = 0;
+    while ((1 << c.sortCsh) < chunk) ++c.sortCsh;
+    c.nChunk = cdiv(nslot, chunk);
     // column ranks along a 2-D Morton curve
     std::vector<std::pair<uint32_t, int>> keys;
     for (int x = 0; x < c.nc[0]; ++x)
@@ -1223,10 +1239,9 @@ void nlist_setup(Ctx &c) {
     MDX_HIP(hipMemcpyAsync(c.colXY, xy.data(), sizeof(int2) * xy.size(), hipMemcpyHostToDevice,
                            c.stream));
     MDX_HIP(hipStreamSynchronize(c.stream));
-    if (!c.cellOf) {
-        c.cellOf = dalloc<int>(c, c.n);
-        c.perm = dalloc<int>(c, c.n);
-        c.perm2 = dalloc<int>(c, c.n);
+    if (!c.cellNext) {
+        c.cellNext = dalloc<int>(c, c.n);
+        c.chunkSum = dalloc<int>(c, 2048);
     }
     // one wave per atom (k_build_wave) measured fastest for dense water and
     // LJ alike; mdx_tune revisits the width
@@ -1293,25 +1308,16 @@ static void run_build(Ctx &c, bool sync) {
         c.waveMax = dalloc<int>(c, needSlots);
         c.waveMaxN = (int)needSlots;
     }
-    int threads = 256;
-    int cur = c.cur, nxt = 1 - c.cur;
+    const int threads = 256;
+    const int cur = c.cur, scr = 1 - c.cur;  // the records are sorted in place; scr: scratch copies
     const int nslot = 2 * c.ncell;
-    MolMapArgs mm{};
-    bool mapFused = false;
     const double4 *cen = c.cenById;
     MDX_REQUIRE(!cen || (c.buildPos && !c.e3b.on), 3,
                 "a centroid list needs its build positions and takes no E3B molecule list");
-    c.centroidList = cen != nullptr;
-    if (c.capture && c.fuseStep) {
-        launch<bin_scan_body, 1024>(c, cdiv(c.n, 1024), 0, rebuild_gate(c), c.n, c.pos[cur], c.q[cur], c.box, c.ncell, c.colRank, c.cellOf, c.cellCount, cen, c.id[cur], nslot, c.cellStart, c.cellFill, c.boxLast, c.dFlags + 11);
-    } else {
-        launch<bin_body, 256>(c, cdiv(c.n, threads), 0, rebuild_gate(c), c.n, c.pos[cur], c.q[cur], c.box, c.ncell, c.colRank, c.cellOf, c.cellCount, cen, c.id[cur]);
-        launch<scan_body, 1024>(c, 1, 0, rebuild_gate(c), nslot, c.cellCount, c.cellStart, c.cellFill, c.box, c.boxLast);
-    }
-    launch<place_body, 256>(c, cdiv(c.n, threads), 0, rebuild_gate(c), c.n, c.cellOf, c.cellFill, c.perm);
-    launch<cellsort_body, 64>(c, nslot, 0, rebuild_gate(c), nslot, c.cellStart, c.perm, c.perm2, c.id[cur]);
-    launch<permute_body, 256>(c, cdiv(c.n, threads), 0, rebuild_gate(c), c.n, c.perm2, c.pos[cur], c.vel[cur], c.q[cur], c.type[cur], c.id[cur], c.pos[nxt], c.vel[nxt], c.q[nxt], c.type[nxt], c.id[nxt], c.idToIdx, c.posLast, c.xq, c.box,
-                              c.refreshed && c.pppm.on && c.hasCharges ? c.meshRec : nullptr, cen, c.buildPos);
+    MDX_REQUIRE(!c.e3b.on || c.rlist >= (double)c.e3b.r2b + c.skin - 1e-9, 1,
+                "E3B needs rCut + padding >= 6.2 A + padding (the molecule list is taken from the "
+                "pair list)");
+    const bool waveBuild = c.buildTeam != 8 && c.buildTeam != 16 && c.buildTeam != 32;
     const bool excl = c.exclOff && c.maxExcl > 0;
     if (excl) {
         MDX_REQUIRE(!c.capture || c.exclIdxN == (size_t)c.n * c.maxExcl, 3,
@@ -1322,49 +1328,84 @@ static void run_build(Ctx &c, bool sync) {
             c.exclIdx = dalloc<uint32_t>(c, c.exclIdxN);
         }
     }
-    if (c.capture) {
-        // a captured step keeps fixed buffers: the sorted records come back,
-        // with the exclusion rows and the cleared E3B oxygen map
-        launch<copy_back_body, 256>(c, cdiv(c.n, threads), 0, rebuild_gate(c), c.n, c.pos[nxt], c.vel[nxt], c.q[nxt], c.type[nxt], c.id[nxt], c.pos[cur], c.vel[cur], c.q[cur], c.type[cur], c.id[cur], c.exclOff, c.exclIds, c.idToIdx, excl ? c.maxExcl : 0, c.exclIdx, c.e3b.on ? c.e3b.atomMolO : nullptr, c.rigid.on ? c.rigid.member : nullptr);
-        // The P3M chain needs the sorted sites, their mesh records (the
-        // permutation wrote them, the first half kick having refreshed them)
-        // and the cells, not the list: its stream forks here, so the list
-        // build below runs beside it.
-        if (c.refreshed && c.side && c.meshStream && !c.rec && c.pppm.on) {
-            MDX_HIP(hipEventRecord(c.evFork, c.stream));
-            c.forked = true;
-        }
-    } else {
-        c.cur = nxt;
-        if (excl)
-            launch<excl_idx_body, 256>(c, cdiv(c.n, threads), 0, nullptr, c.n, c.id[c.cur], c.exclOff, c.exclIds, c.idToIdx, c.maxExcl, c.exclIdx);
+    c.centroidList = cen != nullptr;
+    // the build's map workgroups clear the counts for the next binning; an
+    // eager build does not rely on an earlier one having got that far
+    if (!c.capture) fill_int(c, c.chunkSum, c.nChunk, 0);
+    DecideArgs da{};
+    if (c.capture && c.fuseCheck) {
+        da = decide_args(c);
+        da.slots = c.dispSlots;
     }
-    rigid_map(c);
-    flex_map(c);
+    launch<bin_body, 256>(c, cdiv(c.n, threads), 0, rebuild_gate(c), c.n, c.pos[cur], c.vel[cur], c.q[cur], c.type[cur], c.id[cur], c.pos[scr], c.vel[scr], c.q[scr], c.type[scr], c.id[scr], c.box, c.ncell, c.colRank, c.cellHead, c.cellNext, c.chunkSum, c.sortCsh, cen, da);
+    SortArgs sa{};
+    sa.n = c.n;
+    sa.nslot = nslot;
+    sa.cpw = c.sortCpw;
+    sa.csh = c.sortCsh;
+    sa.head = c.cellHead;
+    sa.next = c.cellNext;
+    sa.chunkSum = c.chunkSum;
+    sa.start = c.cellStart;
+    sa.pos0 = c.pos[scr];
+    sa.vel0 = c.vel[scr];
+    sa.q0 = c.q[scr];
+    sa.type0 = c.type[scr];
+    sa.id0 = c.id[scr];
+    sa.pos1 = c.pos[cur];
+    sa.vel1 = c.vel[cur];
+    sa.q1 = c.q[cur];
+    sa.type1 = c.type[cur];
+    sa.id1 = c.id[cur];
+    sa.idToIdx = c.idToIdx;
+    sa.last = c.posLast;
+    sa.xq = c.xq;
+    sa.rec = c.refreshed && c.pppm.on && c.hasCharges ? c.meshRec : nullptr;
+    sa.cen = cen;
+    sa.bpos = c.buildPos;
+    sa.atomMolO = c.e3b.on ? c.e3b.atomMolO : nullptr;
+    sa.member = c.rigid.on ? c.rigid.member : nullptr;
+    sa.maxExcl = excl ? c.maxExcl : 0;
+    sa.exclOff = c.exclOff;
+    sa.exclIds = c.exclIds;
+    sa.exclRow = c.exclIdx;
+    sa.slots = da.slots;
+    sa.bx = c.box;
+    sa.boxLast = c.boxLast;
+    launch<sort_body, kSortThreads>(c, c.nChunk, 0, rebuild_gate(c), sa);
+    // The P3M chain needs the sorted sites, their mesh records (written by the
+    // sort, the first half kick having refreshed them) and the cells, not the
+    // list: its stream forks here, so the list build below runs beside it.
+    if (c.capture && c.refreshed && c.side && c.meshStream && !c.rec && c.pppm.on) {
+        MDX_HIP(hipEventRecord(c.evFork, c.stream));
+        c.forked = true;
+    }
+    if (excl && !waveBuild)
+        launch<excl_idx_body, 256>(c, cdiv((long long)c.n * c.maxExcl, threads), 0, rebuild_gate(c), (long long)c.n * c.maxExcl, c.idToIdx, c.exclIdx);
+    MolMapArgs mm{};
+    mm.idToIdx = c.idToIdx;
     if (c.e3b.on) {
-        // indices were permuted: drop the old map (captured steps did so in k_copy_back)
-        if (!c.capture) fill_int(c, c.e3b.atomMolO, c.n, -1, nullptr);
-        const int nmolR = c.capture && c.rigid.on ? c.rigid.nmol : 0;  // see rigid_map
-        mm.blocks = cdiv(std::max(c.e3b.nmol, nmolR), threads);
         mm.nmol = c.e3b.nmol;
         mm.molIds = c.e3b.molIds;
-        mm.idToIdx = c.idToIdx;
         mm.molAtoms = c.e3b.molAtoms;
         mm.atomMolO = c.e3b.atomMolO;
-        mm.nmolR = nmolR;
+    }
+    if (c.rigid.on) {
+        mm.nmolR = c.rigid.nmol;
         mm.rigidIds = c.rigid.ids;
         mm.rigidAtoms = c.rigid.atoms;
         mm.member = c.rigid.member;
-        // the wave build takes the map as extra workgroups; the team builds launch it first
-        if (c.fuseStep && c.buildTeam != 8 && c.buildTeam != 16 && c.buildTeam != 32) {
-            mapFused = true;
-        } else {
-            launch<mol_atoms_body, 256>(c, mm.blocks, 0, rebuild_gate(c), mm.nmol, mm.molIds, mm.idToIdx, mm.molAtoms, mm.atomMolO, mm.nmolR, mm.rigidIds, mm.rigidAtoms, mm.member);
-        }
-        MDX_REQUIRE(c.rlist >= (double)c.e3b.r2b + c.skin - 1e-9, 1,
-                    "E3B needs rCut + padding >= 6.2 A + padding (the molecule list is taken from the "
-                    "pair list)");
     }
+    if (c.flex.on) {
+        mm.nmolF = c.flex.nmol;
+        mm.flexIds = c.flex.ids;
+        mm.flexAtoms = c.flex.atoms;
+    }
+    mm.nchunk = c.nChunk;
+    mm.chunkSum = c.chunkSum;
+    mm.blocks = cdiv(std::max({mm.nmol, mm.nmolR, mm.nmolF, mm.nchunk}), threads);
+    // the wave build takes the maps as extra workgroups; the team builds launch them first
+    if (!waveBuild) launch<mol_map_body, 256>(c, mm.blocks, 0, rebuild_gate(c), mm);
     for (;;) {
         // a captured step keeps the running maximum of the chunk in dFlags[1..2]
         if (!c.capture) fill_int(c, c.dFlags + 1, 2, 0);
@@ -1374,7 +1415,7 @@ static void run_build(Ctx &c, bool sync) {
                 case 8: launch_build<8>(c, c.cur); break;
                 case 16: launch_build<16>(c, c.cur); break;
                 case 32: launch_build<32>(c, c.cur); break;
-                default: launch_build_wave(c, c.cur, mapFused ? mm : MolMapArgs{}); break;
+                default: launch_build_wave(c, c.cur, mm); break;
             }
         }
         c.waveMaxB = 0;
@@ -1551,23 +1592,15 @@ DecideArgs decide_args(const Ctx &c) {
 void skin_check(Ctx &c) { check_part(c); }
 
 void skin_decide(Ctx &c) {
-    const DecideArgs d = decide_args(c);
-    const float *part = c.ringPart ? c.ringPart : d.part;
-    const int nb = c.ringPart ? c.ringPartNb : check_blocks(c);
-    launch<decide_body, 64>(c, 1, 0, nb, part, d.dmax, d.flags, d.half2, d.every, d.baroEvery, d.thermo);
+    DecideArgs d = decide_args(c);
+    if (c.ringPart) d.part = c.ringPart;
+    launch<decide_body, 64>(c, 1, 0, c.ringPart ? c.ringPartNb : check_blocks(c), d);
 }
 
 void decide_step(Ctx &c) {
-    // all-rigid captured steps: the rigid first half wrote the partial maxima
-    // and took the decisions in its last workgroup
-    if (c.decided) {
-        c.decided = false;
-        return;
-    }
-    const int fused = c.fuseCheck ? fused_check_blocks(c) : 0;
-    if (!fused) check_part(c);
-    const DecideArgs d = decide_args(c);
-    launch<decide_body, 64>(c, 1, 0, fused ? fused : check_blocks(c), d.part, d.dmax, d.flags, d.half2, d.every, d.baroEvery, d.thermo);
+    if (c.fuseCheck) return;  // the binning decides from the first half's maxima
+    check_part(c);
+    skin_decide(c);
 }
 
 void check_max(Ctx &c, int parity) {

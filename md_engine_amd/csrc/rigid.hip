@@ -139,45 +139,21 @@ __device__ __forceinline__ void dist_forces(const unsigned long long *f, int4 a,
     }
 }
 
-// squared minimum-image displacement, the same expressions as the list's
-// skin check (dist2 of the neighbor-list code), so the maxima agree bit for bit
-__device__ __forceinline__ double disp2(const double4 &a, const double4 &b, const Geometry &g) {
-    double d[3] = {b.x - a.x, b.y - a.y, b.z - a.z};
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-        if (g.periodic[k]) {
-            double img = rint(d[k] * g.invL[k]);
-            d[k] = d[k] - img * g.L[k];
-        }
-    return d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-}
-
-// part != nullptr: also the skin check's per-workgroup maxima (k_check_part)
-// of the sites' displacement since the last build and of the displacement
-// plus 2 dt |v|, from the positions and velocities just written; valid when
-// every site belongs to a rigid molecule.
+// slots != nullptr (captured all-rigid steps): also the skin check's largest
+// displacement since the last build, from the positions just written.
 // With xq set (captured all-rigid steps) the kick also does the force
 // evaluation's position refresh for its sites - FP32 positions, the P3M mesh
 // records of the charged ones, cleared fixed-point force rows (read above)
 // and, in workgroup 0, the cleared energy / virial accumulators - so no
 // separate refresh launch is needed (a rebuild's permutation rewrites xq and
 // the records in the new order).
-struct RefreshArgs {
-    float4 *xq;
-    float4 *rec;
-    const float *q;
-    unsigned long long *force;
-    unsigned long long *acc;
-    int nacc;
-};
-
 __device__ __forceinline__ void rigid_vv1_body(int blk, int nblk, RigidArgs r, double4 *__restrict__ pos, double4 *__restrict__ vel,
                                                    const unsigned long long *__restrict__ f,
-                                                   const double4 *__restrict__ last, double dt2,
-                                                   float *__restrict__ part, DecideArgs da, RefreshArgs ra) {
+                                                   const double4 *__restrict__ last, unsigned *__restrict__ slots,
+                                                   RefreshArgs ra) {
     r.g = r.bx->geo;
     const int m = blk * blockDim.x + threadIdx.x;
-    float d2 = 0.f, p2 = 0.f;
+    float d2 = 0.f;
     if (ra.xq && blk == 0)
         for (int k = threadIdx.x; k < ra.nacc; k += blockDim.x) ra.acc[k] = 0ull;
     if (m < r.nmol) {
@@ -206,68 +182,33 @@ __device__ __forceinline__ void rigid_vv1_body(int blk, int nblk, RigidArgs r, d
     vel[a.x] = make_double4(vO.x, vO.y, vO.z, wO.w);
     vel[a.y] = make_double4(vH1.x, vH1.y, vH1.z, wH1.w);
     vel[a.z] = make_double4(vH2.x, vH2.y, vH2.z, wH2.w);
-    double4 sp[4], sv[4];
+    double4 sp[4];
     sp[0] = make_double4(nO.x, nO.y, nO.z, pO.w);
     sp[1] = make_double4(nH1.x, nH1.y, nH1.z, pH1.w);
     sp[2] = make_double4(nH2.x, nH2.y, nH2.z, pH2.w);
-    sv[0] = make_double4(vO.x, vO.y, vO.z, wO.w);
-    sv[1] = make_double4(vH1.x, vH1.y, vH1.z, wH1.w);
-    sv[2] = make_double4(vH2.x, vH2.y, vH2.z, wH2.w);
     if (a.w >= 0) {
         const d3 nM = nO + (0.5 * (1.0 - r.gamma)) * ((B3 - A3) + (C3 - A3));
         const double4 pM = pos[a.w];
         sp[3] = make_double4(nM.x, nM.y, nM.z, pM.w);
-        sv[3] = make_double4(0.0, 0.0, 0.0, vel[a.w].w);
         pos[a.w] = sp[3];
-        vel[a.w] = sv[3];
+        vel[a.w] = make_double4(0.0, 0.0, 0.0, vel[a.w].w);
     }
     if (ra.xq) {
         const int site[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             if (site[s] < 0) continue;
-            const double4 p = sp[s];
-            const float qs = ra.q[site[s]];
-            ra.xq[site[s]] = make_float4((float)(p.x - r.g.lo[0]), (float)(p.y - r.g.lo[1]), (float)(p.z - r.g.lo[2]), qs);
-            if (ra.rec && qs != 0.0f) ra.rec[site[s]] = mesh_record(p, r.bx->mesh);
-            ra.force[3 * (size_t)site[s] + 0] = 0ull;
-            ra.force[3 * (size_t)site[s] + 1] = 0ull;
-            ra.force[3 * (size_t)site[s] + 2] = 0ull;
+            refresh_site(ra, site[s], sp[s], r.bx, r.g);
         }
     }
-    if (part) {
+    if (slots) {
         const int site[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            if (site[s] < 0) continue;
-            const double dd = disp2(sp[s], last[site[s]], r.g);
-            const double4 v = sv[s];
-            const double p = sqrt(dd) + dt2 * sqrt(v.x * v.x + v.y * v.y + v.z * v.z);
-            d2 = fmaxf(d2, (float)dd);
-            p2 = fmaxf(p2, (float)(p * p));
-        }
+        for (int s = 0; s < 4; ++s)
+            if (site[s] >= 0) d2 = fmaxf(d2, (float)disp2(sp[s], last[site[s]], r.g));
     }
     }
-    if (part) {
-        __shared__ float red[2][2];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            d2 = fmaxf(d2, __shfl_xor(d2, o, 64));
-            p2 = fmaxf(p2, __shfl_xor(p2, o, 64));
-        }
-        const int w = threadIdx.x >> 6;
-        if ((threadIdx.x & 63) == 0) {
-            red[0][w] = d2;
-            red[1][w] = p2;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            part[2 * blk] = fmaxf(red[0][0], red[0][1]);
-            part[2 * blk + 1] = fmaxf(red[1][0], red[1][1]);
-        }
-        // the step's decisions in the last workgroup (one launch fewer)
-        if (da.ticket && last_block(da.ticket, nblk)) decide_wg(nblk, da);
-    }
+    if (slots) disp_fold(d2, slots, blk);
 }
 
 // kick = false: only the velocity constraint and the M placement (start of a run)
@@ -365,9 +306,8 @@ __device__ __forceinline__ void rigid_vv2_body(int blk, int nblk, RigidArgs r, d
 
 // molecule -> current site indices, and the per-site membership flag that
 // keeps the plain integrator off these sites
-__device__ __forceinline__ void rigid_map_body(int blk, int nblk, const int *__restrict__ gate, int nmol, const int4 *__restrict__ ids, const int *__restrict__ idToIdx,
+__device__ __forceinline__ void rigid_map_body(int blk, int nblk, int nmol, const int4 *__restrict__ ids, const int *__restrict__ idToIdx,
                             int4 *__restrict__ atoms, int *__restrict__ member) {
-    if (gate && *gate == 0) return;
     const int m = blk * blockDim.x + threadIdx.x;
     if (m >= nmol) return;
     const int4 i = ids[m];
@@ -492,46 +432,27 @@ void dilate(Ctx &c, const int *gate) {
 
 void rigid_map(Ctx &c) {
     if (!c.rigid.on) return;
-    // captured list rebuilds clear member in k_copy_back and, with E3B on,
-    // map the molecules in the E3B map kernel (fewer gated launches per step)
-    if (c.capture && c.e3b.on) return;
-    if (!c.capture) fill_int(c, c.rigid.member, c.n, 0, nullptr);
-    launch<rigid_map_body, 128>(c, cdiv(c.rigid.nmol, 128), 0, rebuild_gate(c), c.rigid.nmol, c.rigid.ids, c.idToIdx, c.rigid.atoms, c.rigid.member);
-}
-
-int fused_check_blocks(const Ctx &c) {
-    const int nb = cdiv(c.rigid.nmol, 128);
-    return c.rigid.on && c.rigid.nsites == c.n && nb <= kCheckBlocks ? nb : 0;
+    // list rebuilds clear member in the sort and map the molecules in the
+    // build's launch; this is the map of a new set-up
+    fill_int(c, c.rigid.member, c.n, 0, nullptr);
+    launch<rigid_map_body, 128>(c, cdiv(c.rigid.nmol, 128), 0, c.rigid.nmol, c.rigid.ids, c.idToIdx, c.rigid.atoms, c.rigid.member);
 }
 
 void rigid_first_half(Ctx &c) {
-    RigidArgs r = make_args(c);
-    // captured steps of all-rigid systems: the skin check's partial maxima
-    // here, and the step's decisions in the launch's last workgroup
-    const bool chk = c.fuseCheck && fused_check_blocks(c) > 0;
-    DecideArgs da{};
+    const RigidArgs r = make_args(c);
     RefreshArgs ra{};
-    if (chk && c.fuseStep) {
-        da = decide_args(c);
-        da.ticket = c.dFlags + 10;
-        c.decided = true;
-        ra.xq = c.xq;
-        ra.rec = c.pppm.on && c.hasCharges ? c.meshRec : nullptr;
-        ra.q = c.q[c.cur];
-        ra.force = c.force;
-        ra.acc = c.acc;
-        ra.nacc = kAccTotal;
-        c.refreshed = true;
-    }
-    launch<rigid_vv1_body, 128>(c, cdiv(r.nmol, 128), 0, r, c.pos[c.cur], c.vel[c.cur], c.force, c.posLast, 2.0 * c.dt, chk ? c.checkPart : nullptr, da, ra);
+    if (c.fuseCheck) ra = refresh_args(c);
+    launch<rigid_vv1_body, 128>(c, cdiv(r.nmol, 128), 0, r, c.pos[c.cur], c.vel[c.cur], c.force, c.posLast, c.fuseCheck ? c.dispSlots : nullptr, ra);
 }
 
 void rigid_second_half(Ctx &c, bool kick) {
     RigidArgs r = make_args(c);
     BaroFuse bf{};
     // a captured all-rigid barostat step: the pressure, box and alpha in the
-    // last workgroup (the molecular virial and M V^2 are summed here)
-    if (kick && c.fuseMolVirial && c.fuseStep && c.baro.on && c.capture) {
+    // last workgroup (the molecular virial and M V^2 are summed here), while
+    // its ticket, about 24 ns a workgroup, costs no more than a launch (1.6 us
+    // plus the start of a wave)
+    if (kick && c.fuseMolVirial && c.fuseStep && c.baro.on && c.capture && cdiv(r.nmol, 128) <= 96) {
         bf.ticket = c.dFlags + 9;
         bf.gate = baro_gate(c);
         bf.bx = c.box;

@@ -1,0 +1,114 @@
+"""The two-launch re-sort (bin_body, sort_body) at the shapes where it can go
+wrong, through the neighbor list it leaves: rows against the oracle bit for bit.
+
+* cells that hold far more atoms than the register and LDS paths take (a dense
+  cluster in a large box: the walk through the cell's list);
+* a grid with fewer cells than one chunk, and one with several rounds per chunk
+  (a sparse gas over hundreds of thousands of cell slots);
+* exclusion rows longer than a wave's registers;
+* captured steps of free atoms (first half kick, binning and decisions fused)
+  against the separate launches, bit for bit.
+"""
+import numpy as np
+import pytest
+
+from md_engine_amd import PAIR
+from test_gpu_parity import assert_same_lists, oracle_rows_by_id
+
+pytestmark = pytest.mark.gpu
+
+
+def say(msg):
+    print(msg, flush=True)
+
+
+def _list_engine(factory, x, L, rlist, skin, q=None):
+    e = factory()
+    e.set_system(x, np.zeros(3), L, q=q, inv_mass=np.ones(len(x)))
+    e.lj_set([[(rlist - skin) ** 2]], [[24.0]], [[1.0]])
+    e.nlist_config(rlist, skin)
+    return e
+
+
+@pytest.mark.parametrize("shape", ["cluster", "one_chunk", "sparse"])
+def test_resort_lists_exact(orc, gpu_engine_factory, shape):
+    say(f"re-sort, {shape}")
+    rng = np.random.default_rng(5)
+    if shape == "cluster":
+        # 3,000 atoms in one cell (beyond the 2,048 ranked in LDS), 500 around them
+        L = np.full(3, 24.0)
+        x = np.concatenate([rng.uniform(11.0, 11.2, (3000, 3)), rng.uniform(0, 24, (500, 3))])
+        rlist = 2.5
+    elif shape == "one_chunk":
+        L = np.array([6.1, 6.3, 7.0])
+        x = rng.uniform(0, 1, (333, 3)) * L
+        rlist = 2.9
+    else:
+        # 2 x (124 x 124 x 249) cell slots: several rounds of 256 cells per workgroup
+        L = np.full(3, 125.0)
+        x = rng.uniform(0, 125, (20011, 3))
+        rlist = 2.0
+    q = np.where(rng.random(len(x)) < 0.4, 0.3, 0.0)
+    if shape == "cluster":
+        q[:3000] = 0.0  # one cell slot
+    e = _list_engine(gpu_engine_factory, x, L, rlist, 0.3, q=q)
+    for k in range(2):  # the second build starts from the first one's order
+        e.nlist_update(force=True)
+        gc, grows = e.nlist_get()
+        oc, orows, _ = oracle_rows_by_id(orc, x, np.zeros(3), L, rlist, brute=False)
+        assert_same_lists(gc, grows, oc, orows)
+        x = x + rng.normal(0, 0.2, x.shape)
+        e.set_positions(x)
+    e.close()
+
+
+def test_long_exclusion_rows(orc, gpu_engine_factory):
+    """Rows of 3, 70 and 100 exclusions: registers, LDS and beyond one per lane."""
+    say("long exclusion rows")
+    rng = np.random.default_rng(6)
+    n, L = 400, np.full(3, 9.0)
+    x = rng.uniform(0, 9, (n, 3))
+    e = _list_engine(gpu_engine_factory, x, L, 2.5, 0.3)
+    partners = [set() for _ in range(n)]
+    for i, m in ((3, 3), (50, 70), (51, 100)):
+        for j in rng.choice([k for k in range(100, n)], m, replace=False):
+            partners[i].add(int(j))
+            partners[int(j)].add(i)
+    off = np.concatenate([[0], np.cumsum([len(p) for p in partners])]).astype(np.int32)
+    tagged = np.array([j | (1 + j % 3) << 30 for p in partners for j in sorted(p)], np.uint32)
+    e.exclusions_set(off, tagged)
+    e.nlist_update(force=True)
+    gc, grows = e.nlist_get()
+    tags = {(i, j): 1 + j % 3 for i in range(n) for j in partners[i]}
+    oc, orows, _ = oracle_rows_by_id(orc, x, np.zeros(3), L, 2.5, brute=True)
+    for i in range(n):
+        want = [int(r) & 0x3FFFFFFF for r in orows[i]]
+        assert [int(r) for r in grows[i]] == [j | (tags.get((i, j), 0) << 30) for j in want], i
+    e.close()
+
+
+@pytest.mark.parametrize("n", [256, 257, 4000])
+def test_fused_first_half_equals_separate(orc, gpu_engine_factory, n):
+    """Free atoms, captured steps: kick, check, decisions and refresh in one
+    launch give the separate launches' trajectory bit for bit."""
+    say(f"fused first half, {n} atoms")
+    from md_engine_amd import systems
+
+    x, L, lo = systems.fcc_lj(10, 0.8442)
+    x = x[:n] if n == 4000 else x[np.random.default_rng(1).choice(4000, n, replace=False)]
+    v = systems.maxwell_boltzmann(np.ones(n), 1.2, seed=4)
+    out = []
+    for fuse in (1, 0):
+        e = gpu_engine_factory()
+        e.set_system(x, lo, L, v=v, inv_mass=np.ones(n))
+        e.lj_set([[6.25]], [[24.0]], [[1.0]])
+        e.nlist_config(2.8, 0.3)
+        e.integrator_set(0.005, 1.0)
+        e.option("fuse_step", fuse)
+        e.run(150, PAIR)
+        st = e.nlist_stats()
+        out.append((*e.get_system(), st["rebuilds"], st["violations"]))
+        e.close()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    assert out[0][2] == out[1][2] and out[0][2] > 3
+    assert out[0][3] == 0
