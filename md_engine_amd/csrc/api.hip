@@ -157,19 +157,6 @@ double pressure_now(Ctx &c) {
     return (v(ACC_MOL + 1) * c.baro.mvv + W - v(ACC_MOL)) / (3.0 * vol) * c.baro.nktv2p;
 }
 
-// FixPressureBerendsen::stepFinal (src/Fixes/FixPressureBerendsen.cu): mu =
-// (1 - dt/period (P0 - P)/B)^(1/3) clamped to 1 -+ maxDilation, applied to
-// the box about its centre and to the centres of mass; the cell grid is set
-// up again when its cell count would change, P3M refreshes alpha and G.
-bool regrid_if_needed(Ctx &c);
-
-void barostat_apply(Ctx &c) {
-    acc_clear(c, ACC_MOL, 2);  // the captured step relies on the per-step clear instead
-    baro_step(c, nullptr);
-    box_pull(c);
-    regrid_if_needed(c);
-}
-
 // After the box changed on the device: set the grid up again when a cell edge
 // fell below r_list / reach (the list would miss pairs) or the box grew by a
 // whole cell (finer cells are cheaper).
@@ -187,6 +174,24 @@ bool regrid_if_needed(Ctx &c) {
     return regrid;
 }
 
+// True when no dilation of `steps` barostat applications can make
+// regrid_if_needed set the grid up again: every cell edge stays above
+// r_list / reach and no axis grows by a cell (factors 1 -+ maxDilation a step,
+// with a part in 10^9 of slack for rounding).  Reading the box back after
+// every application waits for the GPU (39 us of a 250 us step).
+bool box_keeps_grid(const Ctx &c, int steps) {
+    const double up = std::pow(1.0 + c.baro.maxDil, steps) * (1.0 + 1e-9);
+    const double down = std::pow(1.0 - c.baro.maxDil, steps) * (1.0 - 1e-9);
+    for (int d = 0; d < 3; ++d) {
+        const double edge = c.rlist / c.reach[d] * (1.0 + 1e-9), L = c.geo.L[d];
+        if (c.geo.periodic[d] && (L * down < c.nc[d] * edge || c.rlist >= 0.5 * L * down)) return false;
+        if (std::max(1, (int)std::floor(L * up * grid_headroom(c) / edge)) > c.nc[d]) return false;
+    }
+    return true;
+}
+
+constexpr int kForkSites = 65536;
+
 void compute(Ctx &c, int flags) {
     const bool energy = flags & MDX_ENERGY;
     // a trace-only request still gets the full tensor from the terms that
@@ -203,7 +208,11 @@ void compute(Ctx &c, int flags) {
     // on the side stream beside the pair and E3B kernels: all three start
     // from the refreshed positions and add into the fixed-point force and
     // accumulator buffers, whose integer sums do not depend on the order.
-    const bool fork = mesh && c.capture && !c.rec && c.side && c.meshStream;
+    // Outside a graph the fork and the join are two cross-stream waits of about
+    // 10 us each, which only large systems get back (2,048 sites 88 -> 106 us a
+    // step, 16,384 145 -> 167, 32,768 210 -> 209, 131,072 544 -> 501).
+    const bool eagerFork = c.inRun && !c.prof && c.n >= kForkSites;
+    const bool fork = mesh && (c.capture || eagerFork) && !c.rec && c.side && c.meshStream;
     const bool forked = c.forked;  // recorded by this step's rebuild after its copy-back
     c.forked = false;
     if (fork) {
@@ -358,8 +367,8 @@ void snapshot_restore(Ctx &c) {
     }
 }
 
-// Reads the dMax slot written one step earlier (waits only for that step's
-// check, while later work keeps the GPU busy).  Returns the rebuild decision
+// Reads the check of one step earlier (waits only for that step's check,
+// while later work keeps the GPU busy).  Returns the rebuild decision
 // for the current step and counts a violation when the list of the step
 // that was checked was already older than the skin allows.
 bool lagged_rebuild_decision(Ctx &c, int parity) {
@@ -372,12 +381,19 @@ bool lagged_rebuild_decision(Ctx &c, int parity) {
     return std::sqrt((double)p2) > half;
 }
 
-void check_and_copy(Ctx &c, int parity) {
-    check_max(c, parity);
-    MDX_HIP(hipMemcpyAsync(c.pinned + 2 + 2 * parity, c.dMax + 2 * parity, sizeof(unsigned) * 2,
-                           hipMemcpyDeviceToHost, c.stream));
+// The skin check of the current positions into pinned slot `parity` and its
+// event; fused: from the maxima the first half kick left.
+void check_step(Ctx &c, int parity, bool fused) {
+    if (fused) check_out(c, parity);
+    else check_max(c, parity);
     MDX_HIP(hipEventRecord(c.stepEvent[parity], c.stream));
 }
+
+// A step of all-rigid molecules or of free atoms: the first half kick also
+// refreshes the positions of the force evaluation and measures the
+// displacements (flexible molecules place their M sites in between).
+bool fuses_check(const Ctx &c) { return c.fuseStep && !c.flex.on && (!c.rigid.on || c.rigid.nsites == c.n); }
+bool all_rigid(const Ctx &c) { return c.rigid.on && c.rigid.nsites == c.n && !c.nh.on; }
 
 template <class T>
 void upload(Ctx &c, T *dst, const T *src, size_t count) {
@@ -399,13 +415,9 @@ void captured_step(Ctx &c, int fflags) {
     // all-water systems without a Nose-Hoover chain: the rigid second half
     // sums the molecular virial terms and the thermostat's m v^2 (no separate
     // passes over the molecules; k_decide clears the m v^2 sum)
-    const bool allRigid = c.rigid.on && c.rigid.nsites == c.n && !c.nh.on;
-    c.fuseMolVirial = c.baro.on && allRigid;
-    c.fuseThermo = c.thermoOn && allRigid;
-    // all-rigid systems and free atoms: the first half refreshes the positions
-    // of the force evaluation and measures the displacements for the binning
-    // (flexible molecules place their M sites between the drift and the refresh)
-    c.fuseCheck = c.fuseStep && !c.flex.on && (!c.rigid.on || c.rigid.nsites == c.n);
+    c.fuseMolVirial = c.baro.on && all_rigid(c);
+    c.fuseThermo = c.thermoOn && all_rigid(c);
+    c.fuseCheck = fuses_check(c);
     integrate_first_half(c);
     decide_step(c);
     nlist_rebuild_async(c);  // every kernel gated by dFlags[3]
@@ -815,6 +827,14 @@ hipGraphExec_t capture_merged(const std::vector<Ctx *> &cs, int steps, int fflag
     return exec;
 }
 
+// the second stream of a run's steps, at the default priority like the main one
+void mesh_stream_make(Ctx &c) {
+    if (!c.meshStream || c.side) return;
+    MDX_HIP(hipStreamCreateWithFlags(&c.side, hipStreamNonBlocking));
+    MDX_HIP(hipEventCreateWithFlags(&c.evFork, hipEventDisableTiming));
+    MDX_HIP(hipEventCreateWithFlags(&c.evJoin, hipEventDisableTiming));
+}
+
 hipGraphExec_t capture_steps(const std::vector<Ctx *> &cs, int steps, int fflags, const RingSpec *ring = nullptr,
                              BatchKeep *keep = nullptr) {
     if (cs.size() > 1 && keep && cs[0]->batchMerge) {
@@ -823,11 +843,7 @@ hipGraphExec_t capture_steps(const std::vector<Ctx *> &cs, int steps, int fflags
     }
     Ctx &c0 = *cs[0];
     for (Ctx *c : cs)
-        if (c->pppm.on && c->meshStream && !c->side) {  // default priority, like the main stream
-            MDX_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
-            MDX_HIP(hipEventCreateWithFlags(&c->evFork, hipEventDisableTiming));
-            MDX_HIP(hipEventCreateWithFlags(&c->evJoin, hipEventDisableTiming));
-        }
+        if (c->pppm.on) mesh_stream_make(*c);
     std::vector<hipEvent_t> evs(cs.size() * 2, nullptr);
     for (auto &e : evs) MDX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     std::vector<bool> prof(cs.size());
@@ -1034,7 +1050,6 @@ void run_captured(const std::vector<Ctx *> &cs, int nsteps, int flags, const Rin
                     else compute(c, fflags);
                 }
                 // chunk state: displacement slots, running row maxima, counters, turn
-                fill_int(c, (int *)c.dMax, 4, 0);
                 fill_int(c, (int *)c.dispSlots, kDispSlots * kDispStride, 0);
                 fill_int(c, c.dFlags + 1, 5, 0);
                 // device turn counter: the thermostat and barostat gates take it
@@ -1311,7 +1326,6 @@ int mdx_create(int device, mdx_ctx **out) {
         pppm_scratch_init(c.device);  // device address of the no-allocation entry point's scratch
         c.acc = dalloc<unsigned long long>(c, kAccTotal);
         c.dFlags = dalloc<int>(c, 12);
-        c.dMax = dalloc<unsigned>(c, 4);
         c.dispSlots = dalloc<unsigned>(c, kDispSlots * kDispStride);
         c.checkPart = dalloc<float>(c, 2 * kCheckBlocks);
         c.thermo = dalloc<unsigned long long>(c, 2);
@@ -1319,7 +1333,6 @@ int mdx_create(int device, mdx_ctx **out) {
         std::memset(c.pinned, 0, sizeof(int) * 8);
         MDX_HIP(hipEventCreateWithFlags(&c.capEvent, hipEventDisableTiming));
         for (int k = 0; k < 2; ++k) MDX_HIP(hipEventCreateWithFlags(&c.stepEvent[k], hipEventDisableTiming));
-        MDX_HIP(hipMemsetAsync(c.dMax, 0, sizeof(unsigned) * 4, c.stream));
         MDX_HIP(hipMemsetAsync(c.dFlags, 0, sizeof(int) * 12, c.stream));
         MDX_HIP(hipMemsetAsync(c.acc, 0, sizeof(unsigned long long) * kAccTotal, c.stream));
     });
@@ -2057,8 +2070,9 @@ int mdx_run(mdx_ctx *ctx, int nsteps, int flags) {
         struct InRun {
             Ctx &c;
             explicit InRun(Ctx &c_) : c(c_) { c.inRun = true; }
-            ~InRun() { c.inRun = false; }
+            ~InRun() { c.inRun = c.refreshed = c.baroFused = c.fuseCheck = c.fuseMolVirial = c.fuseThermo = false; }
         } inRun(c);
+        if (c.pppm.on && c.n >= kForkSites) mesh_stream_make(c);
         constexpr int kChunk = 64;
         int done = 0, chunkNo = 0;
         bool forcedDone = false;
@@ -2070,26 +2084,38 @@ int mdx_run(mdx_ctx *ctx, int nsteps, int flags) {
                 ensure_list(c);
                 compute(c, fflags);
             }
-            // the "previous step" check for step 0 of the chunk, from cleared slots
-            fill_int(c, (int *)c.dMax, 4, 0);
-            check_and_copy(c, 1);
+            fill_int(c, (int *)c.dispSlots, kDispSlots * kDispStride, 0);
+            fill_int(c, c.dFlags + 1, 2, 0);
+            check_step(c, 1, false);  // the "previous step" check for step 0 of the chunk
+            // the host follows the device box step by step only where the
+            // chunk's largest dilation could change the cell grid
+            const bool boxSafe = c.baro.on && box_keeps_grid(c, len);
             for (int s = 0; s < len; ++s) {
                 const int par = s & 1;
                 const bool baro = c.baro.on && (c.turn + 1) % c.baro.every == 0;
+                const bool thermo = c.thermoOn && (c.turn + 1) % c.thermoEvery == 0;
+                c.fuseCheck = fuses_check(c);
                 integrate_first_half(c);
-                if (lagged_rebuild_decision(c, 1 - par)) nlist_rebuild_async(c);
-                check_and_copy(c, par);
+                if (c.fuseCheck) check_step(c, par, true);
+                const bool rebuild = lagged_rebuild_decision(c, 1 - par);
+                if (rebuild) nlist_rebuild_async(c);
+                // displacements from the list in use: again after a rebuild
+                if (rebuild || !c.fuseCheck) check_step(c, par, false);
                 compute(c, fflags | (baro ? kFlagVirialTrace : 0));
                 integrate_second_half(c);
                 ++c.turn;
-                if (c.thermoOn && c.turn % c.thermoEvery == 0) thermostat_apply(c);
+                c.fuseCheck = false;
+                if (thermo) thermostat_apply(c);
                 if (baro) {
-                    barostat_apply(c);
+                    baro_step(c, nullptr);
+                    if (!boxSafe) {
+                        box_pull(c);
+                        regrid_if_needed(c);
+                    }
                     if (!c.listValid) {
                         ensure_list(c);
                         compute(c, fflags);
-                        fill_int(c, (int *)c.dMax, 4, 0);
-                        check_and_copy(c, par);
+                        check_step(c, par, false);
                     }
                 }
             }
@@ -2097,6 +2123,7 @@ int mdx_run(mdx_ctx *ctx, int nsteps, int flags) {
             lagged_rebuild_decision(c, (len - 1) & 1);  // count a violation in the last step
             const bool forced = !forcedDone && c.replayChunk == chunkNo + 1;
             forcedDone = forcedDone || forced;
+            if (c.baro.on) box_pull(c);
             if (!capacity_ok(c) || forced) {
                 // a build overflowed its rows: redo the chunk with the grown rows
                 snapshot_restore(c);

@@ -103,7 +103,7 @@ BaroArgs baro_args(const Ctx &c) {
     ba.q2 = c.pppm.totalQ2;
     ba.rcut = c.pppm.rcut;
     for (int a = 0; a < 3; ++a) ba.minL[a] = c.nc[a] * (c.rlist / c.reach[a] * (1.0 + 1e-9));
-    ba.rescaled = c.fuseMolVirial && c.thermoOn ? 1 : 0;
+    ba.rescaled = c.fuseMolVirial && c.fuseThermo ? 1 : 0;
     ba.tmode = c.thermoTau > 0 ? 1 : 0;
     ba.tgate = thermo_gate(c);
     ba.thermo = c.thermo;

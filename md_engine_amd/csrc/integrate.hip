@@ -44,21 +44,21 @@ __device__ __forceinline__ void vv1_body(int blk, int nblk, int n, double4 *__re
     pos[i] = x;
 }
 
-// The first half kick and drift of a captured step of free atoms, with what
+// The first half kick and drift of a run's step of free atoms, with what
 // the all-rigid first half also does: the force evaluation's position refresh
-// (RefreshArgs) and the skin check's largest displacement.  One launch and one
+// (RefreshArgs) and the skin check's maxima.  One launch and one
 // pass over the state instead of four (kick, check, decisions, refresh; 14.2 +
 // 9.4 + 4.9 + 8.2 us for 500,000 atoms, all of it bandwidth, and three of the
 // twelve launches of a small fluid's step).
 __device__ __forceinline__ void vv1_step_body(int blk, int nblk, int n, double4 *__restrict__ pos,
                                               double4 *__restrict__ vel, double hdtf, double dt,
-                                              const double4 *__restrict__ last, const BoxDev *__restrict__ bx,
-                                              unsigned *__restrict__ slots, RefreshArgs ra) {
+                                              const double4 *__restrict__ last, double dt2,
+                                              const BoxDev *__restrict__ bx, unsigned *__restrict__ slots,
+                                              RefreshArgs ra) {
     const Geometry g = bx->geo;
-    if (blk == 0)
-        for (int k = threadIdx.x; k < ra.nacc; k += blockDim.x) ra.acc[k] = 0ull;
+    if (blk == 0) refresh_clear(ra);
     const int i = blk * blockDim.x + threadIdx.x;
-    float d2 = 0.f;
+    float d2 = 0.f, p2 = 0.f;
     if (i < n) {
         double4 v = vel[i], x = pos[i];
         const double4 x0 = last[i];
@@ -74,9 +74,12 @@ __device__ __forceinline__ void vv1_step_body(int blk, int nblk, int n, double4 
             pos[i] = x;
         }
         refresh_site(ra, i, x, bx, g);
-        d2 = (float)disp2(x, x0, g);
+        const double dd = disp2(x, x0, g);
+        const double p = sqrt(dd) + dt2 * sqrt(v.x * v.x + v.y * v.y + v.z * v.z);
+        d2 = (float)dd;
+        p2 = (float)(p * p);
     }
-    disp_fold(d2, slots, blk);
+    disp_fold(d2, p2, slots, blk);
 }
 
 // half kick only (the drift of a ring polymer is its normal-mode propagation)
@@ -284,7 +287,7 @@ void integrate_first_half(Ctx &c) {
     const int threads = 256;
     if (c.nh.on) nh_half(c, false);
     if (c.fuseCheck && !c.rigid.on) {
-        launch<vv1_step_body, 256>(c, cdiv(c.n, threads), 0, c.n, c.pos[c.cur], c.vel[c.cur], 0.5 * c.dt * c.ftmToV, c.dt, c.posLast, c.box, c.dispSlots, refresh_args(c));
+        launch<vv1_step_body, 256>(c, cdiv(c.n, threads), 0, c.n, c.pos[c.cur], c.vel[c.cur], 0.5 * c.dt * c.ftmToV, c.dt, c.posLast, 2.0 * c.dt, c.box, c.dispSlots, refresh_args(c));
         return;
     }
     const int *member = c.rigid.on ? c.rigid.member : nullptr;

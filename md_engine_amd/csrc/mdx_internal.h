@@ -453,7 +453,7 @@ struct Ctx {
     bool vtrace = false;  // set by compute for the terms it launches
     bool fuseMolVirial = false;  // captured barostat steps: rigid second half sums ACC_MOL
     bool fuseThermo = false;     // captured thermostat steps: rigid second half sums m v^2
-    bool fuseCheck = false;      // captured steps: the first half gives the skin check's maxima, the binning decides
+    bool fuseCheck = false;      // the first half refreshes and gives the skin check's maxima (captured: the binning decides)
     bool deferMSpread = false;   // compute leaves the M-site forces for a later flex_spread_m (ring contraction)
     hipStream_t stream = nullptr;
     // second stream of captured steps: the P3M chain runs beside the pair and
@@ -529,10 +529,9 @@ struct Ctx {
     bool baroFused = false;       // the rigid second half of this captured step ran the barostat step
     bool fuseStep = true;         // option "fuse_step": captured steps fold small launches into others
     int graphSteps = 0;           // mdx_run: 1 = captured steps (option "graph")
-    unsigned *dMax = nullptr;     // 2 slots x (max |x - x_last|^2, max predicted^2) as float bits
-    unsigned *dispSlots = nullptr; // captured steps: max |x - x_last|^2 as float bits, kDispSlots words a line apart
+    unsigned *dispSlots = nullptr; // max |x - x_last|^2 and max predicted^2 as float bits, kDispSlots pairs a line apart
     float *checkPart = nullptr;   // per-workgroup maxima of the displacement check (2 x kCheckBlocks)
-    int *pinned = nullptr;        // host-pinned: [0..1] last build's max counts, [2..5] dMax copies, [6] stream overflow
+    int *pinned = nullptr;        // host-pinned: [0..1] last build's max counts, [2..5] two skin checks (d^2, predicted^2), [6] stream overflow; written by kernels
     hipEvent_t capEvent = nullptr;
     bool capPending = false;
     long long listViolations = 0; // steps whose list was older than the skin allows
@@ -924,7 +923,6 @@ constexpr int kDispSlots = 32, kDispStride = 16;
 struct DecideArgs {
     const float *part;           // decide_body: per-workgroup maxima
     unsigned *slots;             // bin_body: the maxima words, nullptr when decide_body took the decisions
-    unsigned *dmax;
     int *flags;
     float half2;
     int every, baroEvery;
@@ -959,23 +957,32 @@ __device__ __forceinline__ void decide_write(const DecideArgs &d, bool rebuild) 
         d.thermo[1] = 0ull;
     }
     flags[8] = (d.baroEvery > 0 && turn % d.baroEvery == 0) ? 1 : 0;
-    d.dmax[0] = 0u;
-    d.dmax[1] = 0u;
 }
 
-// a workgroup's largest squared displacement (a lane value per thread) into
-// its word: non-negative floats order like their bit patterns
-__device__ __forceinline__ void disp_fold(float d2, unsigned *slots, int blk) {
+// a workgroup's maxima (lane values d2, p2) into its words: non-negative
+// floats order like their bit patterns
+__device__ __forceinline__ void disp_fold(float d2, float p2, unsigned *slots, int blk) {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) d2 = fmaxf(d2, __shfl_xor(d2, o, 64));
-    if ((threadIdx.x & 63) == 0)
-        atomicMax(&slots[((blk + (threadIdx.x >> 6)) & (kDispSlots - 1)) * kDispStride], __float_as_uint(d2));
+    for (int o = 32; o > 0; o >>= 1) {
+        d2 = fmaxf(d2, __shfl_xor(d2, o, 64));
+        p2 = fmaxf(p2, __shfl_xor(p2, o, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        unsigned *w = slots + ((blk + (threadIdx.x >> 6)) & (kDispSlots - 1)) * kDispStride;
+        atomicMax(w, __float_as_uint(d2));
+        atomicMax(w + 1, __float_as_uint(p2));
+    }
 }
-__device__ __forceinline__ float disp_max(const unsigned *slots) {
-    float d2 = __uint_as_float(slots[(threadIdx.x & (kDispSlots - 1)) * kDispStride]);
+__device__ __forceinline__ float disp_max(const unsigned *slots, int word = 0) {
+    float d2 = __uint_as_float(slots[(threadIdx.x & (kDispSlots - 1)) * kDispStride + word]);
 #pragma unroll
     for (int o = kDispSlots / 2; o > 0; o >>= 1) d2 = fmaxf(d2, __shfl_xor(d2, o, 64));
     return d2;
+}
+
+// a word of pinned host memory that the host reads after an event
+__device__ __forceinline__ void host_store(int *p, int v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // True in the last workgroup of a launch to get here (every thread of every
@@ -1023,6 +1030,9 @@ struct RefreshArgs {
     int nacc;
 };
 RefreshArgs refresh_args(Ctx &c);  // for this context, marking the refresh as done
+__device__ __forceinline__ void refresh_clear(const RefreshArgs &ra) {  // one workgroup
+    for (int k = threadIdx.x; k < ra.nacc; k += blockDim.x) ra.acc[k] = 0ull;
+}
 __device__ __forceinline__ void refresh_site(const RefreshArgs &ra, int i, const double4 &p, const BoxDev *bx,
                                              const Geometry &g) {
     const float qs = ra.q[i];
@@ -1132,7 +1142,8 @@ void nlist_rebuild_async(Ctx &c);     // rebuild now; capacity checked later (ca
 bool capacity_ok(Ctx &c);             // false: rows grew, results since the last check are invalid
 bool grow_if_needed(Ctx &c);
 constexpr int kCheckBlocks = 512;     // workgroups of the displacement check
-void check_max(Ctx &c, int parity);   // max displacement / speed into dMax slot `parity`
+void check_max(Ctx &c, int parity);   // max displacement / prediction into pinned slot `parity`
+void check_out(Ctx &c, int parity);   // the same from the words a fused first half left
 void decide_step(Ctx &c);             // captured step: device rebuild / thermostat gates
 void skin_check(Ctx &c);              // the displacement check's partial maxima only
 void skin_decide(Ctx &c);             // the decisions from them (a ring's table when set)

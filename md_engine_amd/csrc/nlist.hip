@@ -216,7 +216,10 @@ __device__ __forceinline__ void place_atom(const SortArgs &a, int o, int k, int 
 constexpr int kSortThreads = 256;
 constexpr int kSortCap = 2048;  // atoms a round ranks in LDS
 __device__ __forceinline__ void sort_body(int blk, int nblk, const int *__restrict__ gate, SortArgs a) {
-    if (a.slots && blk == 0 && threadIdx.x < kDispSlots) a.slots[threadIdx.x * kDispStride] = 0u;
+    if (a.slots && blk == 0 && threadIdx.x < kDispSlots) {
+        a.slots[threadIdx.x * kDispStride] = 0u;
+        a.slots[threadIdx.x * kDispStride + 1] = 0u;
+    }
     if (gate && *gate == 0) return;
     __shared__ int sIdx[kSortCap], sKey[kSortCap];
     __shared__ unsigned char sCell[kSortCap];
@@ -1108,11 +1111,18 @@ __device__ __forceinline__ void fill_int_body(int blk, int nblk, const int *__re
 }
 
 // Longest pair row and molecule row of the build from the per-wave slots,
-// folded into the running maxima flags[1], flags[2] (one workgroup).
+// folded into the running maxima flags[1], flags[2] (one workgroup), and, for
+// an eager build, with the stream overflow bits into the host's pinned words.
 __device__ __forceinline__ void row_max_body(int blk, int nblk, const int *__restrict__ gate, int na, const int *__restrict__ a,
-                                                  int nb, const int *__restrict__ b, int *__restrict__ flags) {
+                                                  int nb, const int *__restrict__ b, int *__restrict__ flags,
+                                                  int *__restrict__ host) {
     if (gate && *gate == 0) return;
     row_max_wg(na, a, nb, b, flags);
+    if (host && threadIdx.x == 0) {
+        host_store(host, flags[1]);
+        host_store(host + 1, flags[2]);
+        host_store(host + 6, flags[7]);
+    }
 }
 
 uint32_t morton2(uint32_t x, uint32_t y) {
@@ -1242,6 +1252,7 @@ void nlist_setup(Ctx &c) {
     if (!c.cellNext) {
         c.cellNext = dalloc<int>(c, c.n);
         c.chunkSum = dalloc<int>(c, 2048);
+        MDX_HIP(hipMemsetAsync(c.chunkSum, 0, sizeof(int) * 2048, c.stream));
     }
     // one wave per atom (k_build_wave) measured fastest for dense water and
     // LJ alike; mdx_tune revisits the width
@@ -1282,7 +1293,7 @@ RowMaxArgs row_max_args(Ctx &c) {
 
 void row_max_flush(Ctx &c) {
     const RowMaxArgs rm = row_max_args(c);
-    if (rm.on) launch<row_max_body, 1024>(c, 1, 0, rm.gate, rm.na, rm.a, rm.nb, rm.b, rm.flags);
+    if (rm.on) launch<row_max_body, 1024>(c, 1, 0, rm.gate, rm.na, rm.a, rm.nb, rm.b, rm.flags, nullptr);
 }
 
 void prepare_forces(Ctx &c) {
@@ -1329,9 +1340,8 @@ static void run_build(Ctx &c, bool sync) {
         }
     }
     c.centroidList = cen != nullptr;
-    // the build's map workgroups clear the counts for the next binning; an
-    // eager build does not rely on an earlier one having got that far
-    if (!c.capture) fill_int(c, c.chunkSum, c.nChunk, 0);
+    // (the map workgroups of a build clear the chunk counts for the next
+    // binning; nothing between the binning and them throws)
     DecideArgs da{};
     if (c.capture && c.fuseCheck) {
         da = decide_args(c);
@@ -1407,8 +1417,8 @@ static void run_build(Ctx &c, bool sync) {
     // the wave build takes the maps as extra workgroups; the team builds launch them first
     if (!waveBuild) launch<mol_map_body, 256>(c, mm.blocks, 0, rebuild_gate(c), mm);
     for (;;) {
-        // a captured step keeps the running maximum of the chunk in dFlags[1..2]
-        if (!c.capture) fill_int(c, c.dFlags + 1, 2, 0);
+        // the builds of a run keep the running maximum of the chunk in dFlags[1..2]
+        if (!c.capture && sync) fill_int(c, c.dFlags + 1, 2, 0);
         {
             ProfScope ps(c, PK_BUILD);
             switch (c.buildTeam) {
@@ -1432,12 +1442,10 @@ static void run_build(Ctx &c, bool sync) {
             c.rowMaxPending = true;
             return;
         }
-        launch<row_max_body, 1024>(c, 1, 0, rebuild_gate(c), c.waveMaxA, c.waveMax, c.waveMaxB, c.waveMax + wave_slots_a(c), c.dFlags);
-        if (c.capture) return;  // rows checked by the host after the chunk
         // largest row counts -> pinned host memory; checked now (sync) or at
         // the next synchronisation point (capacity_ok)
-        MDX_HIP(hipMemcpyAsync(c.pinned, c.dFlags + 1, sizeof(int) * 2, hipMemcpyDeviceToHost, c.stream));
-        MDX_HIP(hipMemcpyAsync(c.pinned + 6, c.dFlags + 7, sizeof(int), hipMemcpyDeviceToHost, c.stream));
+        launch<row_max_body, 1024>(c, 1, 0, rebuild_gate(c), c.waveMaxA, c.waveMax, c.waveMaxB, c.waveMax + wave_slots_a(c), c.dFlags, c.capture ? nullptr : c.pinned);
+        if (c.capture) return;  // rows checked by the host after the chunk
         if (!sync) {
             MDX_HIP(hipEventRecord(c.capEvent, c.stream));
             c.capPending = true;
@@ -1513,9 +1521,7 @@ namespace {
 // Lag-1 rebuild decision for the step loop: per site d = |x - x_last| and the
 // prediction p = d + 2 dt |v| (an M site, moved by its molecule, never moves
 // further than its fastest heavy site); max d^2 and max p^2 over all sites go
-// into one slot of dMax as float bits (non-negative floats order like their
-// bit patterns); the other slot is cleared for the next step.  The host reads
-// the slot one step later.
+// to one of two pinned host slots.  The host reads the slot one step later.
 // Grid-stride over the sites with a workgroup reduction: one atomic pair per
 // workgroup (same-address atomics serialise in L2).
 // Per-workgroup maxima into part[2 b], part[2 b + 1] (float bits); a
@@ -1556,16 +1562,26 @@ __device__ __forceinline__ void check_part_body(int blk, int nblk, int n, const 
     }
 }
 
-// slot = max(slot, this check) as float bits; the other slot cleared for the next step
-__device__ __forceinline__ void check_reduce_body(int blk, int nblk, int nb, const float *__restrict__ part, unsigned *__restrict__ slot,
-                               unsigned *__restrict__ other) {
+// One wave: a check's maxima straight into the host's pinned words (a store
+// of the kernel; a device-to-host copy is a launch of its own and left 5 us
+// between this and the next kernel), from the per-workgroup maxima or from the
+// words of a fused first half, which it clears.
+__device__ __forceinline__ void check_reduce_body(int blk, int nblk, int nb, const float *__restrict__ part,
+                                                  unsigned *__restrict__ slots, int *__restrict__ host) {
     float d2, p2;
-    part_max(nb, part, d2, p2);
+    if (slots) {
+        d2 = disp_max(slots, 0);
+        p2 = disp_max(slots, 1);
+        if (threadIdx.x < kDispSlots) {
+            slots[threadIdx.x * kDispStride] = 0u;
+            slots[threadIdx.x * kDispStride + 1] = 0u;
+        }
+    } else {
+        part_max(nb, part, d2, p2);
+    }
     if (threadIdx.x == 0) {
-        slot[0] = max(slot[0], __float_as_uint(d2));
-        slot[1] = max(slot[1], __float_as_uint(p2));
-        other[0] = 0u;
-        other[1] = 0u;
+        host_store(host, __float_as_int(d2));
+        host_store(host + 1, __float_as_int(p2));
     }
 }
 }  // namespace
@@ -1579,7 +1595,6 @@ static void check_part(Ctx &c) {
 DecideArgs decide_args(const Ctx &c) {
     DecideArgs d{};
     d.part = c.checkPart;
-    d.dmax = c.dMax;
     d.flags = c.dFlags;
     const float half = (float)(0.5 * c.skin);
     d.half2 = half * half;
@@ -1605,7 +1620,11 @@ void decide_step(Ctx &c) {
 
 void check_max(Ctx &c, int parity) {
     check_part(c);
-    launch<check_reduce_body, 64>(c, 1, 0, check_blocks(c), c.checkPart, c.dMax + 2 * parity, c.dMax + 2 * (1 - parity));
+    launch<check_reduce_body, 64>(c, 1, 0, check_blocks(c), c.checkPart, nullptr, c.pinned + 2 + 2 * parity);
+}
+
+void check_out(Ctx &c, int parity) {
+    launch<check_reduce_body, 64>(c, 1, 0, 0, nullptr, c.dispSlots, c.pinned + 2 + 2 * parity);
 }
 
 }  // namespace mdx

@@ -139,9 +139,11 @@ __device__ __forceinline__ void dist_forces(const unsigned long long *f, int4 a,
     }
 }
 
-// slots != nullptr (captured all-rigid steps): also the skin check's largest
-// displacement since the last build, from the positions just written.
-// With xq set (captured all-rigid steps) the kick also does the force
+// slots != nullptr (all-rigid steps): also the skin check's maxima of the
+// displacement since the last build and of the displacement plus 2 dt |v|,
+// from the positions and velocities just written (an M site, moved by its
+// molecule, counts with its own).
+// With xq set (all-rigid steps) the kick also does the force
 // evaluation's position refresh for its sites - FP32 positions, the P3M mesh
 // records of the charged ones, cleared fixed-point force rows (read above)
 // and, in workgroup 0, the cleared energy / virial accumulators - so no
@@ -149,13 +151,12 @@ __device__ __forceinline__ void dist_forces(const unsigned long long *f, int4 a,
 // the records in the new order).
 __device__ __forceinline__ void rigid_vv1_body(int blk, int nblk, RigidArgs r, double4 *__restrict__ pos, double4 *__restrict__ vel,
                                                    const unsigned long long *__restrict__ f,
-                                                   const double4 *__restrict__ last, unsigned *__restrict__ slots,
-                                                   RefreshArgs ra) {
+                                                   const double4 *__restrict__ last, double dt2,
+                                                   unsigned *__restrict__ slots, RefreshArgs ra) {
     r.g = r.bx->geo;
     const int m = blk * blockDim.x + threadIdx.x;
-    float d2 = 0.f;
-    if (ra.xq && blk == 0)
-        for (int k = threadIdx.x; k < ra.nacc; k += blockDim.x) ra.acc[k] = 0ull;
+    float d2 = 0.f, p2 = 0.f;
+    if (ra.xq && blk == 0) refresh_clear(ra);
     if (m < r.nmol) {
     const int4 a = r.atoms[m];
     d3 fO, fH1, fH2;
@@ -205,10 +206,16 @@ __device__ __forceinline__ void rigid_vv1_body(int blk, int nblk, RigidArgs r, d
         const int site[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
         for (int s = 0; s < 4; ++s)
-            if (site[s] >= 0) d2 = fmaxf(d2, (float)disp2(sp[s], last[site[s]], r.g));
+            if (site[s] >= 0) {
+                const d3 v = s == 0 ? vO : s == 1 ? vH1 : s == 2 ? vH2 : mk(0.0, 0.0, 0.0);
+                const double dd = disp2(sp[s], last[site[s]], r.g);
+                const double p = sqrt(dd) + dt2 * sqrt(v.x * v.x + v.y * v.y + v.z * v.z);
+                d2 = fmaxf(d2, (float)dd);
+                p2 = fmaxf(p2, (float)(p * p));
+            }
     }
     }
-    if (slots) disp_fold(d2, slots, blk);
+    if (slots) disp_fold(d2, p2, slots, blk);
 }
 
 // kick = false: only the velocity constraint and the M placement (start of a run)
@@ -442,7 +449,7 @@ void rigid_first_half(Ctx &c) {
     const RigidArgs r = make_args(c);
     RefreshArgs ra{};
     if (c.fuseCheck) ra = refresh_args(c);
-    launch<rigid_vv1_body, 128>(c, cdiv(r.nmol, 128), 0, r, c.pos[c.cur], c.vel[c.cur], c.force, c.posLast, c.fuseCheck ? c.dispSlots : nullptr, ra);
+    launch<rigid_vv1_body, 128>(c, cdiv(r.nmol, 128), 0, r, c.pos[c.cur], c.vel[c.cur], c.force, c.posLast, 2.0 * c.dt, c.fuseCheck ? c.dispSlots : nullptr, ra);
 }
 
 void rigid_second_half(Ctx &c, bool kick) {
@@ -452,7 +459,7 @@ void rigid_second_half(Ctx &c, bool kick) {
     // last workgroup (the molecular virial and M V^2 are summed here), while
     // its ticket, about 24 ns a workgroup, costs no more than a launch (1.6 us
     // plus the start of a wave)
-    if (kick && c.fuseMolVirial && c.fuseStep && c.baro.on && c.capture && cdiv(r.nmol, 128) <= 96) {
+    if (kick && c.fuseMolVirial && c.fuseStep && c.baro.on && cdiv(r.nmol, 128) <= 96) {
         bf.ticket = c.dFlags + 9;
         bf.gate = baro_gate(c);
         bf.bx = c.box;

@@ -171,3 +171,42 @@ def test_virial_trace_matches_full_tensor(gpu_engine_factory, terms):
     # FP32 pair arithmetic summed in another order: ~1e-6 of the diagonal's size
     assert abs(w_tr - w_full) <= 1e-5 * scale
     e.close()
+
+
+@pytest.mark.parametrize("sign", [1, -1])
+def test_eager_barostat_through_grid_changes(orc, gpu_engine_factory, sign):
+    """An eager barostat run that crosses cell-grid changes both ways: far from
+    one the host does not follow the box inside a chunk, near one it does.
+    Runs whose dilation is clamped at every step (P0 far above or below the
+    pressure) must end in the box the clamp gives, with an exact list on a grid
+    that fits it."""
+    say(f"eager barostat through grid changes, {'growing' if sign > 0 else 'shrinking'} box")
+    box = systems.tip4p2005_box(343, seed=35, min_sep=1.8)
+    v = start_velocities(orc, box, seed=8)
+    rc, skin, steps, dil = 7.0, 1.0, 150, 2e-4
+    e, flags = water_md_engine(gpu_engine_factory, box, v, rc=rc, skin=skin, sz=(32, 32, 32), order=5, e3b=True,
+                               dt=1.0)
+    kb, mvv = systems.REAL_BOLTZ, systems.REAL_MVV_TO_ENG
+    e.option("graph", 0)
+    e.thermostat(True, 298.0, 5, 0.0, kb, mvv)
+    # FixPressureBerendsen shrinks the box while P < P0
+    e.barostat(True, -sign * 1e9, 1.0, 1, bulk_modulus=1e-3, max_dilation=dil, mvv_to_eng=mvv)
+    grids = set()
+    for n in (1, steps, steps, steps - 1):
+        e.run(n, flags)
+        grids.add(tuple(e.nlist_stats()["cells"]))
+    lo, L = e.get_box()
+    want = box["L"][0] * (1.0 + sign * dil) ** (3 * steps)
+    assert np.allclose(L, want, rtol=1e-9)
+    assert len(grids) > 1, grids
+    cells = e.nlist_stats()["cells"]
+    assert all(L[a] / cells[a] >= (rc + skin) / r for a, r in enumerate((2, 2, 4)))
+    e.nlist_update(force=True)
+    from test_gpu_parity import assert_same_lists, oracle_rows_by_id
+
+    x, _ = e.get_system()
+    gc, grows = e.nlist_get()
+    excl = orc.exclusions_bfs(len(x), systems.water_bonds(box["mol"]))
+    oc, orows, _ = oracle_rows_by_id(orc, x, lo, L, rc + skin, excl=excl, brute=False)
+    assert_same_lists(gc, grows, oc, orows)
+    e.close()
