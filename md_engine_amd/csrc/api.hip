@@ -1393,6 +1393,7 @@ int mdx_system_set(mdx_ctx *ctx, int n, const double *x, const double *v, const 
                 c.id[b] = dalloc<int>(c, n);
             }
             c.idToIdx = dalloc<int>(c, n);
+            c.io = dalloc<double>(c, 6 * (size_t)n);
             c.xq = dalloc<float4>(c, n);
             c.meshRec = dalloc<float4>(c, n);
             c.force = dalloc<unsigned long long>(c, 3 * (size_t)n);
@@ -1457,12 +1458,8 @@ int mdx_positions_set(mdx_ctx *ctx, const double *x) {
     return guarded(ctx, [&](Ctx &c) {
         require_system(c);
         MDX_REQUIRE(x, MDX_ERR_ARG, "positions required");
-        std::vector<int> idx(c.n);
-        MDX_HIP(hipMemcpyAsync(idx.data(), c.idToIdx, sizeof(int) * c.n, hipMemcpyDeviceToHost, c.stream));
-        MDX_HIP(hipStreamSynchronize(c.stream));
-        std::vector<double4> hp(c.n);
-        for (int i = 0; i < c.n; ++i) hp[idx[i]] = make_double4(x[3 * i], x[3 * i + 1], x[3 * i + 2], 0.0);
-        upload(c, c.pos[c.cur], hp.data(), c.n);
+        upload(c, c.io, x, 3 * (size_t)c.n);
+        unpack_positions(c, c.io);
         MDX_HIP(hipStreamSynchronize(c.stream));
         c.listValid = false;
     });
@@ -1471,26 +1468,11 @@ int mdx_positions_set(mdx_ctx *ctx, const double *x) {
 int mdx_system_get(mdx_ctx *ctx, double *x, double *v) {
     return guarded_ro(ctx, [&](Ctx &c) {
         require_system(c);
-        std::vector<int> idx(c.n);
-        std::vector<double4> hp(c.n), hv(c.n);
-        MDX_HIP(hipMemcpyAsync(idx.data(), c.idToIdx, sizeof(int) * c.n, hipMemcpyDeviceToHost, c.stream));
-        MDX_HIP(hipMemcpyAsync(hp.data(), c.pos[c.cur], sizeof(double4) * c.n, hipMemcpyDeviceToHost, c.stream));
-        MDX_HIP(hipMemcpyAsync(hv.data(), c.vel[c.cur], sizeof(double4) * c.n, hipMemcpyDeviceToHost, c.stream));
+        const size_t m = 3 * (size_t)c.n;
+        pack_state(c, x ? c.io : nullptr, v ? c.io + m : nullptr);
+        if (x) MDX_HIP(hipMemcpyAsync(x, c.io, sizeof(double) * m, hipMemcpyDeviceToHost, c.stream));
+        if (v) MDX_HIP(hipMemcpyAsync(v, c.io + m, sizeof(double) * m, hipMemcpyDeviceToHost, c.stream));
         MDX_HIP(hipStreamSynchronize(c.stream));
-        for (int i = 0; i < c.n; ++i) {
-            const double4 &p = hp[idx[i]];
-            const double4 &w = hv[idx[i]];
-            if (x) {
-                x[3 * i] = p.x;
-                x[3 * i + 1] = p.y;
-                x[3 * i + 2] = p.z;
-            }
-            if (v) {
-                v[3 * i] = w.x;
-                v[3 * i + 1] = w.y;
-                v[3 * i + 2] = w.z;
-            }
-        }
     });
 }
 
@@ -1997,13 +1979,9 @@ int mdx_forces_get(mdx_ctx *ctx, double *f) {
     return guarded_ro(ctx, [&](Ctx &c) {
         require_system(c);
         MDX_REQUIRE(f, MDX_ERR_ARG, "output required");
-        std::vector<unsigned long long> hf(3 * (size_t)c.n);
-        std::vector<int> ids(c.n);
-        MDX_HIP(hipMemcpyAsync(hf.data(), c.force, sizeof(unsigned long long) * hf.size(), hipMemcpyDeviceToHost, c.stream));
-        MDX_HIP(hipMemcpyAsync(ids.data(), c.id[c.cur], sizeof(int) * c.n, hipMemcpyDeviceToHost, c.stream));
+        pack_forces(c, c.io);
+        MDX_HIP(hipMemcpyAsync(f, c.io, sizeof(double) * 3 * (size_t)c.n, hipMemcpyDeviceToHost, c.stream));
         MDX_HIP(hipStreamSynchronize(c.stream));
-        for (int k = 0; k < c.n; ++k)
-            for (int a = 0; a < 3; ++a) f[3 * ids[k] + a] = (double)(long long)hf[3 * k + a] * kFxInv;
     });
 }
 

@@ -205,6 +205,44 @@ __device__ __forceinline__ void nh_start_body(int blk, int nblk, const unsigned 
     for (int k = 1; k < M; ++k) frc[k] = (mass[k - 1] * vel[k - 1] * vel[k - 1] - kT) / mass[k];
 }
 
+// The boundary's arrays are n x 3 by atom id; the kernels below change between
+// them (in a staging buffer) and the cell-ordered records, so that the host
+// copies plain arrays.  On the host the permutation of 500,000 atoms took
+// most of the 7.0 ms of a read-back (copies of 4-vectors and a random walk).
+__device__ __forceinline__ void pack_state_body(int blk, int nblk, int n, const int *__restrict__ idToIdx,
+                                                const double4 *__restrict__ pos, const double4 *__restrict__ vel,
+                                                double *__restrict__ x, double *__restrict__ v) {
+    const int i = blk * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int k = idToIdx[i];
+    if (x) {
+        const double4 p = pos[k];
+        x[3 * (size_t)i] = p.x;
+        x[3 * (size_t)i + 1] = p.y;
+        x[3 * (size_t)i + 2] = p.z;
+    }
+    if (v) {
+        const double4 w = vel[k];
+        v[3 * (size_t)i] = w.x;
+        v[3 * (size_t)i + 1] = w.y;
+        v[3 * (size_t)i + 2] = w.z;
+    }
+}
+__device__ __forceinline__ void unpack_pos_body(int blk, int nblk, int n, const int *__restrict__ idToIdx,
+                                                const double *__restrict__ x, double4 *__restrict__ pos) {
+    const int i = blk * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const size_t b = 3 * (size_t)i;
+    pos[idToIdx[i]] = make_double4(x[b], x[b + 1], x[b + 2], 0.0);
+}
+__device__ __forceinline__ void pack_force_body(int blk, int nblk, int n, const int *__restrict__ idToIdx,
+                                                const unsigned long long *__restrict__ f, double *__restrict__ out) {
+    const int i = blk * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const size_t k = 3 * (size_t)idToIdx[i], b = 3 * (size_t)i;
+    for (int a = 0; a < 3; ++a) out[b + a] = fx_to_d(f[k + a]);
+}
+
 __device__ __forceinline__ void vscale_dev_body(int blk, int nblk, int n, double4 *__restrict__ vel, const double *__restrict__ scale) {
     int i = blk * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -247,6 +285,16 @@ void thermostat_apply(Ctx &c) {
     if (!c.fuseThermo) thermo_measure(c);  // else summed by the rigid second half
     const double coupling = c.thermoTau > 0 ? c.thermoEvery * c.dt / c.thermoTau : 1.0;
     launch<vscale_body, 256>(c, cdiv(c.n, 256), 0, thermo_gate(c), c.n, c.vel[c.cur], c.thermo, c.tconv, c.thermoT, c.thermoTau > 0 ? 1 : 0, coupling);
+}
+
+void pack_state(Ctx &c, double *x, double *v) {
+    launch<pack_state_body, 256>(c, cdiv(c.n, 256), 0, c.n, c.idToIdx, c.pos[c.cur], c.vel[c.cur], x, v);
+}
+void unpack_positions(Ctx &c, const double *x) {
+    launch<unpack_pos_body, 256>(c, cdiv(c.n, 256), 0, c.n, c.idToIdx, x, c.pos[c.cur]);
+}
+void pack_forces(Ctx &c, double *f) {
+    launch<pack_force_body, 256>(c, cdiv(c.n, 256), 0, c.n, c.idToIdx, c.force, f);
 }
 
 void acc_read(Ctx &c, double out[ACC_N]) {

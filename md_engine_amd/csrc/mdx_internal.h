@@ -473,6 +473,7 @@ struct Ctx {
     int *id[2] = {nullptr, nullptr};
     int cur = 0;
     int *idToIdx = nullptr;
+    double *io = nullptr;                  // 6 n: staging of the boundary's n x 3 arrays
     float4 *xq = nullptr;
     float4 *meshRec = nullptr;             // per charged site: mesh offsets and point (mesh_record)
     unsigned long long *force = nullptr;   // 3 per atom
@@ -1348,6 +1349,10 @@ void integrate_first_half(Ctx &c);
 // thermostat half step and half kick without the drift (ring polymers)
 void integrate_kick_first(Ctx &c);
 void integrate_second_half(Ctx &c);
+// n x 3 arrays by id in device memory from and to the cell-ordered records
+void pack_state(Ctx &c, double *x, double *v);  // either may be nullptr
+void unpack_positions(Ctx &c, const double *x);
+void pack_forces(Ctx &c, double *f);
 // accumulator slots summed over the replicas (synchronises the stream)
 void acc_read(Ctx &c, double out[ACC_N]);
 // clear slots [slot, slot + count) in every replica
