@@ -1132,6 +1132,7 @@ void run_captured(const std::vector<Ctx *> &cs, int nsteps, int flags, const Rin
             for (size_t k = 0; k < cs.size(); ++k) {
                 Ctx &c = *cs[k];
                 c.nRebuilds += hs[k][3];
+                if (hs[k][3]) c.listNeed = list_need(c);  // what the graph's builds left
                 c.turn += len;
                 // the box grew by a cell: the next chunk takes a finer grid
                 if (c.baro.on && regrid_if_needed(c)) regrid = true;
@@ -1406,6 +1407,7 @@ int mdx_system_set(mdx_ctx *ctx, int n, const double *x, const double *v, const 
         c.qHost.assign(n, 0.0f);
         c.typeHost.assign(n, 0);
         c.pairFlagsDirty = true;
+        c.needDirty = true;
         c.hasCharges = false;
         c.nCharged = 0;
         c.maxType = 0;
@@ -1605,6 +1607,11 @@ int mdx_nlist_get(mdx_ctx *ctx, int32_t *counts, uint32_t *tagged_ids, int row_c
     return guarded_ro(ctx, [&](Ctx &c) {
         require_system(c);
         MDX_REQUIRE(c.listValid, MDX_ERR_STATE, "no neighbor list built");
+        nlist_complete(c);
+        if (!c.wholeList) {
+            c.wholeList = true;
+            ++c.apiEpoch;  // cached step graphs build without it
+        }
         const int n = c.n;
         std::vector<int> cnt(n), ids(n);
         std::vector<uint32_t> nl((size_t)n * c.cap);
@@ -1662,6 +1669,7 @@ int mdx_lj_set(mdx_ctx *ctx, int ntypes, const double *rc2, const double *eps24,
         c.ljOn = true;
         c.ljEps.assign(eps24, eps24 + T2);
         c.pairFlagsDirty = true;
+        list_setup_changed(c);
     });
 }
 
@@ -1680,6 +1688,7 @@ int mdx_ewald_real_set(mdx_ctx *ctx, int enable, double alpha, double qqr, doubl
         c.qqr = (float)qqr;
         c.rq2 = (float)(r_cut * r_cut);
         if (c.n > 0) box_upload(c);
+        list_setup_changed(c);
     });
 }
 
@@ -1818,6 +1827,10 @@ int mdx_e3b_set(mdx_ctx *ctx, int nmol, const int32_t *mol_ids, const double par
         E.molIds = dalloc<int4>(c, nmol);
         E.molAtoms = dalloc<int4>(c, nmol);
         E.atomMolO = dalloc<int>(c, c.n);
+        if (!E.molIdsOfO) E.molIdsOfO = dalloc<int>(c, c.n);
+        std::vector<int> ofO(c.n, -1);
+        for (int m = 0; m < nmol; ++m) ofO[ids[m].x] = m;
+        upload(c, E.molIdsOfO, ofO.data(), c.n);
         E.tot = dalloc<float4>(c, nmol);
         E.nlCount = dalloc<int>(c, nmol);
         E.cap = 64;
@@ -1828,6 +1841,7 @@ int mdx_e3b_set(mdx_ctx *ctx, int nmol, const int32_t *mol_ids, const double par
         E.oxIds.resize(nmol);
         for (int m = 0; m < nmol; ++m) E.oxIds[m] = ids[m].x;
         update_ox_flag(c);
+        c.needDirty = true;
         c.listValid = false;
     });
 }
@@ -2587,6 +2601,7 @@ int mdx_nlist_totals(mdx_ctx *ctx, int64_t *pair_entries, int64_t *mol_entries) 
     return guarded_ro(ctx, [&](Ctx &c) {
         require_system(c);
         MDX_REQUIRE(c.listValid, MDX_ERR_STATE, "no neighbor list built");
+        nlist_complete(c);
         std::vector<int> cnt(c.n);
         MDX_HIP(hipMemcpyAsync(cnt.data(), c.nlCount, sizeof(int) * c.n, hipMemcpyDeviceToHost, c.stream));
         std::vector<int> mc(c.e3b.on ? c.e3b.nmol : 0);

@@ -541,6 +541,11 @@ struct Ctx {
     int buildMode = 0;            // 0 (default) and 2 per-atom teams
     long long nRebuilds = 0;
     bool listValid = false;
+    // parts of the rows (row_parts): what the current list holds, and what the
+    // set-up's kernels read (recomputed when the set-up changed)
+    unsigned long long listNeed = 0, needMask = 0;
+    bool needDirty = true;
+    bool wholeList = false;       // mdx_nlist_get was called: builds make whole rows
     // Ring polymers with one list on the centroids (GridGPU.cu:163-189,
     // 888-895): while a ring call runs, the build bins and pairs atoms by the
     // centroid of their ring (cenById, by atom id) instead of their own
@@ -561,6 +566,7 @@ struct Ctx {
     int exclSpan = 0;             // largest |id_i - id_j| over excluded pairs
     uint32_t *exclIdx = nullptr;  // per atom: maxExcl partners, id | tag << 30 (team builds: index | tag << 30)
     size_t exclIdxN = 0;
+    bool exclByIdx = false;       // the last build was a team build: exclIdx holds indices
 
     // LJ + Ewald real space
     bool ljOn = false;
@@ -1142,6 +1148,9 @@ void fill_int(Ctx &c, int *p, int count, int v, const int *gate = nullptr);  // 
 void nlist_rebuild_async(Ctx &c);     // rebuild now; capacity checked later (capacity_ok)
 bool capacity_ok(Ctx &c);             // false: rows grew, results since the last check are invalid
 bool grow_if_needed(Ctx &c);
+unsigned long long list_need(Ctx &c); // the parts of the rows the set-up's kernels read
+void nlist_complete(Ctx &c);          // the parts of the rows that no kernel reads, for the whole list's readers
+void list_setup_changed(Ctx &c);      // force terms or charges changed: rows completed if they need more than is built
 constexpr int kCheckBlocks = 512;     // workgroups of the displacement check
 void check_max(Ctx &c, int parity);   // max displacement / prediction into pinned slot `parity`
 void check_out(Ctx &c, int parity);   // the same from the words a fused first half left

@@ -507,11 +507,23 @@ __device__ __forceinline__ bool in_run(uint32_t ex, int s0, int s1) {
     return ex != ~0u && j >= s0 && j < s1;
 }
 
+// Which parts of its row an atom needs (bit 0 charged partners, bit 1
+// charge-free ones), from list_need's mask: four bits a type, the low two for
+// charged atoms of the type, the high two for charge-free ones.  The pair and
+// E3B kernels read only these parts (in TIP4P water a charged site reads its
+// charged partners and an oxygen its charge-free ones: 0.6 of the entries), so
+// a step's build leaves the rest out; nlist_complete adds it when the whole
+// list is asked for.
+__device__ __forceinline__ unsigned row_parts(unsigned long long need, int type, float q) {
+    return (unsigned)(need >> (4 * type + (q != 0.0f ? 0 : 2))) & 3u;
+}
+
 template <int T, bool SHIFT>
 __device__ __forceinline__ void build_body(int blk, int nblk, const int *__restrict__ gate, 
     int n, const double4 *__restrict__ pos, const float4 *__restrict__ xq, const BoxDev *__restrict__ bx,
     const int *__restrict__ colRank, const int *__restrict__ cellStart, int ncell,
-    double rlist2, const uint32_t *__restrict__ exclIdx, int maxExcl, int cap,
+    double rlist2, const uint32_t *__restrict__ exclIdx, int maxExcl, const int *__restrict__ type,
+    unsigned long long need, int cap,
     uint32_t *__restrict__ nl, int *__restrict__ nlCount, int *__restrict__ nlCountA, int *__restrict__ flags,
     int *__restrict__ waveMax) {
     if (gate && *gate == 0) return;
@@ -546,10 +558,11 @@ __device__ __forceinline__ void build_body(int blk, int nblk, const int *__restr
         const uint32_t ex0 = maxExcl > 0 ? exRow[0] : ~0u, ex1 = maxExcl > 1 ? exRow[1] : ~0u;
         const uint32_t ex2 = maxExcl > 2 ? exRow[2] : ~0u, ex3 = maxExcl > 3 ? exRow[3] : ~0u;
         int nrun = 0;
+        const unsigned parts = row_parts(need, type[i], xi.w);
 #pragma unroll 1
         for (int cls = 0; cls < 2; ++cls) {
             const int *cs = cellStart + cls * ncell;
-            for (int c0 = 0; c0 < ncol; c0 += T) {
+            for (int c0 = 0; (parts >> cls & 1u) && c0 < ncol; c0 += T) {
                 const int col = c0 + tl;
                 int st0 = 0, len0 = 0, st1 = 0, len1 = 0;
                 uint32_t code0 = 0, code1 = 0;
@@ -757,6 +770,20 @@ __device__ __forceinline__ uint32_t excl_entry(const ExclArgs &x, int i, int q) 
     return e == ~0u ? e : (uint32_t)x.idToIdx[e & 0x3FFFFFFFu] | (e & 0xC0000000u);
 }
 
+// The E3B molecule list made by the wave build: for an oxygen of E3B water, the
+// molecules of the oxygens among its row's hits within (r2b + skin), in row
+// order (what e3b_list_body makes of a finished row).  As a launch of its own,
+// reading the rows back, it took 14.2 us a rebuild for 8,192 molecules and
+// 25.5 us for 32,768; here it is a second ballot in a quarter of the waves.
+struct OxListArgs {
+    const int *mol;  // by atom id: molecule index of an oxygen, else -1 (nullptr: no E3B)
+    const int *id;
+    double r2;
+    float r2f;       // r2 with the pre-test's margin
+    int cap;
+    int *nl, *count, *wmax;
+};
+
 struct RunEntry {
     int vend;      // end of the run in the stream
     int off;       // atom index = stream position + off
@@ -768,7 +795,7 @@ template <bool SHIFT>
 __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__restrict__ gate,
     int n, const double4 *__restrict__ pos, const float4 *__restrict__ xq, const BoxDev *__restrict__ bx,
     const int *__restrict__ colRank, const int *__restrict__ cellStart, int ncell,
-    double rlist2, ExclArgs ex, int cap,
+    double rlist2, ExclArgs ex, const int *__restrict__ type, unsigned long long need, OxListArgs ox, int cap,
     uint32_t *__restrict__ nl, int *__restrict__ nlCount, int *__restrict__ nlCountA, int *__restrict__ flags,
     int *__restrict__ waveMax) {
     if (gate && *gate == 0) return;
@@ -805,13 +832,15 @@ __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__
     const int maxExcl = ex.maxExcl;
     const uint32_t ex0 = (uint32_t)__builtin_amdgcn_readlane((int)exv, 0), ex1 = (uint32_t)__builtin_amdgcn_readlane((int)exv, 1);
     const uint32_t ex2 = (uint32_t)__builtin_amdgcn_readlane((int)exv, 2), ex3 = (uint32_t)__builtin_amdgcn_readlane((int)exv, 3);
+    const unsigned parts = row_parts(need, type[i], xi.w);
+    const int mol = ox.mol ? ox.mol[ox.id[i]] : -1;  // an E3B oxygen's molecule: its list is made here too
     // ---- table: one (class, column) per lane
     const int cls = lane >> 5, col = lane & 31;
     const int *cs = cellStart + cls * ncell;
     int st0 = 0, len0 = 0, st1 = 0, len1 = 0;
     uint32_t f0 = 0, f1 = 0;
     float s0x = xi.x, s0y = xi.y, s0z = xi.z, s1x = xi.x, s1y = xi.y, s1z = xi.z;
-    if (col < ncol) {
+    if (col < ncol && (parts >> cls & 1u)) {
         const int a = col / sy, b = col - a * sy;
         const int xx = axis_cell(a, cx, cg.nc[0], rx, g.periodic[0]);
         const int yy = axis_cell(b, cy, cg.nc[1], ry, g.periodic[1]);
@@ -905,7 +934,7 @@ __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__
     // ---- walk
     const uint32_t e0 = ex0 & 0x3FFFFFFFu, e1 = ex1 & 0x3FFFFFFFu, e2 = ex2 & 0x3FFFFFFFu, e3 = ex3 & 0x3FFFFFFFu;
     uint32_t *row = nl + (size_t)i * cap;
-    int cnt = 0, cntA = 0;
+    int cnt = 0, cntA = 0, cntO = 0;
     int ra = 0;  // run of the current chunk start (uniform)
     for (int p0 = 0; p0 < total; p0 += 64 * U) {
         uint32_t jv[U];
@@ -963,6 +992,20 @@ __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__
                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)cnt));
                 if (k < cap) row[k] = (uint32_t)j | (tag << 30);
             }
+            if (mol >= 0) {  // uniform: the oxygens among the hits within the molecule list's radius
+                int mj = -1;
+                if (hit && r2f <= ox.r2f) {
+                    mj = ox.mol[ox.id[j]];
+                    if (mj >= 0 && !(dist2(pi, pos[j], g) < ox.r2)) mj = -1;
+                }
+                const unsigned long long mo = __ballot(mj >= 0);
+                if (mj >= 0) {
+                    const int k = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mo >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)mo, (uint32_t)cntO));
+                    if (k < ox.cap) ox.nl[(size_t)mol * ox.cap + k] = mj;
+                }
+                cntO += __popcll(mo);
+            }
             // the charged/charge-free split falls inside this chunk
             if (p <= totalA && totalA < p + 64) {
                 const int below = totalA - p;
@@ -977,6 +1020,10 @@ __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__
         nlCount[i] = cnt;
         nlCountA[i] = cntA;
         waveMax[i] = cnt;
+        if (mol >= 0) {
+            ox.count[mol] = cntO;
+            ox.wmax[mol] = cntO;
+        }
     }
 }
 
@@ -1092,7 +1139,7 @@ template <bool SHIFT>
 __device__ __forceinline__ void build_map_body(int blk, int nblk, const int *__restrict__ gate,
     int n, const double4 *__restrict__ pos, const float4 *__restrict__ xq, const BoxDev *__restrict__ bx,
     const int *__restrict__ colRank, const int *__restrict__ cellStart, int ncell,
-    double rlist2, ExclArgs ex, int cap,
+    double rlist2, ExclArgs ex, const int *__restrict__ type, unsigned long long need, OxListArgs ox, int cap,
     uint32_t *__restrict__ nl, int *__restrict__ nlCount, int *__restrict__ nlCountA, int *__restrict__ flags,
     int *__restrict__ waveMax, MolMapArgs mm) {
     const int nb = nblk - mm.blocks;
@@ -1100,8 +1147,8 @@ __device__ __forceinline__ void build_map_body(int blk, int nblk, const int *__r
         mol_map_body(blk - nb, mm.blocks, gate, mm);
         return;
     }
-    build_wave_body<SHIFT>(blk, nb, gate, n, pos, xq, bx, colRank, cellStart, ncell, rlist2, ex, cap, nl, nlCount,
-                           nlCountA, flags, waveMax);
+    build_wave_body<SHIFT>(blk, nb, gate, n, pos, xq, bx, colRank, cellStart, ncell, rlist2, ex, type, need, ox, cap, nl,
+                           nlCount, nlCountA, flags, waveMax);
 }
 
 __device__ __forceinline__ void fill_int_body(int blk, int nblk, const int *__restrict__ gate, int n, int *__restrict__ p, int v) {
@@ -1146,47 +1193,56 @@ uint32_t morton2(uint32_t x, uint32_t y) {
 // slots of the pair-list waves in c.waveMax; the molecule-list slots follow
 size_t wave_slots_a(const Ctx &c) { return (size_t)c.n + 4; }
 
-// with the molecule maps of the rebuild in the same launch
-void launch_build_wave(Ctx &c, int cur, const MolMapArgs &mm) {
-    const ExclArgs ex{c.exclOff ? c.maxExcl : 0, c.exclIdx, c.idToIdx};
+// whether every candidate of a run sits in one known image of the stencil
+bool build_shifts(const Ctx &c) {
     MDX_REQUIRE(std::min(c.nc[0], 2 * c.reach[0] + 1) * std::min(c.nc[1], 2 * c.reach[1] + 1) <= kMaxCols, 1,
                 "stencil wider than the build kernel's column table");
-    const int blocks = cdiv(c.n, 4);
-    const double4 *bpos = c.cenById ? c.buildPos : c.pos[cur];  // ring centroids or the positions
-    bool shift = true;
     for (int a = 0; a < 3; ++a)
-        if (c.geo.periodic[a] && c.nc[a] < 2 * c.reach[a] + 1) shift = false;
-    if (shift)
-        launch<build_map_body<true>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, c.box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, ex, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm);
+        if (c.geo.periodic[a] && c.nc[a] < 2 * c.reach[a] + 1) return false;
+    return true;
+}
+
+// with the molecule maps of the rebuild in the same launch, and the E3B list
+void launch_build_wave(Ctx &c, const double4 *bpos, const BoxDev *box, const MolMapArgs &mm) {
+    const ExclArgs ex{c.exclOff ? c.maxExcl : 0, c.exclIdx, c.idToIdx};
+    OxListArgs ox{};
+    if (c.e3b.on) {
+        const double rc = (double)c.e3b.r2b + c.skin, lmax = std::max({c.geo.L[0], c.geo.L[1], c.geo.L[2]});
+        ox.mol = c.e3b.molIdsOfO;
+        ox.id = c.id[c.cur];
+        ox.r2 = rc * rc;
+        ox.r2f = (float)(rc * rc * (1.0 + 1e-5) + 1e-5 * rc * lmax);  // far above the FP32 rounding of r^2
+        ox.cap = c.e3b.cap;
+        ox.nl = c.e3b.nl;
+        ox.count = c.e3b.nlCount;
+        ox.wmax = c.waveMax + wave_slots_a(c);
+        c.waveMaxB = c.e3b.nmol;
+    }
+    const int blocks = cdiv(c.n, 4);
+    if (build_shifts(c))
+        launch<build_map_body<true>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, ex, c.type[c.cur], c.listNeed, ox, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm);
     else
-        launch<build_map_body<false>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, c.box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, ex, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm);
+        launch<build_map_body<false>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, ex, c.type[c.cur], c.listNeed, ox, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm);
     c.waveMaxA = blocks * 4;
 }
 
 template <int T>
-void launch_build(Ctx &c, int cur) {
-    MDX_REQUIRE(std::min(c.nc[0], 2 * c.reach[0] + 1) * std::min(c.nc[1], 2 * c.reach[1] + 1) <= kMaxCols, 1,
-                "stencil wider than the build kernel's column table");
-    int threads = 256;
-    int blocks = cdiv((long long)c.n * T, threads);
-    const double4 *bpos = c.cenById ? c.buildPos : c.pos[cur];  // ring centroids or the positions
-    // image shifts need every periodic axis to hold the full stencil
-    bool shift = true;
-    for (int a = 0; a < 3; ++a)
-        if (c.geo.periodic[a] && c.nc[a] < 2 * c.reach[a] + 1) shift = false;
-    if (shift)
-        launch<build_body<T, true>, 256>(c, blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, c.box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, c.exclIdx, c.exclOff ? c.maxExcl : 0, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax);
+void launch_build(Ctx &c, const double4 *bpos, const BoxDev *box) {
+    const int threads = 256;
+    const int blocks = cdiv((long long)c.n * T, threads);
+    if (build_shifts(c))
+        launch<build_body<T, true>, 256>(c, blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, c.exclIdx, c.exclOff ? c.maxExcl : 0, c.type[c.cur], c.listNeed, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax);
     else
-        launch<build_body<T, false>, 256>(c, blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, c.box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, c.exclIdx, c.exclOff ? c.maxExcl : 0, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax);
+        launch<build_body<T, false>, 256>(c, blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, c.exclIdx, c.exclOff ? c.maxExcl : 0, c.type[c.cur], c.listNeed, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax);
     c.waveMaxA = blocks * (threads / 64);
 }
 
 template <int T>
-void launch_e3b_list(Ctx &c, int cur) {
+void launch_e3b_list(Ctx &c, const double4 *bpos, const BoxDev *box) {
     int threads = 256;
     int blocks = cdiv((long long)c.e3b.nmol * T, threads);
     double rc = (double)c.e3b.r2b + c.skin;
-    launch<e3b_list_body<T>, 256>(c, blocks, 0, rebuild_gate(c), c.e3b.nmol, c.e3b.molAtoms, c.e3b.atomMolO, c.pos[cur], c.box, rc * rc, c.cap, c.nl, c.nlCount, c.nlCountA, c.e3b.oxUncharged ? 1 : 0, c.e3b.cap, c.e3b.nl, c.e3b.nlCount, c.waveMax + wave_slots_a(c));
+    launch<e3b_list_body<T>, 256>(c, blocks, 0, rebuild_gate(c), c.e3b.nmol, c.e3b.molAtoms, c.e3b.atomMolO, bpos, box, rc * rc, c.cap, c.nl, c.nlCount, c.nlCountA, c.e3b.oxUncharged ? 1 : 0, c.e3b.cap, c.e3b.nl, c.e3b.nlCount, c.waveMax + wave_slots_a(c));
     c.waveMaxB = blocks * (threads / 64);
 }
 
@@ -1309,6 +1365,91 @@ void nlist_check(Ctx &c) {
     launch<check_body, 256>(c, cdiv(c.n, threads), 0, c.n, c.pos[c.cur], c.posLast, c.box, thr * thr, c.dFlags);
 }
 
+// The rows from the sorted atoms at bpos (FP32 copies in xq), and the E3B
+// list; grows them and builds again where they overflowed (sync), else leaves
+// the check to the next synchronisation point.
+static void build_rows(Ctx &c, const double4 *bpos, const BoxDev *box, const MolMapArgs &mm, bool sync, bool wave) {
+    for (;;) {
+        // the builds of a run keep the running maximum of the chunk in dFlags[1..2]
+        if (!c.capture && sync) fill_int(c, c.dFlags + 1, 2, 0);
+        c.waveMaxB = 0;
+        {
+            ProfScope ps(c, PK_BUILD);
+            if (wave) launch_build_wave(c, bpos, box, mm);
+            else if (c.buildTeam == 8) launch_build<8>(c, bpos, box);
+            else if (c.buildTeam == 32) launch_build<32>(c, bpos, box);
+            else launch_build<16>(c, bpos, box);
+        }
+        if (c.e3b.on && !wave) {  // the wave build makes this list itself
+            switch (c.e3b.listTeam) {
+                case 8: launch_e3b_list<8>(c, bpos, box); break;
+                case 16: launch_e3b_list<16>(c, bpos, box); break;
+                default: launch_e3b_list<32>(c, bpos, box); break;
+            }
+        }
+        if (c.capture && c.fuseStep) {
+            // the row maxima ride on the position refresh that follows; the
+            // host checks the rows after the chunk
+            c.rowMaxPending = true;
+            return;
+        }
+        // largest row counts -> pinned host memory; checked now (sync) or at
+        // the next synchronisation point (capacity_ok)
+        launch<row_max_body, 1024>(c, 1, 0, rebuild_gate(c), c.waveMaxA, c.waveMax, c.waveMaxB, c.waveMax + wave_slots_a(c), c.dFlags, c.capture ? nullptr : c.pinned);
+        if (c.capture) return;  // rows checked by the host after the chunk
+        if (!sync) {
+            MDX_HIP(hipEventRecord(c.capEvent, c.stream));
+            c.capPending = true;
+            return;
+        }
+        MDX_HIP(hipStreamSynchronize(c.stream));
+        if (!grow_if_needed(c)) return;
+    }
+}
+
+// The parts of the rows that the set-up's kernels read, as row_parts' mask;
+// all of them for a ring's centroid lists, whose build positions do not
+// outlive the ring call, and once a program has read the list back (it may do
+// so after every step, and each time pay for a completing build).
+unsigned long long list_need(Ctx &c) {
+    if (c.cenById || c.wholeList) return ~0ull;
+    if (c.needDirty) {
+        const std::vector<int> fl = pair_type_flag_table(c);
+        const bool coul = c.ewaldReal && c.hasCharges;
+        unsigned long long need = 0;
+        for (int t = 0; t < kMaxTypes; ++t) {
+            const unsigned long long lj = (unsigned long long)(c.ljOn ? fl[t] & 3 : 0);
+            need |= (lj | (coul ? 1ull : 0ull)) << (4 * t) | lj << (4 * t + 2);
+        }
+        // the E3B list reads an oxygen's whole row, or the charge-free part of
+        // charge-free oxygens
+        if (c.e3b.on)
+            for (int o : c.e3b.oxIds)
+                need |= (c.e3b.oxUncharged ? 2ull : 3ull) << (4 * c.typeHost[o] + (c.qHost[o] != 0.0f ? 0 : 2));
+        c.needMask = need;
+        c.needDirty = false;
+    }
+    return c.needMask;
+}
+
+// The whole rows of the current list: built again from the positions and the
+// box of its build, in the order that build left.
+void nlist_complete(Ctx &c) {
+    if (!c.listValid || c.listNeed == ~0ull) return;
+    MDX_REQUIRE(!c.capture, 3, "the list cannot be completed while a step is captured");
+    capacity_ok(c);
+    launch<xq_body, 256>(c, cdiv(c.n, 256), 0, c.n, c.posLast, c.q[c.cur], c.xq, c.boxLast);
+    c.listNeed = ~0ull;
+    // the exclusion rows are as that build's kernel reads them
+    build_rows(c, c.posLast, c.boxLast, MolMapArgs{}, true, !c.exclByIdx);
+    refresh_xq(c);
+}
+
+void list_setup_changed(Ctx &c) {
+    c.needDirty = true;
+    if (c.listValid && !c.centroidList && (list_need(c) & ~c.listNeed)) nlist_complete(c);
+}
+
 static void run_build(Ctx &c, bool sync) {
     // per-wave row maxima: n + 4 slots cover the build at up to 64 lanes per
     // atom (workgroups of 4 waves), the rest the molecule list likewise
@@ -1340,6 +1481,7 @@ static void run_build(Ctx &c, bool sync) {
         }
     }
     c.centroidList = cen != nullptr;
+    c.exclByIdx = !waveBuild;
     // (the map workgroups of a build clear the chunk counts for the next
     // binning; nothing between the binning and them throws)
     DecideArgs da{};
@@ -1416,45 +1558,9 @@ static void run_build(Ctx &c, bool sync) {
     mm.blocks = cdiv(std::max({mm.nmol, mm.nmolR, mm.nmolF, mm.nchunk}), threads);
     // the wave build takes the maps as extra workgroups; the team builds launch them first
     if (!waveBuild) launch<mol_map_body, 256>(c, mm.blocks, 0, rebuild_gate(c), mm);
-    for (;;) {
-        // the builds of a run keep the running maximum of the chunk in dFlags[1..2]
-        if (!c.capture && sync) fill_int(c, c.dFlags + 1, 2, 0);
-        {
-            ProfScope ps(c, PK_BUILD);
-            switch (c.buildTeam) {
-                case 8: launch_build<8>(c, c.cur); break;
-                case 16: launch_build<16>(c, c.cur); break;
-                case 32: launch_build<32>(c, c.cur); break;
-                default: launch_build_wave(c, c.cur, mm); break;
-            }
-        }
-        c.waveMaxB = 0;
-        if (c.e3b.on) {
-            switch (c.e3b.listTeam) {
-                case 8: launch_e3b_list<8>(c, c.cur); break;
-                case 16: launch_e3b_list<16>(c, c.cur); break;
-                default: launch_e3b_list<32>(c, c.cur); break;
-            }
-        }
-        if (c.capture && c.fuseStep) {
-            // the row maxima ride on the position refresh that follows; the
-            // host checks the rows after the chunk
-            c.rowMaxPending = true;
-            return;
-        }
-        // largest row counts -> pinned host memory; checked now (sync) or at
-        // the next synchronisation point (capacity_ok)
-        launch<row_max_body, 1024>(c, 1, 0, rebuild_gate(c), c.waveMaxA, c.waveMax, c.waveMaxB, c.waveMax + wave_slots_a(c), c.dFlags, c.capture ? nullptr : c.pinned);
-        if (c.capture) return;  // rows checked by the host after the chunk
-        if (!sync) {
-            MDX_HIP(hipEventRecord(c.capEvent, c.stream));
-            c.capPending = true;
-            break;
-        }
-        MDX_HIP(hipStreamSynchronize(c.stream));
-        if (grow_if_needed(c)) continue;
-        break;
-    }
+    c.listNeed = list_need(c);
+    build_rows(c, cen ? c.buildPos : c.pos[cur], c.box, mm, sync, waveBuild);
+    if (c.capture) return;
     c.nRebuilds++;
     c.listValid = true;
 }

@@ -112,3 +112,63 @@ def test_fused_first_half_equals_separate(orc, gpu_engine_factory, n):
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
     assert out[0][2] == out[1][2] and out[0][2] > 3
     assert out[0][3] == 0
+
+
+@pytest.mark.parametrize("graph", [0, 1])
+@pytest.mark.parametrize("team", [0, 16])
+def test_whole_list_from_partial_rows(orc, gpu_engine_factory, graph, team):
+    """Builds leave out the parts of the rows that no kernel reads (an oxygen's
+    charged partners, a charged site's charge-free ones); the list that is read
+    back is whole all the same, after runs and after the force terms change to
+    ones that read more, and the forces then are those of a fresh engine."""
+    say(f"partial rows, graph {graph}, team {team}")
+    from md_engine_amd import E3B, PPPM, systems
+    from test_gpu_water_md import start_velocities, water_md_engine
+
+    box = systems.tip4p2005_box(343, seed=36, min_sep=1.8)
+    n, L = len(box["x"]), box["L"]
+    excl = orc.exclusions_bfs(n, systems.water_bonds(box["mol"]))
+
+    def make(v):
+        e, flags = water_md_engine(gpu_engine_factory, box, v, rc=7.0, skin=1.0, sz=(32, 32, 32), order=5, e3b=True,
+                                   dt=1.0)
+        e.teams_set(team)
+        return e, flags
+
+    e, flags = make(start_velocities(orc, box, seed=9))
+    e.option("graph", graph)
+
+    def oracle_list():
+        x, _ = e.get_system()
+        return (x, *oracle_rows_by_id(orc, x, box["lo"], L, 8.0, excl=excl, brute=False)[:2])
+
+    for _ in range(2):
+        e.run(70, flags)
+        e.nlist_update(force=True)
+        x, oc, orows = oracle_list()
+        read = e.pair_entries_read()
+        assert e.nlist_totals()[0] == int(oc.sum())  # completed, then partial again by the run
+        assert e.pair_entries_read() == read and read[0] < 0.75 * oc.sum()
+    v = e.get_system()[1]
+    g, _ = make(v)  # a reader of the list: whole rows from then on
+    g.option("graph", graph)
+    g.set_positions(x)
+    for _ in range(2):
+        g.nlist_update(force=True)
+        assert_same_lists(*g.nlist_get(), oc, orows)
+    for k in (e, g):
+        k.compute(flags)
+    assert np.array_equal(e.forces(), g.forces())
+    g.close()
+    # LJ between every pair of types: every part of every row is read now
+    rc2 = np.full((3, 3), 49.0)
+    eps24, sig6 = np.full((3, 3), 24 * 0.05), np.full((3, 3), 1.0)
+    f, _ = make(np.zeros_like(box["x"]))
+    f.set_positions(x)
+    out = []
+    for k in (e, f):
+        k.lj_set(rc2, eps24, sig6)
+        k.compute(PAIR | PPPM | E3B)
+        out.append(k.forces())
+        k.close()
+    assert np.array_equal(out[0], out[1])
