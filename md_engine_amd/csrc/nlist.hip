@@ -791,7 +791,20 @@ struct RunEntry {
     float xs[3];   // the atom in the run's image frame
 };
 
-template <bool SHIFT>
+// The canonical distance of the few candidates near a cutoff: the box and the
+// atom are read again here (the barrier keeps the loads from moving out of the
+// branch) instead of living in scalar registers through the walk, whose
+// number decides how many waves a SIMD holds: 500,000 LJ atoms 651 -> 525 us.
+// The builds that also make the E3B list need more vector registers and lose
+// a wave to the extra addresses (313 -> 330 us at 131,072 sites), so they keep
+// the values.
+__device__ __forceinline__ double dist2_at(const double4 *__restrict__ pos, int i, int j, const BoxDev *bx) {
+    asm volatile("" : "+s"(bx), "+s"(i));
+    return dist2(pos[i], pos[j], bx->geo);
+}
+
+// OX: the set-up has E3B water (the list code costs registers).
+template <bool SHIFT, bool OX>
 __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__restrict__ gate,
     int n, const double4 *__restrict__ pos, const float4 *__restrict__ xq, const BoxDev *__restrict__ bx,
     const int *__restrict__ colRank, const int *__restrict__ cellStart, int ncell,
@@ -833,7 +846,7 @@ __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__
     const uint32_t ex0 = (uint32_t)__builtin_amdgcn_readlane((int)exv, 0), ex1 = (uint32_t)__builtin_amdgcn_readlane((int)exv, 1);
     const uint32_t ex2 = (uint32_t)__builtin_amdgcn_readlane((int)exv, 2), ex3 = (uint32_t)__builtin_amdgcn_readlane((int)exv, 3);
     const unsigned parts = row_parts(need, type[i], xi.w);
-    const int mol = ox.mol ? ox.mol[ox.id[i]] : -1;  // an E3B oxygen's molecule: its list is made here too
+    const int mol = OX ? ox.mol[ox.id[i]] : -1;  // an E3B oxygen's molecule: its list is made here too
     // ---- table: one (class, column) per lane
     const int cls = lane >> 5, col = lane & 31;
     const int *cs = cellStart + cls * ncell;
@@ -970,7 +983,7 @@ __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__
                 r2f = dist2f(xi, cur, pf);
             }
             bool hit = r2f < pf.lo2;
-            if (!hit && r2f <= pf.hi2) hit = dist2(pi, pos[j], g) < rlist2;
+            if (!hit && r2f <= pf.hi2) hit = (OX ? dist2(pi, pos[j], g) : dist2_at(pos, i, j, bx)) < rlist2;
             uint32_t tag = 0;
             if ((int)jv[u] < 0) {
                 hit = hit && j != i;
@@ -992,7 +1005,7 @@ __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__
                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)cnt));
                 if (k < cap) row[k] = (uint32_t)j | (tag << 30);
             }
-            if (mol >= 0) {  // uniform: the oxygens among the hits within the molecule list's radius
+            if (OX && mol >= 0) {  // uniform: the oxygens among the hits within the molecule list's radius
                 int mj = -1;
                 if (hit && r2f <= ox.r2f) {
                     mj = ox.mol[ox.id[j]];
@@ -1020,7 +1033,7 @@ __device__ __forceinline__ void build_wave_body(int blk, int nblk, const int *__
         nlCount[i] = cnt;
         nlCountA[i] = cntA;
         waveMax[i] = cnt;
-        if (mol >= 0) {
+        if (OX && mol >= 0) {
             ox.count[mol] = cntO;
             ox.wmax[mol] = cntO;
         }
@@ -1135,7 +1148,7 @@ __device__ __forceinline__ void mol_map_body(int blk, int nblk, const int *__res
     }
 }
 
-template <bool SHIFT>
+template <bool SHIFT, bool OX>
 __device__ __forceinline__ void build_map_body(int blk, int nblk, const int *__restrict__ gate,
     int n, const double4 *__restrict__ pos, const float4 *__restrict__ xq, const BoxDev *__restrict__ bx,
     const int *__restrict__ colRank, const int *__restrict__ cellStart, int ncell,
@@ -1147,7 +1160,7 @@ __device__ __forceinline__ void build_map_body(int blk, int nblk, const int *__r
         mol_map_body(blk - nb, mm.blocks, gate, mm);
         return;
     }
-    build_wave_body<SHIFT>(blk, nb, gate, n, pos, xq, bx, colRank, cellStart, ncell, rlist2, ex, type, need, ox, cap, nl,
+    build_wave_body<SHIFT, OX>(blk, nb, gate, n, pos, xq, bx, colRank, cellStart, ncell, rlist2, ex, type, need, ox, cap, nl,
                            nlCount, nlCountA, flags, waveMax);
 }
 
@@ -1219,10 +1232,14 @@ void launch_build_wave(Ctx &c, const double4 *bpos, const BoxDev *box, const Mol
         c.waveMaxB = c.e3b.nmol;
     }
     const int blocks = cdiv(c.n, 4);
-    if (build_shifts(c))
-        launch<build_map_body<true>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, ex, c.type[c.cur], c.listNeed, ox, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm);
-    else
-        launch<build_map_body<false>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, ex, c.type[c.cur], c.listNeed, ox, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm);
+#define MDX_BUILD(S, O) launch<build_map_body<S, O>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, ex, c.type[c.cur], c.listNeed, ox, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm)
+    const bool shift = build_shifts(c);
+    if (ox.mol) {
+        if (shift) MDX_BUILD(true, true); else MDX_BUILD(false, true);
+    } else {
+        if (shift) MDX_BUILD(true, false); else MDX_BUILD(false, false);
+    }
+#undef MDX_BUILD
     c.waveMaxA = blocks * 4;
 }
 
