@@ -877,18 +877,19 @@ __device__ __forceinline__ void field_pack_body(int blk, int nblk, int ng, const
 }
 
 // ---------------------------------------------------------------------------
-// The mesh solve in three passes, for power-of-two meshes whose planes fit
-// one workgroup's LDS: the transforms of E_field_cu's pipeline
+// The mesh solve in three passes, for power-of-two meshes (each plane in one
+// workgroup's LDS): the transforms of E_field_cu's pipeline
 // (FixChargeEwald.cu: forward R2C of the charge mesh, E_hat_d =
 // i k_d G rho_hat, inverse C2R of each component), here as
 //   pass 1, one workgroup per x plane: the plane's charges (fixed point, read
 //     and cleared for the next spread; or the owner spread's real mesh), real
 //     FFTs along z two rows at a time (one complex FFT of row a + i row b,
 //     split by Hermitian symmetry), complex FFTs along y -> S1[x][ky][kz];
-//   pass 2, one wave per (ky, group of kz columns, component d): complex FFT
-//     along x gives rho_hat(kx, ky, kz), and i k_d G rho_hat goes back along
-//     x -> S2[d][x][ky][kz]; with energy or virial requested a fourth wave per
-//     column group sums them (kspace_ev_point) from its own rho_hat;
+//   pass 2, one wave per (ky, group of kz columns, component d), or per group
+//     with all three components: complex FFT along x gives rho_hat(kx, ky, kz),
+//     and i k_d G rho_hat goes back along x -> S2[d][x][ky][kz]; with energy or
+//     virial requested another wave per column group sums them
+//     (kspace_ev_point) from its own rho_hat;
 //   pass 3, one workgroup per (x plane, component): inverse complex FFTs along
 //     y, then the Hermitian inverse along z two rows at a time (row a + i row
 //     b, the imaginary parts of the kz = 0 and nz/2 terms dropped as a real
@@ -898,16 +899,23 @@ __device__ __forceinline__ void field_pack_body(int blk, int nblk, int ng, const
 // half-spectrum arrays (rho_hat, E_hat).  Every transform belongs to one
 // wave (its stages need no workgroup barrier): a Stockham autosort FFT
 // (natural order in and out) of radix-8 stages and one radix-4 or radix-2
-// stage, each lane doing whole radix-R butterflies in registers between two
-// LDS buffers (Govindaraju et al., "High performance discrete Fourier
-// transforms on graphics processors", SC 2008).
+// stage, each lane doing whole radix-R butterflies in registers (Govindaraju
+// et al., "High performance discrete Fourier transforms on graphics
+// processors", SC 2008).  A wave's lines fill its registers, so every stage,
+// the split of a row pair and its join run in place: one LDS copy of the plane
+// instead of three (a 128 x 128 plane 71 KB, two workgroups a CU), which also
+// lets planes move in and out whole and contiguous.  Bound by the vector
+// instructions of the stages for large planes, by the chain of latencies for
+// small ones.  The three launches: 32^3 25.2 -> 21.1 us, 32 x 32 x 64 27.1 ->
+// 21.7, 64^3 31.5 -> 26.1 (three buffers, runtime lengths); 128^3 88 -> 70
+// (library transforms with the conversion and field kernels around them;
+// over 42 boxes on meshes of 64 and 128 the forces' error against FP64 is 0.94
+// of the library's).
 constexpr int kFftMax = 128;      // longest axis; twiddles exp(-2 pi i k / 128), k < 128
 constexpr int kFftThreads = 256;  // pass 2: 4 waves, one (ky, columns, component) task each
-constexpr int kFftPlaneThreads = 512;  // passes 1 and 3: 8 waves, one group of lines each
 constexpr int kFftWavePts = 512;  // points a wave transforms at a time (lines x length)
 
 __device__ __forceinline__ int fft_log2(int n) { return __ffs(n) - 1; }
-
 
 // Workgroup barrier ordering LDS only: the passes read global memory that
 // earlier launches wrote and write what later launches read, so their
@@ -934,8 +942,11 @@ __device__ __forceinline__ void fft_twiddles(float2 *tw) {
     }
 }
 
-__device__ __forceinline__ float2 cmul(float2 a, float2 b) {
-    return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+// a * w, or a * conj(w) in the inverse; contracted by hand, so that every copy
+// of the transforms rounds alike
+__device__ __forceinline__ float2 cmul(float2 a, float2 w, bool inv) {
+    return inv ? make_float2(fmaf(a.x, w.x, a.y * w.y), fmaf(a.y, w.x, -(a.x * w.y)))
+               : make_float2(fmaf(a.x, w.x, -(a.y * w.y)), fmaf(a.y, w.x, a.x * w.y));
 }
 
 // multiplication by -i (forward) or +i (inverse)
@@ -984,137 +995,173 @@ __device__ __forceinline__ void small_dft<8>(float2 (&v)[8], bool inv) {
     }
 }
 
-// One Stockham stage of radix R (sub-transforms of length ns done so far) of
-// the calling wave's nl transforms of n points, element e of line l at
-// l * ls + e * es.  Neighbouring lanes take neighbouring lines.
-template <int R>
-__device__ __forceinline__ void wave_stage(const float2 *src, float2 *dst, int n, int ns, int nl, int ls, int es,
-                                           const float2 *tw, bool inv) {
-    const int nb = n / R;
-    const int step = kFftMax / (ns * R);
-    const float rnl = 1.0f / (float)nl;
-    for (int t = threadIdx.x & 63; t < nl * nb; t += 64) {
-        const int j = fft_div(t, rnl), l = t - j * nl;
-        const int jm = j & (ns - 1);
-        const float2 *sp = src + l * ls;
-        float2 v[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = sp[(j + r * nb) * es];
-#pragma unroll
-        for (int r = 1; r < R; ++r) {
-            float2 w = tw[(r * jm * step) & (kFftMax - 1)];
-            if (inv) w.y = -w.y;
-            v[r] = cmul(v[r], w);
-        }
-        small_dft<R>(v, inv);
-        float2 *dp = dst + l * ls;
-        const int base = (j - jm) * R + jm;
-#pragma unroll
-        for (int r = 0; r < R; ++r) dp[(base + r * ns) * es] = v[r];
-    }
-}
+// Place of element e of a line: the radix-8 stages write 8 elements apart,
+// which without the swap would put 8 lanes on one bank.
+__device__ __forceinline__ int fft_swz(int e) { return e ^ ((e >> 3) & 7); }
 
-// The calling wave's nl transforms of n points (a power of two, 2..128) from
-// a, with b the other buffer (the same layout); returns the one holding the
-// result.  The wave's earlier LDS writes to a are visible to it.
-__device__ __forceinline__ float2 *wave_fft(float2 *a, float2 *b, int n, int nl, int ls, int es, const float2 *tw,
-                                            bool inv) {
-    int ns = 1;
+// One Stockham stage of radix R (sub-transforms of length NS done so far) of
+// the calling wave's nl transforms of N points, element e of line l at
+// base(l) + fft_swz(e) * es.  Neighbouring lanes take neighbouring lines.  In
+// place: a wave's lines hold at most kFftWavePts points, 8 a lane, so it reads
+// all of them into registers before it writes any (its LDS accesses are
+// processed in order).  N is a template argument (a runtime length's index
+// arithmetic cost as much as the butterflies); the lane is made opaque so that
+// the addresses of every length are not computed ahead of the loops around.
+template <int R, int N, int NS, class Base>
+__device__ __forceinline__ void wave_stage(float2 *a, int nl, Base base, int es, const float2 *tw, bool inv) {
+    constexpr int NB = N / R, NL = kFftWavePts / N, K = kFftWavePts / 64 / R, step = kFftMax / (NS * R);
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    float2 v[K][R];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int t = lane + 64 * k, l = t & (NL - 1), j = t / NL, jm = j & (NS - 1);
+        if (l < nl) {
+            const float2 *sp = a + base(l);
+#pragma unroll
+            for (int r = 0; r < R; ++r) v[k][r] = sp[fft_swz(j + r * NB) * es];
+            if (NS > 1) {  // the first stage's factors are all 1
+#pragma unroll
+                for (int r = 1; r < R; ++r)
+                    v[k][r] = cmul(v[k][r], tw[(r * jm * step) & (kFftMax - 1)], inv);
+            }
+            small_dft<R>(v[k], inv);
+        }
+    }
     wave_sync();
-    while (ns < n) {
-        const int rem = n / ns;
-        if (rem >= 8) {
-            wave_stage<8>(a, b, n, ns, nl, ls, es, tw, inv);
-            ns *= 8;
-        } else if (rem == 4) {
-            wave_stage<4>(a, b, n, ns, nl, ls, es, tw, inv);
-            ns *= 4;
-        } else {
-            wave_stage<2>(a, b, n, ns, nl, ls, es, tw, inv);
-            ns *= 2;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int t = lane + 64 * k, l = t & (NL - 1), j = t / NL, jm = j & (NS - 1);
+        if (l < nl) {
+            float2 *dp = a + base(l);
+#pragma unroll
+            for (int r = 0; r < R; ++r) dp[fft_swz((j - jm) * R + jm + r * NS) * es] = v[k][r];
         }
-        float2 *x = a;
-        a = b;
-        b = x;
-        wave_sync();
     }
-    return a;
+    wave_sync();
 }
 
-// true when an n-point wave_fft ends in its first buffer (even stage count)
-__device__ __forceinline__ bool fft_ends_in_a(int n) {
-    int stages = 0;
-    for (int ns = 1; ns < n;) {
-        const int rem = n / ns;
-        ns *= rem >= 8 ? 8 : rem;
-        ++stages;
+template <int N, int NS, class Base>
+__device__ __forceinline__ void wave_stages(float2 *a, int nl, Base base, int es, const float2 *tw, bool inv) {
+    if constexpr (NS < N) {
+        constexpr int R = N / NS >= 8 ? 8 : N / NS;
+        wave_stage<R, N, NS>(a, nl, base, es, tw, inv);
+        wave_stages<N, NS * R>(a, nl, base, es, tw, inv);
     }
-    return (stages & 1) == 0;
 }
 
+// The calling wave's nl <= kFftWavePts / n transforms of n points (32, 64 or
+// 128), in place; the wave's earlier LDS writes are visible to it.
+template <class Base>
+__device__ __forceinline__ void wave_fft(float2 *a, int n, int nl, Base base, int es, const float2 *tw, bool inv) {
+    wave_sync();
+    switch (n) {
+        case 32: wave_stages<32, 1>(a, nl, base, es, tw, inv); break;
+        case 64: wave_stages<64, 1>(a, nl, base, es, tw, inv); break;
+        default: wave_stages<128, 1>(a, nl, base, es, tw, inv); break;
+    }
+}
+
+// A plane in LDS: row y (half spectrum, nz / 2 + 1 points) at fft_swz(y) rows
+// of fft_pitch; the pitch puts the 4 columns by 8 rows that half a wave takes
+// of a 128-row plane on 32 different bank pairs.  Rows 2r and 2r + 1 share the
+// room of one line of nz complex points.
+__device__ __forceinline__ int fft_pitch(int nz) { return nz / 2 + 4; }
+__device__ __forceinline__ int fft_pair(int r, int pitch) { return (fft_swz(2 * r) & ~1) * pitch; }
+
+template <int NT>
 __device__ __forceinline__ void fft_pass1_body(int blk, int nblk, const BoxDev *__restrict__ bx, long long *__restrict__ mesh,
                                                const float *__restrict__ real, float2 *__restrict__ S1) {
     extern __shared__ float2 fsh[];
     const MeshGeo m = bx->mesh;
     const int ny = m.sz[1], nz = m.sz[2], szh = nz / 2 + 1;
-    const int lz = fft_log2(nz);
-    const int rs = nz + 1;  // padded row pitch of the z transforms
-    const int cap = max((ny / 2) * rs, ny * szh);
-    float2 *tw = fsh;
-    float2 *A = tw + kFftMax, *B = A + cap, *Pl = B + cap;
-    fft_twiddles(tw);
-    const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    // the plane as ny / 2 row pairs (pitch rs): row 2r in .x, row 2r + 1 in .y
+    const int lz = fft_log2(nz), pitch = fft_pitch(nz);
+    float2 *tw = fsh, *A = tw + kFftMax;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    constexpr int nw = NT / 64;
+    // the plane as ny / 2 row pairs: row 2r in .x, row 2r + 1 in .y; a thread
+    // takes two neighbouring points of both
     const size_t base = (size_t)blk * ny * nz;
-    const int total = ny * nz;
-    constexpr int U = 8;
-    for (int t0 = threadIdx.x; t0 < total; t0 += U * kFftPlaneThreads) {
-        float v[U];
+    const int total = ny * nz / 4;
+    constexpr int U = 4;
+    for (int t0 = threadIdx.x; t0 < total; t0 += U * NT) {
+        float2 a[U], b[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int t = t0 + u * kFftPlaneThreads;
-            if (t < total) v[u] = mesh ? (float)((double)mesh[base + t] * kMeshInv) : real[base + t];
+            const int t = t0 + u * NT, r = t >> (lz - 1), z = 2 * (t & (nz / 2 - 1));
+            if (t < total) {
+                const size_t at = base + 2 * r * nz + z;
+                if (mesh) {
+                    const longlong2 p = *(const longlong2 *)(mesh + at), q = *(const longlong2 *)(mesh + at + nz);
+                    a[u] = make_float2((float)((double)p.x * kMeshInv), (float)((double)p.y * kMeshInv));
+                    b[u] = make_float2((float)((double)q.x * kMeshInv), (float)((double)q.y * kMeshInv));
+                } else {
+                    a[u] = *(const float2 *)(real + at);
+                    b[u] = *(const float2 *)(real + at + nz);
+                }
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int t = t0 + u * kFftPlaneThreads;
+            const int t = t0 + u * NT, r = t >> (lz - 1), z = 2 * (t & (nz / 2 - 1));
             if (t < total) {
-                if (mesh) mesh[base + t] = 0;
-                const int y = t >> lz, z = t & (nz - 1);
-                ((float *)(A + (y >> 1) * rs + z))[y & 1] = v[u];
+                const size_t at = base + 2 * r * nz + z;
+                if (mesh) {
+                    *(longlong2 *)(mesh + at) = make_longlong2(0, 0);
+                    *(longlong2 *)(mesh + at + nz) = make_longlong2(0, 0);
+                }
+                float2 *Z = A + fft_pair(r, pitch);
+                Z[fft_swz(z)] = make_float2(a[u].x, b[u].x);
+                Z[fft_swz(z + 1)] = make_float2(a[u].y, b[u].y);
+            }
+        }
+    }
+    fft_twiddles(tw);
+    fft_sync();
+    // z: groups of row pairs per wave; each wave splits its own pairs into their rows
+    const int lzw = kFftWavePts / nz;
+    const float rszh = 1.0f / (float)szh;
+    for (int r0 = wave * lzw; r0 < ny / 2; r0 += nw * lzw) {
+        const int nl = min(lzw, ny / 2 - r0);
+        wave_fft(A, nz, nl, [=](int l) { return fft_pair(r0 + l, pitch); }, 1, tw, false);
+        constexpr int K = kFftWavePts / 128 + 1;  // nl * szh <= 256 + 512 / nz, nz >= 32
+        float2 e[K], o[K];
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+            const int t = lane + 64 * u;
+            if (t < nl * szh) {
+                const int rr = fft_div(t, rszh), k = t - rr * szh;
+                const float2 *Z = A + fft_pair(r0 + rr, pitch);
+                const float2 P = Z[fft_swz(k)], Q = Z[fft_swz((nz - k) & (nz - 1))];
+                e[u] = make_float2(0.5f * (P.x + Q.x), 0.5f * (P.y - Q.y));
+                o[u] = make_float2(0.5f * (P.y + Q.y), -0.5f * (P.x - Q.x));
+            }
+        }
+        wave_sync();
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+            const int t = lane + 64 * u;
+            if (t < nl * szh) {
+                const int rr = fft_div(t, rszh), k = t - rr * szh, y = 2 * (r0 + rr);
+                A[fft_swz(y) * pitch + k] = e[u];
+                A[fft_swz(y + 1) * pitch + k] = o[u];
             }
         }
     }
     fft_sync();
-    // z: groups of row pairs per wave; each wave splits its own rows into Pl
-    const int lzw = kFftWavePts / nz;
-    const float2 *Z = A;
-    for (int r0 = wave * lzw; r0 < ny / 2; r0 += nw * lzw) {
-        const int nl = min(lzw, ny / 2 - r0);
-        Z = wave_fft(A + r0 * rs, B + r0 * rs, nz, nl, rs, 1, tw, false) - r0 * rs;
-        const float rszh = 1.0f / (float)szh;
-        for (int t = threadIdx.x & 63; t < nl * szh; t += 64) {
-            const int rr = fft_div(t, rszh), k = t - rr * szh, r = r0 + rr;
-            const float2 P = Z[r * rs + k], Q = Z[r * rs + ((nz - k) & (nz - 1))];
-            Pl[2 * r * szh + k] = make_float2(0.5f * (P.x + Q.x), 0.5f * (P.y - Q.y));
-            Pl[(2 * r + 1) * szh + k] = make_float2(0.5f * (P.y + Q.y), -0.5f * (P.x - Q.x));
-        }
-    }
-    fft_sync();
-    // y: groups of kz columns per wave, written out column group by group
+    // y: groups of kz columns per wave
     const int lyw = kFftWavePts / ny;
+    for (int c0 = wave * lyw; c0 < szh; c0 += nw * lyw)
+        wave_fft(A, ny, min(lyw, szh - c0), [=](int l) { return c0 + l; }, pitch, tw, false);
+    fft_sync();
     float2 *out = S1 + (size_t)blk * ny * szh;
-    for (int c0 = wave * lyw; c0 < szh; c0 += nw * lyw) {
-        const int nl = min(lyw, szh - c0);
-        const float2 *Y = wave_fft(Pl + c0, A + c0, ny, nl, 1, szh, tw, false) - c0;
-        const float rnl = 1.0f / (float)nl;
-        for (int t = threadIdx.x & 63; t < ny * nl; t += 64) {
-            const int y = fft_div(t, rnl), k = c0 + t - y * nl;
-            out[y * szh + k] = Y[y * szh + k];
-        }
+    for (int t = threadIdx.x; t < ny * szh; t += NT) {
+        const int y = fft_div(t, rszh);
+        out[t] = A[fft_swz(y) * pitch + t - y * szh];
     }
 }
 
+template <bool ALL>
 __device__ __forceinline__ void fft_pass2_body(int blk, int nblk, const BoxDev *__restrict__ bx, const float *__restrict__ G,
                                                const float2 *__restrict__ S1, float2 *__restrict__ S2, int ev,
                                                const int *__restrict__ gate, unsigned long long *__restrict__ acc) {
@@ -1132,14 +1179,17 @@ __device__ __forceinline__ void fft_pass2_body(int blk, int nblk, const BoxDev *
     const int task = blk * (blockDim.x >> 6) + wave;
     // task kinds: components 0..2, and with ev a fourth wave per column group
     // that only sums the k-space energy and virial (off the field waves' path)
-    const int kinds = ev ? 4 : 3;
+    const int comps = ALL ? 1 : 3, kinds = comps + (ev ? 1 : 0);
     if (task >= ny * ngr * kinds) return;
-    const int d = task % kinds, ky = (task / kinds) / ngr, kz0 = ((task / kinds) % ngr) * lw;
-    const bool sums = d == 3 && (!gate || *gate != 0);
-    if (d == 3 && !sums) return;
+    // ALL: neighbouring waves take neighbouring column groups
+    const int kind = ALL ? task / (ny * ngr) : task % kinds, col = ALL ? task % (ny * ngr) : task / kinds;
+    const int ky = col / ngr, kz0 = (col % ngr) * lw;
+    const bool sums = kind == comps && (!gate || *gate != 0);
+    if (kind == comps && !sums) return;
     const int nl = min(lw, szh - kz0);
-    float2 *A = tw + kFftMax + wave * 2 * kFftWavePts, *Bf = A + kFftWavePts;
-    // element (x, column l) at A[l + x * lw]; columns beyond szh are zero
+    float2 *A = tw + kFftMax + wave * kFftWavePts;
+    // element (x, column l), t = l + x * lw; columns beyond szh are zero
+    const auto at = [=](int t) { return (fft_swz(t >> llw) << llw) + (t & (lw - 1)); };
     constexpr int U = kFftWavePts / 64;
     float2 v[U];
     float g[U];
@@ -1155,9 +1205,9 @@ __device__ __forceinline__ void fft_pass2_body(int blk, int nblk, const BoxDev *
         }
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) A[lane + 64 * u] = v[u];
-    float2 *R = wave_fft(A, Bf, nx, lw, 1, lw, tw, false);
-    float2 *F = R == A ? Bf : A;
+    for (int u = 0; u < U; ++u) A[at(lane + 64 * u)] = v[u];
+    const auto line = [](int l) { return l; };
+    wave_fft(A, nx, lw, line, lw, tw, false);
     if (sums) {
         // kspace_ev_point's sums with the per-axis factors taken out of the
         // loop (k_d = m_d (2 pi / L_d), 1 / (4 alpha^2)): one division a point
@@ -1173,7 +1223,7 @@ __device__ __forceinline__ void fft_pass2_body(int blk, int nblk, const BoxDev *
                 const double k0 = (double)(2 * kx > nx ? kx - nx : kx) * ku0;
                 const double k2 = (double)(2 * kz > m.sz[2] ? kz - m.sz[2] : kz) * ku2;
                 const double kl = k0 * k0 + kyd * kyd + k2 * k2;
-                const float2 r = R[t];
+                const float2 r = A[at(t)];
                 const double wgt = (kz == 0 || 2 * kz == m.sz[2]) ? 1.0 : 2.0;
                 const double E = wgt * ((double)r.x * r.x + (double)r.y * r.y) * g[u];
                 vals[0] += hV * E;
@@ -1196,28 +1246,37 @@ __device__ __forceinline__ void fft_pass2_body(int blk, int nblk, const BoxDev *
         }
         return;
     }
-    // k_d of this wave's component: 2 pi m / L_d in FP32 (0 on the Nyquist plane)
-    const int nd = m.sz[d];
-    const float kunit = (float)(2.0 * kPi / m.L[d]);
+    // G rho_hat of the wave's points, then per component k_d = 2 pi m / L_d in
+    // FP32 (0 on the Nyquist plane)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        const int t = lane + 64 * u, l = t & (lw - 1), kx = t >> llw, kz = kz0 + l;
-        const float2 r = R[t];
-        const int id = d == 0 ? kx : (d == 1 ? ky : kz);
-        const int mi = 2 * id > nd ? id - nd : id;
-        const float kd = 2 * id == nd ? 0.0f : kunit * (float)mi;
-        const float gr = g[u] * r.x, gi = g[u] * r.y;
-        F[t] = make_float2(-kd * gi, kd * gr);
+        const float2 r = A[at(lane + 64 * u)];
+        v[u] = make_float2(g[u] * r.x, g[u] * r.y);
     }
-    const float2 *X = wave_fft(F, R, nx, lw, 1, lw, tw, true);
-    float2 *out = S2 + d * nh;
+#pragma unroll 1
+    for (int d = ALL ? 0 : kind; d < (ALL ? 3 : kind + 1); ++d) {
+        const int nd = m.sz[d];
+        const float kunit = (float)(2.0 * kPi / m.L[d]);
+        wave_sync();
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int t = lane + 64 * u, l = t & (lw - 1), x = t >> llw;
-        if (l < nl) out[(x * ny + ky) * szh + kz0 + l] = X[t];
+        for (int u = 0; u < U; ++u) {
+            const int t = lane + 64 * u, l = t & (lw - 1), kx = t >> llw, kz = kz0 + l;
+            const int id = d == 0 ? kx : (d == 1 ? ky : kz);
+            const int mi = 2 * id > nd ? id - nd : id;
+            const float kd = 2 * id == nd ? 0.0f : kunit * (float)mi;
+            A[at(t)] = make_float2(-kd * v[u].y, kd * v[u].x);
+        }
+        wave_fft(A, nx, lw, line, lw, tw, true);
+        float2 *out = S2 + (size_t)d * nh;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int t = lane + 64 * u, l = t & (lw - 1), x = t >> llw;
+            if (l < nl) out[(x * ny + ky) * szh + kz0 + l] = A[at(t)];
+        }
     }
 }
 
+template <int NT>
 __device__ __forceinline__ void fft_pass3_body(int blk, int nblk, const BoxDev *__restrict__ bx,
                                                const float2 *__restrict__ S2, float *__restrict__ E) {
     extern __shared__ float2 fsh[];
@@ -1225,76 +1284,73 @@ __device__ __forceinline__ void fft_pass3_body(int blk, int nblk, const BoxDev *
     const int nx = m.sz[0], ny = m.sz[1], nz = m.sz[2], szh = nz / 2 + 1;
     const size_t nh = (size_t)nx * ny * szh, ng = (size_t)nx * ny * nz;
     const int d = blk / nx, x = blk - d * nx;
-    const int lz = fft_log2(nz);
-    const int rs = nz + 1;  // padded row pitch of the z transforms
-    const int cap = max((ny / 2) * rs, ny * szh);
-    float2 *tw = fsh;
-    float2 *A = tw + kFftMax, *B = A + cap, *Q = B + cap;
+    const int lz = fft_log2(nz), pitch = fft_pitch(nz);
+    float2 *tw = fsh, *A = tw + kFftMax;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    constexpr int nw = NT / 64, U = 4;
+    const float2 *in = S2 + d * nh + (size_t)x * ny * szh;
+    const int total = ny * szh;
+    const float rszh = 1.0f / (float)szh;
+    for (int t0 = threadIdx.x; t0 < total; t0 += U * NT) {
+        float2 v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (t0 + u * NT < total) v[u] = in[t0 + u * NT];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int t = t0 + u * NT, y = fft_div(t, rszh);
+            if (t < total) A[fft_swz(y) * pitch + t - y * szh] = v[u];
+        }
+    }
     fft_twiddles(tw);
     fft_sync();
-    const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6, lane = threadIdx.x & 63;
-    // y: each wave loads and transforms its groups of kz columns
-    const float2 *in = S2 + d * nh + (size_t)x * ny * szh;
+    // y: groups of kz columns per wave
     const int lyw = kFftWavePts / ny;
-    const float2 *P = fft_ends_in_a(ny) ? A : B;  // the same for every wave's columns
-    for (int c0 = wave * lyw; c0 < szh; c0 += nw * lyw) {
-        const int nl = min(lyw, szh - c0);
-        constexpr int U = 8;
-        const float rnl = 1.0f / (float)nl;
-        for (int t0 = lane; t0 < ny * nl; t0 += 64 * U) {
-            float2 v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int t = t0 + 64 * u;
-                if (t < ny * nl) {
-                    const int y = fft_div(t, rnl), k = c0 + t - y * nl;
-                    v[u] = in[y * szh + k];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int t = t0 + 64 * u;
-                if (t < ny * nl) {
-                    const int y = fft_div(t, rnl), k = c0 + t - y * nl;
-                    A[y * szh + k] = v[u];
-                }
-            }
-        }
-        wave_fft(A + c0, B + c0, ny, nl, 1, szh, tw, true);
-    }
+    for (int c0 = wave * lyw; c0 < szh; c0 += nw * lyw)
+        wave_fft(A, ny, min(lyw, szh - c0), [=](int l) { return c0 + l; }, pitch, tw, true);
     fft_sync();
     // z: each wave builds and transforms its groups of row pairs
-    float2 *Pw = P == A ? B : A;  // free now (every wave's y transforms are done)
     const int lzw = kFftWavePts / nz;
     float *out = E + d * ng + (size_t)x * ny * nz;
     for (int r0 = wave * lzw; r0 < ny / 2; r0 += nw * lzw) {
         const int nl = min(lzw, ny / 2 - r0);
-        for (int t = lane; t < nl * nz; t += 64) {
-            const int rr = t >> lz, k = t & (nz - 1), r = r0 + rr;
-            float2 a, b;
-            if (2 * k <= nz) {
-                a = P[2 * r * szh + k];
-                b = P[(2 * r + 1) * szh + k];
-                if (k == 0 || 2 * k == nz) {
+        constexpr int K = kFftWavePts / 64;
+        float2 q[K];
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+            const int t = lane + 64 * u;
+            if (t < nl * nz) {
+                const int y = 2 * (r0 + (t >> lz)), k = t & (nz - 1);
+                const bool low = 2 * k <= nz;
+                const int kk = low ? k : nz - k;
+                float2 a = A[fft_swz(y) * pitch + kk], b = A[fft_swz(y + 1) * pitch + kk];
+                if (!low) {
+                    a.y = -a.y;
+                    b.y = -b.y;
+                } else if (k == 0 || 2 * k == nz) {
                     a.y = 0.0f;
                     b.y = 0.0f;
                 }
-            } else {
-                a = P[2 * r * szh + nz - k];
-                b = P[(2 * r + 1) * szh + nz - k];
-                a.y = -a.y;
-                b.y = -b.y;
+                q[u] = make_float2(a.x - b.y, a.y + b.x);
             }
-            Q[r * rs + k] = make_float2(a.x - b.y, a.y + b.x);
         }
-        const float2 *Z = wave_fft(Q + r0 * rs, Pw + r0 * rs, nz, nl, rs, 1, tw, true) - r0 * rs;
-        for (int t = lane; t < 2 * nl * nz; t += 64) {
-            const int y = 2 * r0 + t / nz, z = t & (nz - 1);
-            out[y * nz + z] = ((const float *)(Z + (y >> 1) * rs + z))[y & 1];
+        wave_sync();
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+            const int t = lane + 64 * u;
+            if (t < nl * nz) A[fft_pair(r0 + (t >> lz), pitch) + fft_swz(t & (nz - 1))] = q[u];
+        }
+        wave_fft(A, nz, nl, [=](int l) { return fft_pair(r0 + l, pitch); }, 1, tw, true);
+        for (int t = lane; t < nl * nz / 2; t += 64) {
+            const int r = r0 + (t >> (lz - 1)), z = 2 * (t & (nz / 2 - 1));
+            const float2 *Z = A + fft_pair(r, pitch);
+            const float2 v0 = Z[fft_swz(z)], v1 = Z[fft_swz(z + 1)];
+            float *row = out + (size_t)2 * r * nz + z;
+            *(float2 *)row = make_float2(v0.x, v1.x);
+            *(float2 *)(row + nz) = make_float2(v0.y, v1.y);
         }
     }
 }
-
 template <int ORDER, int T>
 __device__ __forceinline__ void gather_body(int blk, int nblk, int n, const double4 *__restrict__ pos,
                                                 const float *__restrict__ q, const BoxDev *__restrict__ bx,
@@ -1833,18 +1889,28 @@ static void pppm_plans_on(PppmState &P, hipStream_t s) {
     P.planStream = s;
 }
 
-// LDS bytes of passes 1 and 3 of the mesh solve, 0 where the mesh does not
-// allow it (every axis a power of two from 4 to 128, the planes within
-// 60 KB).  Pass 2 takes kFftMax + 2 * kFftWavePts points per wave.
+// Planes of more points than this take 1,024 threads in passes 1 and 3 (128^3
+// 80 -> 70 us, 64 x 128 x 128 54 -> 47), smaller ones 512 (32^3 21.1 against
+// 23.9 us, 64^3 equal).
+constexpr int kFftBigPlane = 4096;
+// Column groups from which a wave of pass 2 does all three components, reading
+// and transforming rho once: as many as fill the chip's SIMDs by themselves
+// (128^3, 2,176 groups: 78 -> 70 us; 64 x 64 x 128, 576: 33 -> 34; 64^3, 320:
+// 26 -> 28).
+constexpr int kFftAllCols = 1024;
+
+// LDS bytes of passes 1 and 3 of the mesh solve, 0 where the mesh takes the
+// library transforms: every axis must be 32, 64 or 128, and
+// there must be at least 64 planes if they are large (one workgroup each: with
+// fewer most CUs idle through pass 1).  Pass 2 takes kFftMax + kFftWavePts
+// points per wave.
 static size_t lds_fft_shm(const PppmState &P) {
     for (int a = 0; a < 3; ++a) {
         const int n = P.sz[a];
-        if (n < 4 || n > kFftMax || (n & (n - 1))) return 0;
+        if (n < 32 || n > kFftMax || (n & (n - 1))) return 0;
     }
-    const size_t szh = P.sz[2] / 2 + 1;
-    const size_t cap = std::max((size_t)(P.sz[1] / 2) * (P.sz[2] + 1), (size_t)P.sz[1] * szh);
-    const size_t b = sizeof(float2) * (kFftMax + 3 * cap);
-    return b <= 60 * 1024 ? b : 0;
+    if (P.sz[1] * P.sz[2] > kFftBigPlane && P.sz[0] < 64) return 0;
+    return sizeof(float2) * (kFftMax + (size_t)P.sz[1] * (P.sz[2] / 2 + 4));
 }
 
 bool pppm_lds_fft(const PppmState &P) { return P.fftMode == 1 && lds_fft_shm(P) > 0; }
@@ -1864,13 +1930,18 @@ static void mesh_solve(Ctx &c, bool fromReal, int ev, const int *gate) {
         P.lastFft = 1;
         ProfScope ps(c, PK_FFT);
         const int waves = kFftThreads / 64;
-        const int lw = kFftWavePts / sz[0], tasks = sz[1] * ((szh + lw - 1) / lw) * (ev ? 4 : 3);
-        const size_t shm2 = sizeof(float2) * (kFftMax + waves * 2 * kFftWavePts);
-        launch<fft_pass1_body, kFftPlaneThreads>(c, sz[0], shm, c.box, fromReal ? nullptr : P.mesh,
-                                                 fromReal ? P.real : nullptr, P.rhoHat);
-        launch<fft_pass2_body, kFftThreads>(c, cdiv(tasks, waves), shm2, c.box, P.green, P.rhoHat, P.eHat, ev, gate,
-                                            c.acc);
-        launch<fft_pass3_body, kFftPlaneThreads>(c, 3 * sz[0], shm, c.box, P.eHat, P.eReal);
+        const int lw = kFftWavePts / sz[0], cols = sz[1] * ((szh + lw - 1) / lw);
+        const bool all = cols >= kFftAllCols, big = sz[1] * sz[2] > kFftBigPlane;
+        const size_t shm2 = sizeof(float2) * (kFftMax + waves * kFftWavePts);
+        long long *mesh = fromReal ? nullptr : P.mesh;
+        const float *real = fromReal ? P.real : nullptr;
+        if (big) launch<fft_pass1_body<1024>, 1024>(c, sz[0], shm, c.box, mesh, real, P.rhoHat);
+        else launch<fft_pass1_body<512>, 512>(c, sz[0], shm, c.box, mesh, real, P.rhoHat);
+        const int tasks = cols * ((all ? 1 : 3) + (ev ? 1 : 0));
+        if (all) launch<fft_pass2_body<true>, kFftThreads>(c, cdiv(tasks, waves), shm2, c.box, P.green, P.rhoHat, P.eHat, ev, gate, c.acc);
+        else launch<fft_pass2_body<false>, kFftThreads>(c, cdiv(tasks, waves), shm2, c.box, P.green, P.rhoHat, P.eHat, ev, gate, c.acc);
+        if (big) launch<fft_pass3_body<1024>, 1024>(c, 3 * sz[0], shm, c.box, P.eHat, P.eReal);
+        else launch<fft_pass3_body<512>, 512>(c, 3 * sz[0], shm, c.box, P.eHat, P.eReal);
         return;
     }
     P.lastFft = 0;
