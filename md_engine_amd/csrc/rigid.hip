@@ -149,12 +149,20 @@ __device__ __forceinline__ void dist_forces(const unsigned long long *f, int4 a,
 // and, in workgroup 0, the cleared energy / virial accumulators - so no
 // separate refresh launch is needed (a rebuild's permutation rewrites xq and
 // the records in the new order).
+//
+// Bound by the chain of FP64 latencies of SETTLE and then of the sites' stores,
+// refresh and check.  T = 4: four lanes do a molecule's SETTLE alike and take a
+// site each after it, while the wider launch still is about one wave a SIMD:
+// 512 molecules 9.8 -> 7.1 us, 4,096 11.6 -> 8.5, 8,192 13.5 -> 10.7, but
+// 32,768 14.7 -> 18.0, which keep one lane a molecule.
+constexpr int kRigidTeamMax = 16384;
+template <int T>
 __device__ __forceinline__ void rigid_vv1_body(int blk, int nblk, RigidArgs r, double4 *__restrict__ pos, double4 *__restrict__ vel,
                                                    const unsigned long long *__restrict__ f,
                                                    const double4 *__restrict__ last, double dt2,
                                                    unsigned *__restrict__ slots, RefreshArgs ra) {
     r.g = r.bx->geo;
-    const int m = blk * blockDim.x + threadIdx.x;
+    const int m = (blk * blockDim.x + threadIdx.x) / T;
     float d2 = 0.f, p2 = 0.f;
     if (ra.xq && blk == 0) refresh_clear(ra);
     if (m < r.nmol) {
@@ -177,42 +185,27 @@ __device__ __forceinline__ void rigid_vv1_body(int blk, int nblk, RigidArgs r, d
     vH2 = vH2 + idt * (C3 - C1);
     const d3 nO = xO + A3;
     const d3 nH1 = nO + (B3 - A3), nH2 = nO + (C3 - A3);
-    pos[a.x] = make_double4(nO.x, nO.y, nO.z, pO.w);
-    pos[a.y] = make_double4(nH1.x, nH1.y, nH1.z, pH1.w);
-    pos[a.z] = make_double4(nH2.x, nH2.y, nH2.z, pH2.w);
-    vel[a.x] = make_double4(vO.x, vO.y, vO.z, wO.w);
-    vel[a.y] = make_double4(vH1.x, vH1.y, vH1.z, wH1.w);
-    vel[a.z] = make_double4(vH2.x, vH2.y, vH2.z, wH2.w);
-    double4 sp[4];
-    sp[0] = make_double4(nO.x, nO.y, nO.z, pO.w);
-    sp[1] = make_double4(nH1.x, nH1.y, nH1.z, pH1.w);
-    sp[2] = make_double4(nH2.x, nH2.y, nH2.z, pH2.w);
-    if (a.w >= 0) {
-        const d3 nM = nO + (0.5 * (1.0 - r.gamma)) * ((B3 - A3) + (C3 - A3));
-        const double4 pM = pos[a.w];
-        sp[3] = make_double4(nM.x, nM.y, nM.z, pM.w);
-        pos[a.w] = sp[3];
-        vel[a.w] = make_double4(0.0, 0.0, 0.0, vel[a.w].w);
-    }
-    if (ra.xq) {
-        const int site[4] = {a.x, a.y, a.z, a.w};
+    const d3 nM = nO + (0.5 * (1.0 - r.gamma)) * ((B3 - A3) + (C3 - A3));
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            if (site[s] < 0) continue;
-            refresh_site(ra, site[s], sp[s], r.bx, r.g);
+    for (int u = 0; u < 4 / T; ++u) {
+        const int k = T == 1 ? u : (int)(threadIdx.x & 3);
+        const int site = k == 0 ? a.x : k == 1 ? a.y : k == 2 ? a.z : a.w;
+        if (site < 0) continue;
+        const d3 x = k == 0 ? nO : k == 1 ? nH1 : k == 2 ? nH2 : nM;
+        const d3 v = k == 0 ? vO : k == 1 ? vH1 : k == 2 ? vH2 : mk(0.0, 0.0, 0.0);
+        const double xw = k == 0 ? pO.w : k == 1 ? pH1.w : k == 2 ? pH2.w : pos[site].w;
+        const double vw = k == 0 ? wO.w : k == 1 ? wH1.w : k == 2 ? wH2.w : vel[site].w;
+        const double4 sp = make_double4(x.x, x.y, x.z, xw);
+        pos[site] = sp;
+        vel[site] = make_double4(v.x, v.y, v.z, vw);
+        asm volatile("" ::: "memory");  // the molecule's forces were read above; the refresh clears them
+        if (ra.xq) refresh_site(ra, site, sp, r.bx, r.g);
+        if (slots) {
+            const double dd = disp2(sp, last[site], r.g);
+            const double p = sqrt(dd) + dt2 * sqrt(v.x * v.x + v.y * v.y + v.z * v.z);
+            d2 = fmaxf(d2, (float)dd);
+            p2 = fmaxf(p2, (float)(p * p));
         }
-    }
-    if (slots) {
-        const int site[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-            if (site[s] >= 0) {
-                const d3 v = s == 0 ? vO : s == 1 ? vH1 : s == 2 ? vH2 : mk(0.0, 0.0, 0.0);
-                const double dd = disp2(sp[s], last[site[s]], r.g);
-                const double p = sqrt(dd) + dt2 * sqrt(v.x * v.x + v.y * v.y + v.z * v.z);
-                d2 = fmaxf(d2, (float)dd);
-                p2 = fmaxf(p2, (float)(p * p));
-            }
     }
     }
     if (slots) disp_fold(d2, p2, slots, blk);
@@ -449,7 +442,11 @@ void rigid_first_half(Ctx &c) {
     const RigidArgs r = make_args(c);
     RefreshArgs ra{};
     if (c.fuseCheck) ra = refresh_args(c);
-    launch<rigid_vv1_body, 128>(c, cdiv(r.nmol, 128), 0, r, c.pos[c.cur], c.vel[c.cur], c.force, c.posLast, 2.0 * c.dt, c.fuseCheck ? c.dispSlots : nullptr, ra);
+    unsigned *slots = c.fuseCheck ? c.dispSlots : nullptr;
+    if (r.nmol <= kRigidTeamMax)
+        launch<rigid_vv1_body<4>, 128>(c, cdiv(4 * r.nmol, 128), 0, r, c.pos[c.cur], c.vel[c.cur], c.force, c.posLast, 2.0 * c.dt, slots, ra);
+    else
+        launch<rigid_vv1_body<1>, 128>(c, cdiv(r.nmol, 128), 0, r, c.pos[c.cur], c.vel[c.cur], c.force, c.posLast, 2.0 * c.dt, slots, ra);
 }
 
 void rigid_second_half(Ctx &c, bool kick) {
