@@ -284,7 +284,13 @@ void snapshot_save(Ctx &c) {
         MDX_HIP(hipMemcpyAsync(c.snap.posLast, c.posLast, sizeof(double4) * c.n, hipMemcpyDeviceToDevice,
                                c.stream));
         MDX_HIP(hipMemcpyAsync(c.snap.boxLast, c.boxLast, sizeof(BoxDev), hipMemcpyDeviceToDevice, c.stream));
+        // Forces carried into the chunk belong to the positions before the
+        // last step's dilation: the replay takes these, as the chunk did.
+        if (!c.snap.force) c.snap.force = dalloc<unsigned long long>(c, 3 * (size_t)c.n);
+        MDX_HIP(hipMemcpyAsync(c.snap.force, c.force, sizeof(unsigned long long) * 3 * c.n, hipMemcpyDeviceToDevice,
+                               c.stream));
     }
+    c.snap.forceFlags = c.snap.listValid ? c.forceFlags : -1;
     if (c.box) {
         if (!c.snap.box) c.snap.box = dalloc<BoxDev>(c, 1);
         MDX_HIP(hipMemcpyAsync(c.snap.box, c.box, sizeof(BoxDev), hipMemcpyDeviceToDevice, c.stream));
@@ -347,7 +353,10 @@ void snapshot_restore(Ctx &c) {
         MDX_HIP(hipMemcpyAsync(c.box, c.snap.box, sizeof(BoxDev), hipMemcpyDeviceToDevice, c.stream));
         box_pull(c);
         refresh_xq(c);
+        MDX_HIP(hipMemcpyAsync(c.force, c.snap.force, sizeof(unsigned long long) * 3 * c.n, hipMemcpyDeviceToDevice,
+                               c.stream));
     }
+    c.forceFlags = relist ? c.snap.forceFlags : -1;
     c.nRebuilds = c.snap.rebuilds;
     bool moved = false;
     for (int d = 0; d < 3; ++d) moved = moved || c.snap.geo.L[d] != c.geo.L[d] || c.snap.geo.lo[d] != c.geo.lo[d];
@@ -1121,8 +1130,10 @@ void run_captured(const std::vector<Ctx *> &cs, int nsteps, int flags, const Rin
                     // rows grow first: the restore builds the starting list into them
                     if (overflow[k]) grow_if_needed(c);
                     snapshot_restore(c);
-                    if (badGrid[k]) c.nlistConfigured = false;
-                    c.forceFlags = -1;
+                    if (badGrid[k]) {
+                        c.nlistConfigured = false;
+                        c.forceFlags = -1;
+                    }
                 }
                 drop();
                 continue;
@@ -2119,7 +2130,6 @@ int mdx_run(mdx_ctx *ctx, int nsteps, int flags) {
             if (!capacity_ok(c) || forced) {
                 // a build overflowed its rows: redo the chunk with the grown rows
                 snapshot_restore(c);
-                c.forceFlags = -1;
                 continue;
             }
             ++chunkNo;

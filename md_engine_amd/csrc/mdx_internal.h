@@ -612,6 +612,10 @@ struct Ctx {
         bool listValid = false;
         double4 *posLast = nullptr;
         BoxDev *boxLast = nullptr;
+        // the forces carried in with that list (a barostat moved the sites after
+        // their evaluation, so a replay cannot compute them again)
+        unsigned long long *force = nullptr;
+        int forceFlags = -1;
         double *nh = nullptr;                 // Nose-Hoover chain state (4 chain + 2 doubles)
         int nhLen = 0;
         unsigned long long *thermo = nullptr; // thermostat sums (2 words)

@@ -136,3 +136,28 @@ def test_batch_replay_keeps_replicas_in_step(gpu_engine_factory, trigger):
         assert np.array_equal(vb, vs)
     for e in batch:
         e.close()
+
+
+@pytest.mark.parametrize("graph", [0, 1])
+def test_replay_under_a_barostat_is_exact(gpu_engine_factory, graph):
+    """The barostat dilates the sites after a step's forces, and the next
+    step's first kick takes those forces: a chunk replayed from a carried list
+    takes them too, not the forces at the dilated positions."""
+    say(f"replay under a barostat, graph={graph}")
+    out = []
+    for chunk in (0, 2):
+        e, flags = water(gpu_engine_factory, 343, 33, nh=False)
+        e.thermostat(True, 298.0, 10, 0.0, systems.REAL_BOLTZ, systems.REAL_MVV_TO_ENG)
+        e.barostat(True, 1.0, 100.0, 1, 10.0, 1e-5, mvv_to_eng=systems.REAL_MVV_TO_ENG)
+        e.option("graph", graph)
+        e.option("replay_chunk", chunk)
+        e.run(192, flags)
+        x, v = e.get_system()
+        out.append((x, v, e.get_box()[1], e.nlist_stats()["rebuilds"]))
+        e.close()
+    (xr, vr, Lr, nr), (xt, vt, Lt, nt) = out
+    say(f"  max |dx| {np.abs(xr - xt).max():.2e}, rebuilds {nr} / {nt}")
+    assert nr == nt
+    assert np.array_equal(Lr, Lt)
+    assert np.array_equal(xr, xt)
+    assert np.array_equal(vr, vt)
