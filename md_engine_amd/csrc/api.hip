@@ -1130,7 +1130,8 @@ void run_captured(const std::vector<Ctx *> &cs, int nsteps, int flags, const Rin
                     // rows grow first: the restore builds the starting list into them
                     if (overflow[k]) grow_if_needed(c);
                     snapshot_restore(c);
-                    if (badGrid[k]) {
+                    if (badGrid[k]) {  // room for every dilation of a chunk
+                        c.baro.shrink = std::pow(1.0 - c.baro.maxDil, kGraphChunk) * (1.0 - 1e-9);
                         c.nlistConfigured = false;
                         c.forceFlags = -1;
                     }
@@ -2829,6 +2830,7 @@ int mdx_barostat_set(mdx_ctx *ctx, int enable, double pressure, double period, i
         B.every = every;
         B.bulk = bulk_modulus;
         B.maxDil = max_dilation;
+        B.shrink = 1.0;
         B.nktv2p = nktv_to_press;
         B.mvv = mvv_to_eng;
     });

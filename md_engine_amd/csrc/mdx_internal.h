@@ -356,6 +356,7 @@ struct BarostatState {
     double P0 = 1.0, period = 1000.0, bulk = 10.0, maxDil = 1e-5, nktv2p = 68568.415, mvv = 1.0;
     int every = 10;
     double lastP = 0.0;
+    double shrink = 1.0;  // smallest box factor of a chunk, once a chunk outran its grid
 };
 
 // learned E3B three-body surrogate (surrogate.hip)
@@ -1133,8 +1134,9 @@ inline const int *rebuild_gate(const Ctx &c) { return c.capture ? c.dFlags + 3 :
 inline const int *thermo_gate(const Ctx &c) { return c.capture ? c.dFlags + 5 : nullptr; }
 inline const int *baro_gate(const Ctx &c) { return c.capture ? c.dFlags + 8 : nullptr; }
 // cells are sized for a box 0.1 % smaller while a barostat runs, so that the
-// grid outlives about a hundred maximal dilations
-inline double grid_headroom(const Ctx &c) { return c.baro.on ? 0.999 : 1.0; }
+// grid outlives about a hundred maximal dilations of 1e-5; a barostat whose
+// captured chunk shrank the box by more leaves room for a chunk of its own
+inline double grid_headroom(const Ctx &c) { return c.baro.on ? std::min(0.999, c.baro.shrink) : 1.0; }
 
 // per-module entry points ------------------------------------------------------
 // nlist.hip

@@ -1339,6 +1339,7 @@ void nlist_setup(Ctx &c) {
         c.nlCountA = dalloc<int>(c, c.n);
     }
     c.nlistConfigured = true;
+    c.listValid = false;  // the cells of a list built on another grid are gone
     ++c.layoutEpoch;  // cell counts and tables are kernel arguments of captured steps
     box_upload(c);  // cell counts changed
 }

@@ -210,3 +210,45 @@ def test_eager_barostat_through_grid_changes(orc, gpu_engine_factory, sign):
     oc, orows, _ = oracle_rows_by_id(orc, x, lo, L, rc + skin, excl=excl, brute=False)
     assert_same_lists(gc, grows, oc, orows)
     e.close()
+
+
+def test_captured_barostat_through_a_grid_change(orc, gpu_engine_factory):
+    """Captured steps find at the end of a chunk that the box outran its cell
+    grid, and replay it on a coarser one, also where a list was carried into
+    the chunk and where one chunk shrinks the box by more than a grid's usual
+    headroom (4e-4 a step).  Eager steps change the grid inside the chunk.
+
+    A run that sets its grid up computes the forces again, at the dilated
+    positions, for one half kick, eager and captured at different steps: 4e-4
+    of a distance is at most 13 x 4e-4 of a force (r^-13), some 30 kcal/mol/A
+    on a hydrogen, so 0.5 x 1.3e-2 A/fs^2 x 5e-3 = 3e-5 A/fs, 2e-3 A over the
+    64 steps for each of the two."""
+    say("captured barostat through a grid change")
+    box = systems.tip4p2005_box(283, seed=35, min_sep=1.8)
+    v = start_velocities(orc, box, seed=8)
+    out = []
+    for graph in (0, 1):
+        e, flags = water_md_engine(gpu_engine_factory, box, v, rc=7.0, skin=1.0, sz=(32, 32, 32), order=5, e3b=True,
+                                   dt=1.0)
+        e.thermostat(True, 298.0, 5, 0.0, systems.REAL_BOLTZ, systems.REAL_MVV_TO_ENG)
+        e.barostat(True, 1e9, 1.0, 1, bulk_modulus=1e-3, max_dilation=4e-4, mvv_to_eng=systems.REAL_MVV_TO_ENG)
+        e.option("graph", graph)
+        e.run(8, flags)
+        cells = e.nlist_stats()["cells"]
+        e.run(64, flags)
+        assert tuple(e.nlist_stats()["cells"]) != tuple(cells)
+        x, _ = e.get_system()
+        lo, L = e.get_box()
+        assert np.allclose(L, box["L"] * (1.0 - 4e-4) ** 72, rtol=1e-9)
+        out.append(x)
+        e.nlist_update(force=True)
+        from test_gpu_parity import assert_same_lists, oracle_rows_by_id
+
+        gc, grows = e.nlist_get()
+        excl = orc.exclusions_bfs(len(x), systems.water_bonds(box["mol"]))
+        oc, orows, _ = oracle_rows_by_id(orc, x, lo, L, 8.0, excl=excl, brute=False)
+        assert_same_lists(gc, grows, oc, orows)
+        e.close()
+    dx = np.abs(min_image_diff(out[0], out[1], L)).max()
+    say(f"  max |dx| eager against captured {dx:.1e}")
+    assert dx < 4e-3
