@@ -502,7 +502,7 @@ struct Ctx {
     // cell stencil half-width per axis (cell edge >= rlist / reach); thinner z
     // cells cut the z-runs closer to the sphere
     int reach[3] = {2, 2, 4};
-    int ncell = 0;
+    int ncell = 0, ncol = 0;      // cells and cell columns the tables below are made for
     int *colRank = nullptr;
     int *cellStart = nullptr;     // 2 ncell + 1: cells of the charged atoms, then of the charge-free ones
     // re-sort: per cell slot a list of its atoms (head, -1 when empty; next by

@@ -1276,8 +1276,8 @@ void nlist_setup(Ctx &c) {
         int nca = (int)std::floor(c.geo.L[a] * grid_headroom(c) / edge);
         c.nc[a] = std::max(1, nca);
     }
-    int ncell = c.nc[0] * c.nc[1] * c.nc[2];
-    if (ncell != c.ncell) {
+    const int ncol = c.nc[0] * c.nc[1], ncell = ncol * c.nc[2];
+    if (ncell != c.ncell || ncol != c.ncol) {  // a box turned on its side keeps its cells, not its columns
         MDX_REQUIRE(!c.capture, 3, "the cell grid cannot change while a step is captured");
         if (c.ncell) {
             dfree(c, c.colXY);
@@ -1286,8 +1286,9 @@ void nlist_setup(Ctx &c) {
             dfree(c, c.cellStart);
         }
         c.ncell = ncell;
-        c.colRank = dalloc<int>(c, (size_t)c.nc[0] * c.nc[1]);
-        c.colXY = dalloc<int2>(c, (size_t)c.nc[0] * c.nc[1]);
+        c.ncol = ncol;
+        c.colRank = dalloc<int>(c, ncol);
+        c.colXY = dalloc<int2>(c, ncol);
         // two copies of the grid: charged atoms, then charge-free ones
         c.cellHead = dalloc<int>(c, 2 * (size_t)ncell);
         // the sort leaves the lists empty for the next binning

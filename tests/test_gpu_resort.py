@@ -172,3 +172,28 @@ def test_whole_list_from_partial_rows(orc, gpu_engine_factory, graph, team):
         out.append(k.forces())
         k.close()
     assert np.array_equal(out[0], out[1])
+
+
+def test_box_turned_on_its_side(orc, gpu_engine_factory):
+    """An elongated box turned on one engine: 6 x 6 x 24 cells (36 columns),
+    then 12 x 6 x 12 (as many cells, 72 columns) and back."""
+    say("elongated box turned on its side")
+    rng = np.random.default_rng(7)
+    n, rlist = 1500, 10.0
+    q = np.where(rng.random(n) < 0.4, 0.3, 0.0)
+    u = rng.uniform(0, 1, (n, 3))
+    e = None
+    for L, cells in ((np.array([31.0, 31.0, 62.0]), (6, 6, 24)), (np.array([62.0, 31.0, 31.0]), (12, 6, 12)),
+                     (np.array([31.0, 31.0, 62.0]), (6, 6, 24))):
+        x = u * L
+        if e is None:
+            e = _list_engine(gpu_engine_factory, x, L, rlist, 1.0, q=q)
+        else:
+            e.set_box(np.zeros(3), L)
+            e.set_positions(x)
+        e.nlist_update(force=True)
+        assert tuple(e.nlist_stats()["cells"]) == cells
+        gc, grows = e.nlist_get()
+        oc, orows, _ = oracle_rows_by_id(orc, x, np.zeros(3), L, rlist, brute=True)
+        assert_same_lists(gc, grows, oc, orows)
+    e.close()
