@@ -273,6 +273,8 @@ void snapshot_save(Ctx &c) {
     c.snap.turn = c.turn;
     c.snap.rebuilds = c.nRebuilds;
     c.snap.geo = c.geo;
+    c.snap.grid = c.nlistConfigured;
+    for (int a = 0; a < 3; ++a) c.snap.nc[a] = c.nc[a];
     // A list carried into the chunk was built earlier, from other positions:
     // its rows (their order sets the FP32 summation order of the pair sums)
     // and the skin check's reference positions are the build's.  Keep the
@@ -338,6 +340,14 @@ void snapshot_restore(Ctx &c) {
     }
     c.turn = c.snap.turn;
     c.listValid = false;
+    // A barostat may have set another grid up inside the chunk.  The records'
+    // order and the device boxes kept here are of the one it started with.
+    if (!c.snap.grid) {
+        c.nlistConfigured = false;
+    } else if (!c.nlistConfigured || !std::equal(c.nc, c.nc + 3, c.snap.nc)) {
+        c.geo = c.snap.geo;
+        nlist_setup(c, c.snap.nc);
+    }
     const bool relist = c.snap.listValid && c.nlistConfigured;
     if (relist) {
         // Build the chunk's starting list again from the positions and box of
@@ -368,12 +378,7 @@ void snapshot_restore(Ctx &c) {
         if (c.pppm.on) pppm_green_device(c, nullptr);
         moved = true;
     }
-    if (moved) {  // a barostat changed the box during the replayed chunk
-        c.geo = c.snap.geo;
-        // the grid that built the starting list was valid for the starting
-        // box; without a carried list the grid is set up again
-        if (!relist) c.nlistConfigured = false;
-    }
+    if (moved) c.geo = c.snap.geo;  // a barostat changed the box during the replayed chunk
 }
 
 // Reads the check of one step earlier (waits only for that step's check,

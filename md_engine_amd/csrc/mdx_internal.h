@@ -608,6 +608,8 @@ struct Ctx {
         long long turn = 0, rebuilds = 0;
         Geometry geo;
         BoxDev *box = nullptr;
+        bool grid = false;  // a cell grid was set up, and its cells per axis
+        int nc[3] = {0, 0, 0};
         // the list the chunk started with, when one carried into it: the
         // positions and box of its build (a replay rebuilds it from them)
         bool listValid = false;
@@ -1140,7 +1142,7 @@ inline double grid_headroom(const Ctx &c) { return c.baro.on ? std::min(0.999, c
 
 // per-module entry points ------------------------------------------------------
 // nlist.hip
-void nlist_setup(Ctx &c);
+void nlist_setup(Ctx &c, const int *cells = nullptr);  // cells per axis: of the box, or as given
 void nlist_check(Ctx &c);             // sets dFlags[0] when a rebuild is due
 DecideArgs decide_args(const Ctx &c);  // the step decisions of a captured step
 RowMaxArgs row_max_args(Ctx &c);        // a captured build's pending row maxima (clears the request)

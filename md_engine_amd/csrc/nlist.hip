@@ -1265,7 +1265,7 @@ void launch_e3b_list(Ctx &c, const double4 *bpos, const BoxDev *box) {
 
 }  // namespace
 
-void nlist_setup(Ctx &c) {
+void nlist_setup(Ctx &c, const int *cells) {
     MDX_REQUIRE(c.n > 0, 3, "system not set");
     MDX_REQUIRE(c.rlist > 0, 1, "neighbor list cutoff must be positive");
     for (int a = 0; a < 3; ++a) {
@@ -1274,7 +1274,7 @@ void nlist_setup(Ctx &c) {
                         "neighbor cutoff (rCut + padding) must be below half the box length");
         double edge = c.rlist / c.reach[a] * (1.0 + 1e-9);
         int nca = (int)std::floor(c.geo.L[a] * grid_headroom(c) / edge);
-        c.nc[a] = std::max(1, nca);
+        c.nc[a] = cells ? cells[a] : std::max(1, nca);
     }
     const int ncol = c.nc[0] * c.nc[1], ncell = ncol * c.nc[2];
     if (ncell != c.ncell || ncol != c.ncol) {  // a box turned on its side keeps its cells, not its columns

@@ -161,3 +161,40 @@ def test_replay_under_a_barostat_is_exact(gpu_engine_factory, graph):
     assert np.array_equal(Lr, Lt)
     assert np.array_equal(xr, xt)
     assert np.array_equal(vr, vt)
+
+
+def shrinking_water(make, e3b=False):
+    """A box that loses a cell per axis near step 50 of a run: every step
+    shrinks it by the largest dilation."""
+    box = systems.tip4p2005_box(283, seed=35, min_sep=1.8)
+    import oracle
+    from test_gpu_water_md import start_velocities, water_md_engine
+
+    e, flags = water_md_engine(make, box, start_velocities(oracle, box, seed=8), rc=7.0, skin=1.0, sz=(32, 32, 32),
+                               order=5, e3b=e3b, dt=1.0)
+    e.thermostat(True, 298.0, 5, 0.0, systems.REAL_BOLTZ, systems.REAL_MVV_TO_ENG)
+    e.barostat(True, 1e9, 1.0, 1, bulk_modulus=1e-3, max_dilation=4e-4, mvv_to_eng=systems.REAL_MVV_TO_ENG)
+    return e, flags, box
+
+
+def test_replay_of_a_chunk_with_a_grid_change(gpu_engine_factory):
+    """Eager steps under a barostat set a coarser cell grid up inside a chunk;
+    replayed from a carried list, the chunk starts on its own grid again, with
+    the sites in that grid's order, and changes it at the same step."""
+    say("replay of a chunk with a grid change")
+    out = []
+    for chunk in (0, 1):
+        e, flags, _ = shrinking_water(gpu_engine_factory)
+        e.option("graph", 0)
+        e.run(8, flags)
+        cells = e.nlist_stats()["cells"]
+        e.option("replay_chunk", chunk)
+        e.run(64, flags)
+        st = e.nlist_stats()
+        say(f"  cells {cells} -> {st['cells']}, rebuilds {st['rebuilds']}")
+        assert tuple(cells) == (5, 5, 10) and tuple(st["cells"]) == (4, 4, 9)
+        out.append((*e.get_system(), e.get_box()[1], st["rebuilds"]))
+        e.close()
+    assert out[0][3] == out[1][3]
+    for a, b in zip(out[0][:3], out[1][:3]):
+        assert np.array_equal(a, b)
