@@ -2099,6 +2099,7 @@ int mdx_run(mdx_ctx *ctx, int nsteps, int flags) {
             // the host follows the device box step by step only where the
             // chunk's largest dilation could change the cell grid
             const bool boxSafe = c.baro.on && box_keeps_grid(c, len);
+            bool overflow = false;  // of a build before a grid change
             for (int s = 0; s < len; ++s) {
                 const int par = s & 1;
                 const bool baro = c.baro.on && (c.turn + 1) % c.baro.every == 0;
@@ -2122,6 +2123,10 @@ int mdx_run(mdx_ctx *ctx, int nsteps, int flags) {
                         regrid_if_needed(c);
                     }
                     if (!c.listValid) {
+                        // the build on the new grid makes room for itself and
+                        // starts the row maxima anew: what the chunk's builds
+                        // before it found is taken first
+                        overflow = !capacity_ok(c) || overflow;
                         ensure_list(c);
                         compute(c, fflags);
                         check_step(c, par, false);
@@ -2133,7 +2138,8 @@ int mdx_run(mdx_ctx *ctx, int nsteps, int flags) {
             const bool forced = !forcedDone && c.replayChunk == chunkNo + 1;
             forcedDone = forcedDone || forced;
             if (c.baro.on) box_pull(c);
-            if (!capacity_ok(c) || forced) {
+            overflow = !capacity_ok(c) || overflow;
+            if (overflow || forced) {
                 // a build overflowed its rows: redo the chunk with the grown rows
                 snapshot_restore(c);
                 continue;

@@ -198,3 +198,27 @@ def test_replay_of_a_chunk_with_a_grid_change(gpu_engine_factory):
     assert out[0][3] == out[1][3]
     for a, b in zip(out[0][:3], out[1][:3]):
         assert np.array_equal(a, b)
+
+
+def test_overflow_before_a_grid_change_is_replayed(gpu_engine_factory):
+    """A rebuild overflows its rows, and later in the same chunk the box loses
+    a cell: the build on the new grid makes room by itself, and the chunk is
+    replayed all the same, on the grid it started with."""
+    say("row overflow before a grid change in one chunk")
+    out = []
+    for scale in (2, 1):
+        e, flags, box = shrinking_water(gpu_engine_factory)
+        e.option("graph", 0)
+        cap = tight_rows(e, flags)
+        e.option("row_cap", scale * cap)
+        cells = [e.nlist_stats()["cells"]]
+        e.run(64, flags)
+        st = e.nlist_stats()
+        cells.append(st["cells"])
+        say(f"  rows {scale * cap} -> {st['row_cap']}, cells {cells}, rebuilds {st['rebuilds']}")
+        assert tuple(cells[1]) != tuple(cells[0])
+        out.append((*e.get_system(), e.get_box()[1], st["rebuilds"]))
+        e.close()
+    assert out[0][3] == out[1][3]
+    for a, b in zip(out[0][:3], out[1][:3]):
+        assert np.array_equal(a, b)
