@@ -1850,8 +1850,8 @@ int mdx_e3b_set(mdx_ctx *ctx, int nmol, const int32_t *mol_ids, const double par
         upload(c, E.molIdsOfO, ofO.data(), c.n);
         E.tot = dalloc<float4>(c, nmol);
         E.nlCount = dalloc<int>(c, nmol);
-        E.cap = 64;
-        E.nl = dalloc<int>(c, (size_t)nmol * E.cap);
+        E.cap = 0;  // the rows are made with the first list build, for its density
+        E.nl = nullptr;
         upload(c, E.molIds, ids.data(), nmol);
         fill_int(c, E.atomMolO, c.n, -1);
         MDX_HIP(hipStreamSynchronize(c.stream));
@@ -2754,6 +2754,15 @@ int mdx_option_set(mdx_ctx *ctx, const char *name, int value) {
             dfree(c, c.nl);
             c.cap = value;
             c.nl = dalloc<uint32_t>(c, (size_t)c.n * c.cap);
+            c.listValid = false;
+        }
+        else if (k == "e3b_row_cap") {  // likewise the molecule rows
+            MDX_REQUIRE(value >= 16 && c.e3b.on && c.e3b.nl, MDX_ERR_ARG,
+                        "e3b_row_cap: >= 16, after the first list build with E3B");
+            MDX_HIP(hipStreamSynchronize(c.stream));
+            dfree(c, c.e3b.nl);
+            c.e3b.cap = value;
+            c.e3b.nl = dalloc<int>(c, (size_t)c.e3b.nmol * c.e3b.cap);
             c.listValid = false;
         }
         else throw Error{MDX_ERR_ARG, "unknown option " + k};

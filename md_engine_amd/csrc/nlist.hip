@@ -1479,6 +1479,16 @@ static void run_build(Ctx &c, bool sync) {
         c.waveMax = dalloc<int>(c, needSlots);
         c.waveMaxN = (int)needSlots;
     }
+    if (c.e3b.on && !c.e3b.nl) {
+        // molecule rows for the mean density with the pair rows' margin: water
+        // has 52 entries in 7.2 A, and rows of 64 overflowed now and then in
+        // boxes of a few hundred molecules (each overflow replays a chunk)
+        MDX_REQUIRE(!c.capture, 3, "molecule rows must exist before a step is captured");
+        const double r = (double)c.e3b.r2b + c.skin;
+        const double expect = c.e3b.nmol / (c.geo.L[0] * c.geo.L[1] * c.geo.L[2]) * 4.18879020479 * r * r * r;
+        c.e3b.cap = ((int)(expect * 1.3) + 32 + 15) & ~15;
+        c.e3b.nl = dalloc<int>(c, (size_t)c.e3b.nmol * c.e3b.cap);
+    }
     const int threads = 256;
     const int cur = c.cur, scr = 1 - c.cur;  // the records are sorted in place; scr: scratch copies
     const int nslot = 2 * c.ncell;

@@ -57,7 +57,7 @@ def tight_rows(e, flags):
     return cap
 
 
-@pytest.mark.parametrize("graph,trigger", [(0, "forced"), (1, "forced"), (1, "rows")])
+@pytest.mark.parametrize("graph,trigger", [(0, "forced"), (0, "rows"), (1, "forced"), (1, "rows")])
 def test_overflow_replay_with_nose_hoover_is_exact(gpu_engine_factory, graph, trigger):
     """A replayed chunk that starts with a list carried in from an earlier
     build: the replay builds that list again from the positions and box of
@@ -219,6 +219,58 @@ def test_overflow_before_a_grid_change_is_replayed(gpu_engine_factory):
         assert tuple(cells[1]) != tuple(cells[0])
         out.append((*e.get_system(), e.get_box()[1], st["rebuilds"]))
         e.close()
+    assert out[0][3] == out[1][3]
+    for a, b in zip(out[0][:3], out[1][:3]):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("ensemble", ["rescale", "nose", "npt"])
+@pytest.mark.parametrize("graph", [0, 1])
+def test_overflow_of_molecule_rows_is_exact(gpu_engine_factory, graph, ensemble):
+    """E3B molecule rows exactly as long as the starting list's longest: a
+    rebuild somewhere in a chunk overflows them, also where the chunk's last
+    rebuild fits again, and the replayed chunks equal those of loose rows."""
+    import oracle
+    from test_gpu_water_md import start_velocities, water_md_engine
+
+    say(f"overflow of E3B molecule rows, graph={graph}, {ensemble}")
+    box = systems.tip4p2005_box(441, seed=37, min_sep=1.8)
+    v = start_velocities(oracle, box, seed=8)
+    kb, mvv = systems.REAL_BOLTZ, systems.REAL_MVV_TO_ENG
+
+    def longest(e):
+        L = e.get_box()[1]
+        o = e.get_system()[0][box["mol"][:, 0]]
+        d = o[:, None] - o[None]
+        d -= L * np.rint(d / L)
+        return int(((d ** 2).sum(-1) < 7.2 ** 2).sum(1).max() - 1)
+
+    out, grown = [], 0
+    for kind in ("loose", "tight", "sampled"):
+        e, flags = water_md_engine(gpu_engine_factory, box, v, rc=7.0, skin=1.0, sz=(32, 32, 32), order=5, e3b=True,
+                                   dt=2.0)
+        if ensemble == "nose":
+            e.nose_hoover(True, 298.0, 100.0, 10, kb, mvv)
+        else:
+            e.thermostat(True, 298.0, 10, 0.0, kb, mvv)
+        if ensemble == "npt":
+            e.barostat(True, 1.0, 1000.0, 1, mvv_to_eng=mvv)
+        e.option("graph", graph)
+        e.run(16, flags)
+        most = longest(e)
+        # the next run's first build finds this longest row
+        e.option("e3b_row_cap", most if kind == "tight" else 2 * most)
+        if kind == "sampled":
+            for _ in range(48):
+                e.run(4, flags)
+                grown = max(grown, longest(e))
+        else:
+            for _ in range(3):
+                e.run(64, flags)
+            out.append((*e.get_system(), e.get_box()[1], e.nlist_stats()["rebuilds"]))
+        e.close()
+    say(f"  longest row {most} at the start, {grown} later")
+    assert grown > most, "no row grew past the tight capacity"
     assert out[0][3] == out[1][3]
     for a, b in zip(out[0][:3], out[1][:3]):
         assert np.array_equal(a, b)
