@@ -185,7 +185,11 @@ __device__ __forceinline__ void rigid_vv1_body(int blk, int nblk, RigidArgs r, d
     vH2 = vH2 + idt * (C3 - C1);
     const d3 nO = xO + A3;
     const d3 nH1 = nO + (B3 - A3), nH2 = nO + (C3 - A3);
-    const d3 nM = nO + (0.5 * (1.0 - r.gamma)) * ((B3 - A3) + (C3 - A3));
+    // contracted by hand: one lane and four give a molecule the same bits, so
+    // a batch may take either for all of its replicas
+    const double hM = 0.5 * (1.0 - r.gamma);
+    const d3 tM = (B3 - A3) + (C3 - A3);
+    const d3 nM = mk(fma(hM, tM.x, nO.x), fma(hM, tM.y, nO.y), fma(hM, tM.z, nO.z));
 #pragma unroll
     for (int u = 0; u < 4 / T; ++u) {
         const int k = T == 1 ? u : (int)(threadIdx.x & 3);
