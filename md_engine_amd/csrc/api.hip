@@ -1149,7 +1149,7 @@ void run_captured(const std::vector<Ctx *> &cs, int nsteps, int flags, const Rin
             for (size_t k = 0; k < cs.size(); ++k) {
                 Ctx &c = *cs[k];
                 c.nRebuilds += hs[k][3];
-                if (hs[k][3]) c.listNeed = list_need(c);  // what the graph's builds left
+                if (hs[k][3]) list_built(c);
                 c.turn += len;
                 // the box grew by a cell: the next chunk takes a finer grid
                 if (c.baro.on && regrid_if_needed(c)) regrid = true;

@@ -1156,6 +1156,7 @@ void fill_int(Ctx &c, int *p, int count, int v, const int *gate = nullptr);  // 
 void nlist_rebuild_async(Ctx &c);     // rebuild now; capacity checked later (capacity_ok)
 bool capacity_ok(Ctx &c);             // false: rows grew, results since the last check are invalid
 bool grow_if_needed(Ctx &c);
+void list_built(Ctx &c);              // a build of this set-up ran: what the list holds now
 unsigned long long list_need(Ctx &c); // the parts of the rows the set-up's kernels read
 void nlist_complete(Ctx &c);          // the parts of the rows that no kernel reads, for the whole list's readers
 void list_setup_changed(Ctx &c);      // force terms or charges changed: rows completed if they need more than is built

@@ -1216,7 +1216,7 @@ bool build_shifts(const Ctx &c) {
 }
 
 // with the molecule maps of the rebuild in the same launch, and the E3B list
-void launch_build_wave(Ctx &c, const double4 *bpos, const BoxDev *box, const MolMapArgs &mm) {
+void launch_build_wave(Ctx &c, const double4 *bpos, const BoxDev *box, const MolMapArgs &mm, unsigned long long need) {
     const ExclArgs ex{c.exclOff ? c.maxExcl : 0, c.exclIdx, c.idToIdx};
     OxListArgs ox{};
     if (c.e3b.on) {
@@ -1232,7 +1232,7 @@ void launch_build_wave(Ctx &c, const double4 *bpos, const BoxDev *box, const Mol
         c.waveMaxB = c.e3b.nmol;
     }
     const int blocks = cdiv(c.n, 4);
-#define MDX_BUILD(S, O) launch<build_map_body<S, O>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, ex, c.type[c.cur], c.listNeed, ox, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm)
+#define MDX_BUILD(S, O) launch<build_map_body<S, O>, 256>(c, blocks + mm.blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, ex, c.type[c.cur], need, ox, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax, mm)
     const bool shift = build_shifts(c);
     if (ox.mol) {
         if (shift) MDX_BUILD(true, true); else MDX_BUILD(false, true);
@@ -1244,13 +1244,13 @@ void launch_build_wave(Ctx &c, const double4 *bpos, const BoxDev *box, const Mol
 }
 
 template <int T>
-void launch_build(Ctx &c, const double4 *bpos, const BoxDev *box) {
+void launch_build(Ctx &c, const double4 *bpos, const BoxDev *box, unsigned long long need) {
     const int threads = 256;
     const int blocks = cdiv((long long)c.n * T, threads);
     if (build_shifts(c))
-        launch<build_body<T, true>, 256>(c, blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, c.exclIdx, c.exclOff ? c.maxExcl : 0, c.type[c.cur], c.listNeed, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax);
+        launch<build_body<T, true>, 256>(c, blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, c.exclIdx, c.exclOff ? c.maxExcl : 0, c.type[c.cur], need, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax);
     else
-        launch<build_body<T, false>, 256>(c, blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, c.exclIdx, c.exclOff ? c.maxExcl : 0, c.type[c.cur], c.listNeed, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax);
+        launch<build_body<T, false>, 256>(c, blocks, 0, rebuild_gate(c), c.n, bpos, c.xq, box, c.colRank, c.cellStart, c.ncell, c.rlist * c.rlist, c.exclIdx, c.exclOff ? c.maxExcl : 0, c.type[c.cur], need, c.cap, c.nl, c.nlCount, c.nlCountA, c.dFlags, c.waveMax);
     c.waveMaxA = blocks * (threads / 64);
 }
 
@@ -1387,17 +1387,18 @@ void nlist_check(Ctx &c) {
 // The rows from the sorted atoms at bpos (FP32 copies in xq), and the E3B
 // list; grows them and builds again where they overflowed (sync), else leaves
 // the check to the next synchronisation point.
-static void build_rows(Ctx &c, const double4 *bpos, const BoxDev *box, const MolMapArgs &mm, bool sync, bool wave) {
+static void build_rows(Ctx &c, const double4 *bpos, const BoxDev *box, const MolMapArgs &mm, bool sync, bool wave,
+                       unsigned long long need) {
     for (;;) {
         // the builds of a run keep the running maximum of the chunk in dFlags[1..2]
         if (!c.capture && sync) fill_int(c, c.dFlags + 1, 2, 0);
         c.waveMaxB = 0;
         {
             ProfScope ps(c, PK_BUILD);
-            if (wave) launch_build_wave(c, bpos, box, mm);
-            else if (c.buildTeam == 8) launch_build<8>(c, bpos, box);
-            else if (c.buildTeam == 32) launch_build<32>(c, bpos, box);
-            else launch_build<16>(c, bpos, box);
+            if (wave) launch_build_wave(c, bpos, box, mm, need);
+            else if (c.buildTeam == 8) launch_build<8>(c, bpos, box, need);
+            else if (c.buildTeam == 32) launch_build<32>(c, bpos, box, need);
+            else launch_build<16>(c, bpos, box, need);
         }
         if (c.e3b.on && !wave) {  // the wave build makes this list itself
             switch (c.e3b.listTeam) {
@@ -1460,13 +1461,23 @@ void nlist_complete(Ctx &c) {
     launch<xq_body, 256>(c, cdiv(c.n, 256), 0, c.n, c.posLast, c.q[c.cur], c.xq, c.boxLast);
     c.listNeed = ~0ull;
     // the exclusion rows are as that build's kernel reads them
-    build_rows(c, c.posLast, c.boxLast, MolMapArgs{}, true, !c.exclByIdx);
+    build_rows(c, c.posLast, c.boxLast, MolMapArgs{}, true, !c.exclByIdx, ~0ull);
     refresh_xq(c);
 }
 
 void list_setup_changed(Ctx &c) {
     c.needDirty = true;
     if (c.listValid && !c.centroidList && (list_need(c) & ~c.listNeed)) nlist_complete(c);
+}
+
+static bool wave_build(const Ctx &c) { return c.buildTeam != 8 && c.buildTeam != 16 && c.buildTeam != 32; }
+
+// What a build of the current set-up leaves.  A captured build leaves it only
+// when it runs (run_captured asks the device after the chunk).
+void list_built(Ctx &c) {
+    c.listNeed = list_need(c);
+    c.exclByIdx = !wave_build(c);
+    c.centroidList = c.cenById != nullptr;
 }
 
 static void run_build(Ctx &c, bool sync) {
@@ -1498,7 +1509,7 @@ static void run_build(Ctx &c, bool sync) {
     MDX_REQUIRE(!c.e3b.on || c.rlist >= (double)c.e3b.r2b + c.skin - 1e-9, 1,
                 "E3B needs rCut + padding >= 6.2 A + padding (the molecule list is taken from the "
                 "pair list)");
-    const bool waveBuild = c.buildTeam != 8 && c.buildTeam != 16 && c.buildTeam != 32;
+    const bool waveBuild = wave_build(c);
     const bool excl = c.exclOff && c.maxExcl > 0;
     if (excl) {
         MDX_REQUIRE(!c.capture || c.exclIdxN == (size_t)c.n * c.maxExcl, 3,
@@ -1509,8 +1520,6 @@ static void run_build(Ctx &c, bool sync) {
             c.exclIdx = dalloc<uint32_t>(c, c.exclIdxN);
         }
     }
-    c.centroidList = cen != nullptr;
-    c.exclByIdx = !waveBuild;
     // (the map workgroups of a build clear the chunk counts for the next
     // binning; nothing between the binning and them throws)
     DecideArgs da{};
@@ -1587,9 +1596,9 @@ static void run_build(Ctx &c, bool sync) {
     mm.blocks = cdiv(std::max({mm.nmol, mm.nmolR, mm.nmolF, mm.nchunk}), threads);
     // the wave build takes the maps as extra workgroups; the team builds launch them first
     if (!waveBuild) launch<mol_map_body, 256>(c, mm.blocks, 0, rebuild_gate(c), mm);
-    c.listNeed = list_need(c);
-    build_rows(c, cen ? c.buildPos : c.pos[cur], c.box, mm, sync, waveBuild);
+    build_rows(c, cen ? c.buildPos : c.pos[cur], c.box, mm, sync, waveBuild, list_need(c));
     if (c.capture) return;
+    list_built(c);
     c.nRebuilds++;
     c.listValid = true;
 }

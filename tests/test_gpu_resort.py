@@ -197,3 +197,39 @@ def test_box_turned_on_its_side(orc, gpu_engine_factory):
         oc, orows, _ = oracle_rows_by_id(orc, x, np.zeros(3), L, rlist, brute=True)
         assert_same_lists(gc, grows, oc, orows)
     e.close()
+
+
+@pytest.mark.parametrize("first,then", [(64, 16), (16, 64)])
+def test_list_read_after_a_capture_of_another_build(orc, gpu_engine_factory, first, then):
+    """Wave builds keep the exclusion partners by id, team builds by index.
+    Steps captured for the other kind, none of which built a list, leave the
+    current list's rows as their own build left them: the list read back has
+    the tags of the exclusions."""
+    say(f"list of a {first}-lane build read back after captured steps of {then} lanes")
+    from md_engine_amd import systems
+    from test_gpu_water_md import start_velocities, water_md_engine
+
+    box = systems.tip4p2005_box(343, seed=36, min_sep=1.8)
+    e, flags = water_md_engine(gpu_engine_factory, box, start_velocities(orc, box, seed=9), rc=7.0, skin=1.0,
+                               sz=(32, 32, 32), order=5, e3b=False, dt=0.5)
+    e.teams_set(build=first)
+    # the records in an order of cells, not of ids
+    e.compute(flags)
+    before = e.nlist_stats()["rebuilds"]
+    e.option("graph", 1)
+    e.teams_set(build=then)
+    e.run(2, flags)
+    # the run's start builds anew (rigid molecules placed); the steps do not
+    built = e.nlist_stats()["rebuilds"] - before
+    e.teams_set(build=first)
+    e.nlist_update(force=True)
+    e.teams_set(build=then)
+    x, _ = e.get_system()
+    before = e.nlist_stats()["rebuilds"]
+    e.run(2, flags)
+    assert e.nlist_stats()["rebuilds"] == before and built <= 1
+    gc, grows = e.nlist_get()
+    excl = orc.exclusions_bfs(len(x), systems.water_bonds(box["mol"]))
+    oc, orows, _ = oracle_rows_by_id(orc, x, box["lo"], box["L"], 8.0, excl=excl, brute=False)
+    assert_same_lists(gc, grows, oc, orows)
+    e.close()
