@@ -1208,8 +1208,6 @@ size_t wave_slots_a(const Ctx &c) { return (size_t)c.n + 4; }
 
 // whether every candidate of a run sits in one known image of the stencil
 bool build_shifts(const Ctx &c) {
-    MDX_REQUIRE(std::min(c.nc[0], 2 * c.reach[0] + 1) * std::min(c.nc[1], 2 * c.reach[1] + 1) <= kMaxCols, 1,
-                "stencil wider than the build kernel's column table");
     for (int a = 0; a < 3; ++a)
         if (c.geo.periodic[a] && c.nc[a] < 2 * c.reach[a] + 1) return false;
     return true;
@@ -1509,6 +1507,8 @@ static void run_build(Ctx &c, bool sync) {
     MDX_REQUIRE(!c.e3b.on || c.rlist >= (double)c.e3b.r2b + c.skin - 1e-9, 1,
                 "E3B needs rCut + padding >= 6.2 A + padding (the molecule list is taken from the "
                 "pair list)");
+    MDX_REQUIRE(std::min(c.nc[0], 2 * c.reach[0] + 1) * std::min(c.nc[1], 2 * c.reach[1] + 1) <= kMaxCols, 1,
+                "stencil wider than the build kernel's column table");
     const bool waveBuild = wave_build(c);
     const bool excl = c.exclOff && c.maxExcl > 0;
     if (excl) {
@@ -1520,8 +1520,10 @@ static void run_build(Ctx &c, bool sync) {
             c.exclIdx = dalloc<uint32_t>(c, c.exclIdxN);
         }
     }
-    // (the map workgroups of a build clear the chunk counts for the next
-    // binning; nothing between the binning and them throws)
+    const unsigned long long need = list_need(c);
+    // The map workgroups of a build clear the chunk counts for the next
+    // binning, so every refusal stands above it: counts left over would send
+    // the next sort out of range.
     DecideArgs da{};
     if (c.capture && c.fuseCheck) {
         da = decide_args(c);
@@ -1596,7 +1598,7 @@ static void run_build(Ctx &c, bool sync) {
     mm.blocks = cdiv(std::max({mm.nmol, mm.nmolR, mm.nmolF, mm.nchunk}), threads);
     // the wave build takes the maps as extra workgroups; the team builds launch them first
     if (!waveBuild) launch<mol_map_body, 256>(c, mm.blocks, 0, rebuild_gate(c), mm);
-    build_rows(c, cen ? c.buildPos : c.pos[cur], c.box, mm, sync, waveBuild, list_need(c));
+    build_rows(c, cen ? c.buildPos : c.pos[cur], c.box, mm, sync, waveBuild, need);
     if (c.capture) return;
     list_built(c);
     c.nRebuilds++;
