@@ -713,6 +713,22 @@ hipGraphExec_t capture_merged(const std::vector<Ctx *> &cs, int steps, int fflag
         const std::vector<SavedMesh> &saved;
         ~Restore() { restore_meshes(cs, saved); }
     } restore{cs, saved};
+    Ctx::BatchMost most;
+    for (const Ctx *c : cs) {
+        if (c->rigid.on) most.rigidMol = std::max(most.rigidMol, c->rigid.nmol);
+        if (!c->pppm.on || !pppm_lds_fft(c->pppm)) continue;
+        most.meshPlane = std::max(most.meshPlane, c->pppm.sz[1] * c->pppm.sz[2]);
+        most.meshCols = std::max(most.meshCols, fft_cols(c->pppm));
+    }
+    struct Most {
+        const std::vector<Ctx *> &cs;
+        Most(const std::vector<Ctx *> &cs_, const Ctx::BatchMost &m) : cs(cs_) {
+            for (Ctx *c : cs) c->most = m;
+        }
+        ~Most() {
+            for (Ctx *c : cs) c->most = {};
+        }
+    } mostScope{cs, most};
     RecordOps rec;
     if (ring) {
         for (int s = 0; s < steps; ++s) captured_ring_step(cs, *ring, fflags, rec);

@@ -449,6 +449,12 @@ struct Ctx {
         std::vector<uint64_t> key;
         BatchKeep keep;  // what merged batch launches use: tables, block maps, grouped FFTs
     } graphs;
+    // While a batch records this context's launches: the largest of its
+    // replicas, for the rules that choose a kernel by size (each kernel of a
+    // choice gives the same bits, and one for all keeps the launches merged)
+    struct BatchMost {
+        int rigidMol = 0, meshPlane = 0, meshCols = 0;
+    } most;
     bool batchMerge = true;      // option batch_merge: one launch per kernel across a batch
     int batchMerged = 0;         // the last batch capture merged its replicas' launches (1) or not (0)
     bool vtrace = false;  // set by compute for the terms it launches
@@ -1353,6 +1359,7 @@ void ring_apply(const RingSpec &r, Ctx &c0);
 void ring_pppm(Ctx &c0, const RingSpec &r);
 // the mesh solve of these P3M settings runs as the three LDS passes (no hipFFT)
 bool pppm_lds_fft(const PppmState &P);
+int fft_cols(const PppmState &P);  // column groups of the mesh solve's second pass
 
 // flex.hip: molecule indices after a re-sort, M placement, intramolecular
 // forces and the M force spread onto O, H1, H2

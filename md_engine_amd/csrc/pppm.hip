@@ -1915,6 +1915,8 @@ static size_t lds_fft_shm(const PppmState &P) {
 
 bool pppm_lds_fft(const PppmState &P) { return P.fftMode == 1 && lds_fft_shm(P) > 0; }
 
+int fft_cols(const PppmState &P) { return P.sz[1] * cdiv(P.sz[2] / 2 + 1, kFftWavePts / P.sz[0]); }
+
 // Charge mesh -> the planar real field P.eReal, with the k-space energy and
 // virial when ev is set (and the gate, if any, open).  fromReal: the charges
 // are in P.real (owner spread) instead of the fixed-point mesh.
@@ -1930,8 +1932,9 @@ static void mesh_solve(Ctx &c, bool fromReal, int ev, const int *gate) {
         P.lastFft = 1;
         ProfScope ps(c, PK_FFT);
         const int waves = kFftThreads / 64;
-        const int lw = kFftWavePts / sz[0], cols = sz[1] * ((szh + lw - 1) / lw);
-        const bool all = cols >= kFftAllCols, big = sz[1] * sz[2] > kFftBigPlane;
+        const int cols = fft_cols(P);
+        const bool all = std::max(cols, c.most.meshCols) >= kFftAllCols;
+        const bool big = std::max(sz[1] * sz[2], c.most.meshPlane) > kFftBigPlane;
         const size_t shm2 = sizeof(float2) * (kFftMax + waves * kFftWavePts);
         long long *mesh = fromReal ? nullptr : P.mesh;
         const float *real = fromReal ? P.real : nullptr;

@@ -154,7 +154,8 @@ __device__ __forceinline__ void dist_forces(const unsigned long long *f, int4 a,
 // refresh and check.  T = 4: four lanes do a molecule's SETTLE alike and take a
 // site each after it, while the wider launch still is about one wave a SIMD:
 // 512 molecules 9.8 -> 7.1 us, 4,096 11.6 -> 8.5, 8,192 13.5 -> 10.7, but
-// 32,768 14.7 -> 18.0, which keep one lane a molecule.
+// 32,768 14.7 -> 18.0, which keep one lane a molecule.  A batch goes by its
+// largest replica.
 constexpr int kRigidTeamMax = 16384;
 template <int T>
 __device__ __forceinline__ void rigid_vv1_body(int blk, int nblk, RigidArgs r, double4 *__restrict__ pos, double4 *__restrict__ vel,
@@ -447,7 +448,7 @@ void rigid_first_half(Ctx &c) {
     RefreshArgs ra{};
     if (c.fuseCheck) ra = refresh_args(c);
     unsigned *slots = c.fuseCheck ? c.dispSlots : nullptr;
-    if (r.nmol <= kRigidTeamMax)
+    if (std::max(r.nmol, c.most.rigidMol) <= kRigidTeamMax)
         launch<rigid_vv1_body<4>, 128>(c, cdiv(4 * r.nmol, 128), 0, r, c.pos[c.cur], c.vel[c.cur], c.force, c.posLast, 2.0 * c.dt, slots, ra);
     else
         launch<rigid_vv1_body<1>, 128>(c, cdiv(r.nmol, 128), 0, r, c.pos[c.cur], c.vel[c.cur], c.force, c.posLast, 2.0 * c.dt, slots, ra);
@@ -460,7 +461,7 @@ void rigid_second_half(Ctx &c, bool kick) {
     // last workgroup (the molecular virial and M V^2 are summed here), while
     // its ticket, about 24 ns a workgroup, costs no more than a launch (1.6 us
     // plus the start of a wave)
-    if (kick && c.fuseMolVirial && c.fuseStep && c.baro.on && cdiv(r.nmol, 128) <= 96) {
+    if (kick && c.fuseMolVirial && c.fuseStep && c.baro.on && cdiv(std::max(r.nmol, c.most.rigidMol), 128) <= 96) {
         bf.ticket = c.dFlags + 9;
         bf.gate = baro_gate(c);
         bf.bx = c.box;

@@ -52,3 +52,34 @@ def test_in_place_planes(orc, gpu_engine_factory, sz):
     say(f"force RMSE library {d[0]:.2e}, in place {d[1]:.2e}")
     assert max(d) <= 2.5e-6
     e.close()
+
+
+def test_batch_of_several_meshes(gpu_engine_factory):
+    """Replicas whose meshes lie on both sides of the passes' size rules run
+    the same kernels in a batch: one launch a kernel, and each as alone."""
+    from md_engine_amd import PPPM, run_batch
+    from test_gpu_water_md import water_md_engine
+
+    say("batch of 32^3, 64^3, 64 x 64 x 128 and 128^3 meshes")
+    box = systems.tip4p2005_box(512, seed=15)
+    meshes = [(32, 32, 32), (64, 64, 64), (64, 64, 128), (128, 128, 128)]
+
+    def make(sz):
+        e, _ = water_md_engine(gpu_engine_factory, box, np.zeros_like(box["x"]), rc=7.0, skin=1.0, sz=sz, order=3,
+                               e3b=False, dt=1.0)
+        for k, v in (("graph", 1), ("p3m_spread", 0), ("p3m_gather", 1)):  # whatever the tiles of a mesh hold
+            e.option(k, v)
+        return e
+
+    batch = [make(sz) for sz in meshes]
+    run_batch(batch, 20, PPPM)
+    assert batch[0].batch_merged()
+    for e, sz in zip(batch, meshes):
+        alone = make(sz)
+        alone.run(20, PPPM)
+        assert e.pppm_paths()[2] == alone.pppm_paths()[2] == 1
+        for a, b in zip(e.get_system(), alone.get_system()):
+            assert np.array_equal(a, b), sz
+        alone.close()
+    for e in batch:
+        e.close()

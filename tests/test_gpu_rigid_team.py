@@ -51,3 +51,44 @@ def test_teams_of_four_match_one_lane(orc, gpu_engine_factory):
         x4, v4 = free_molecules(gpu_engine_factory, box, v, nmol, steps)
         assert np.array_equal(x4, x1[: 4 * nmol])
         assert np.array_equal(v4, v1[: 4 * nmol])
+
+
+@pytest.mark.parametrize("sizes,baro", [((33, 16384, 16385), False), ((33, 12288, 12289), True)])
+def test_batch_across_the_lines(orc, gpu_engine_factory, sizes, baro):
+    """A batch with replicas on both sides of a size rule (four lanes or one a
+    molecule; the barostat step within the second half or as launches of its
+    own) takes one side for all of them: one launch a kernel, and each replica
+    as it runs alone."""
+    from md_engine_amd import PAIR, run_batch
+
+    say(f"batch of {sizes} molecules, barostat {baro}")
+    box = systems.tip4p2005_box(max(sizes), seed=1)
+    v = start_velocities(orc, box, seed=4)
+
+    def make(nmol):
+        n, mass = 4 * nmol, box["mass"][: 4 * nmol]
+        e = gpu_engine_factory()
+        e.set_system(box["x"][:n], box["lo"], box["L"], v=v[:n], types=box["type"][:n],
+                     inv_mass=np.where(mass > 0, 1.0 / np.maximum(mass, 1e-30), 0.0))
+        e.exclusions_from_bonds(systems.water_bonds(box["mol"][:nmol]))
+        e.nlist_config(4.0, 1.0)
+        eps24, sig6 = systems.water_lj_tables()
+        e.lj_set(np.full((3, 3), 9.0), eps24, sig6)
+        e.rigid_set(box["mol"][:nmol], G["mO"], G["mH"], G["dOH"], G["dHH"], G["gamma"])
+        e.integrator_set(1.0, systems.REAL_FTM_TO_V)
+        if baro:
+            e.barostat(True, 1.0, 1000.0, 1, mvv_to_eng=systems.REAL_MVV_TO_ENG)
+        e.option("graph", 1)
+        return e
+
+    batch = [make(m) for m in sizes]
+    run_batch(batch, 24, PAIR)
+    assert batch[0].batch_merged()
+    for e, m in zip(batch, sizes):
+        alone = make(m)
+        alone.run(24, PAIR)
+        for a, b in zip((*e.get_system(), e.get_box()[1]), (*alone.get_system(), alone.get_box()[1])):
+            assert np.array_equal(a, b), m
+        alone.close()
+    for e in batch:
+        e.close()
