@@ -213,8 +213,10 @@ int mdx_run(mdx_ctx *ctx, int nsteps, int flags);
  * system) by nsteps with one captured graph per 8 steps that holds all of
  * them.  When the replicas run the same kernels (same force terms and set-up,
  * any sizes) every kernel of a step is ONE launch over all replicas, each
- * workgroup reading its replica's arguments from a table (option
- * "batch_merge" 0 on ctxs[0]: one stream per replica instead).  No
+ * workgroup reading its replica's arguments from a table; replicas that run
+ * other kernels (a box too small for a tiled mesh spread, say) are a class
+ * with launches of their own.  Option "batch_merge" 0 on ctxs[0]: every
+ * replica's launches alone, one replica after the other.  No
  * counterpart in the reference, whose integrator runs one system per
  * process; results per replica equal a single-context captured run bit for
  * bit.  Errors are reported on ctxs[0]. */

@@ -615,14 +615,17 @@ void restore_meshes(const std::vector<Ctx *> &cs, const std::vector<SavedMesh> &
 // stands in for its stream, so a launch that bypassed the launch layer is
 // caught (it lands in that graph) instead of running.
 struct RecordOps : StepOps {
+    // a phase of the contexts that recorded the same kernels (each(), one item
+    // for each such class), or a single operation (one())
     struct Item {
-        bool phase = false;                        // each() (else one())
-        bool merged = false;                       // every context recorded the same kernels
-        std::vector<std::vector<LaunchRec>> recs;  // per context (one() items: one)
+        bool phase = false;
+        std::vector<size_t> who;                   // contexts of the class
+        std::vector<std::vector<LaunchRec>> recs;  // of each
     };
     std::vector<Item> items;
     hipStream_t dummy = nullptr;
     bool stray = false;
+    bool split = false;  // some phase has more than one class
 
     RecordOps() { MDX_HIP(hipStreamCreateWithFlags(&dummy, hipStreamNonBlocking)); }
     ~RecordOps() { hipStreamDestroy(dummy); }
@@ -660,21 +663,30 @@ struct RecordOps : StepOps {
         stray = stray || nodes > 0;
     }
 
+    static bool same(const std::vector<LaunchRec> &a, const std::vector<LaunchRec> &b) {
+        if (a.size() != b.size()) return false;
+        for (size_t i = 0; i < a.size(); ++i)
+            if (a[i].kid != b[i].kid || (!a[i].kid && !a[i].host) || a[i].fft != b[i].fft ||
+                a[i].args.size() != b[i].args.size())
+                return false;
+        return true;
+    }
+
     void each(const std::vector<Ctx *> &cs, const std::function<void(Ctx &)> &f) override {
-        Item it;
-        it.phase = true;
-        it.recs.resize(cs.size());
-        for (size_t k = 0; k < cs.size(); ++k) record(*cs[k], it.recs[k], [&] { f(*cs[k]); });
-        it.merged = true;
-        for (size_t k = 1; k < cs.size() && it.merged; ++k) {
-            it.merged = it.recs[k].size() == it.recs[0].size();
-            for (size_t i = 0; it.merged && i < it.recs[0].size(); ++i)
-                it.merged = it.recs[k][i].kid == it.recs[0][i].kid &&
-                            (it.recs[k][i].kid != nullptr || it.recs[k][i].host) &&
-                            it.recs[k][i].fft == it.recs[0][i].fft &&
-                            it.recs[k][i].args.size() == it.recs[0][i].args.size();
+        const size_t first = items.size();
+        for (size_t k = 0; k < cs.size(); ++k) {
+            std::vector<LaunchRec> r;
+            record(*cs[k], r, [&] { f(*cs[k]); });
+            size_t t = first;
+            while (t < items.size() && !same(items[t].recs[0], r)) ++t;
+            if (t == items.size()) {
+                items.emplace_back();
+                items.back().phase = true;
+            }
+            items[t].who.push_back(k);
+            items[t].recs.push_back(std::move(r));
         }
-        items.push_back(std::move(it));
+        split = split || items.size() > first + 1;
     }
 
     void one(Ctx &c, const std::function<void()> &f) override {
@@ -686,15 +698,16 @@ struct RecordOps : StepOps {
 };
 
 // Captured steps of several contexts with one launch per kernel and phase.
-// The steps are recorded first (RecordOps); each kernel of a merged phase
-// becomes one launch over the concatenated grids of its contexts: an
+// The steps are recorded first (RecordOps); each kernel of a phase becomes
+// one launch over the concatenated grids of the contexts of a class: an
 // argument table (one packed argument set per context) and a block map
 // ((context, block, blocks) per workgroup) in device memory, kept with the
-// graph; single operations and unmerged phases become launches of a
-// one-entry table, in recorded order.  P3M transforms of merged phases run
-// once per group of equal meshes (group_ffts).  Returns nullptr when a launch
-// bypassed the layer, or when a batch's replicas recorded different kernels
-// (the caller then captures them as separate streams).
+// graph; single operations become launches of a one-entry table.  Contexts
+// that recorded other kernels are a class of their own, issued after it on the
+// same stream.  P3M transforms run once per group of equal meshes (group_ffts)
+// where all contexts are of one class, else each on its own.  Returns nullptr
+// when a launch bypassed the layer (the caller then captures the contexts one
+// after the other).
 hipGraphExec_t capture_merged(const std::vector<Ctx *> &cs, int steps, int fflags, BatchKeep &keep,
                               const RingSpec *ring) {
     Ctx &c0 = *cs[0];
@@ -737,11 +750,8 @@ hipGraphExec_t capture_merged(const std::vector<Ctx *> &cs, int steps, int fflag
             for (int s = 0; s < steps; ++s) captured_step(c, fflags);
         });
     }
-    bool allMerged = true;
-    for (const auto &it : rec.items)
-        if (it.phase) allMerged = allMerged && it.merged;
-    c0.batchMerged = !rec.stray && allMerged ? 1 : 0;
-    if (rec.stray || (!ring && !allMerged)) return nullptr;
+    c0.batchMerged = !rec.stray && !rec.split ? 1 : 0;
+    if (rec.stray) return nullptr;
 
     // every launch: its argument table and block map in one device block
     struct Emit {
@@ -755,29 +765,26 @@ hipGraphExec_t capture_merged(const std::vector<Ctx *> &cs, int steps, int fflag
     };
     std::vector<Emit> emits;
     for (const auto &it : rec.items) {
-        if (it.merged && it.recs.size() == R && it.phase) {
+        if (it.phase) {
             for (size_t i = 0; i < it.recs[0].size(); ++i) {
                 Emit e;
                 e.op = &it.recs[0][i];
                 if (e.op->kid) {
-                    for (size_t k = 0; k < R; ++k) e.parts.push_back(&it.recs[k][i]);
-                } else if (e.op->fft) {
-                    e.fftKind = e.op->fft;
-                    for (size_t k = 0; k < R; ++k) e.hosts.push_back(&it.recs[k][i]);
+                    for (const auto &r : it.recs) e.parts.push_back(&r[i]);
                 } else {
-                    for (size_t k = 0; k < R; ++k) e.hosts.push_back(&it.recs[k][i]);
+                    if (e.op->fft && it.who.size() == R) e.fftKind = e.op->fft;
+                    for (const auto &r : it.recs) e.hosts.push_back(&r[i]);
                 }
                 emits.push_back(std::move(e));
             }
         } else {
-            for (const auto &r : it.recs)
-                for (const LaunchRec &op : r) {
-                    Emit e;
-                    e.op = &op;
-                    if (op.kid) e.parts.push_back(&op);
-                    else e.hosts.push_back(&op);
-                    emits.push_back(std::move(e));
-                }
+            for (const LaunchRec &op : it.recs[0]) {
+                Emit e;
+                e.op = &op;
+                if (op.kid) e.parts.push_back(&op);
+                else e.hosts.push_back(&op);
+                emits.push_back(std::move(e));
+            }
         }
     }
     auto align_to = [](size_t v, size_t a) { return (v + a - 1) / a * a; };
@@ -871,59 +878,57 @@ hipGraphExec_t capture_steps(const std::vector<Ctx *> &cs, int steps, int fflags
         hipGraphExec_t merged = capture_merged(cs, steps, fflags, *keep, ring);
         if (merged) return merged;
     }
+    // One stream: the contexts' steps one after the other (a ring's
+    // interleaved step by step), a single context with its mesh stream beside.
+    // A stream per replica ended the host process once (twelve boxes of 343 to
+    // 2,048 molecules, for a cause not found), so no batch takes that way.
     Ctx &c0 = *cs[0];
-    for (Ctx *c : cs)
-        if (c->pppm.on) mesh_stream_make(*c);
-    std::vector<hipEvent_t> evs(cs.size() * 2, nullptr);
-    for (auto &e : evs) MDX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    std::vector<bool> prof(cs.size());
+    const bool alone = cs.size() == 1;
+    if (alone && c0.pppm.on) mesh_stream_make(c0);
+    struct Own {
+        const std::vector<Ctx *> &cs;
+        std::vector<hipStream_t> stream;
+        std::vector<char> prof, mesh;
+        Own(const std::vector<Ctx *> &cs_, bool alone) : cs(cs_) {
+            for (Ctx *c : cs) {
+                stream.push_back(c->stream);
+                prof.push_back(c->prof);
+                mesh.push_back(c->meshStream);
+                c->stream = cs[0]->stream;
+                c->prof = false;
+                c->meshStream = c->meshStream && alone;
+                c->capture = true;
+            }
+        }
+        ~Own() {
+            for (size_t k = 0; k < cs.size(); ++k) {
+                cs[k]->stream = stream[k];
+                cs[k]->prof = prof[k];
+                cs[k]->meshStream = mesh[k];
+                cs[k]->capture = false;
+            }
+        }
+    };
     hipGraph_t graph = nullptr;
     MDX_HIP(hipStreamBeginCapture(c0.stream, hipStreamCaptureModeThreadLocal));
     try {
-        MDX_HIP(hipEventRecord(evs[0], c0.stream));
+        Own own(cs, alone);
+        DirectOps direct;
         if (ring) {
-            // the beads run on c0's stream, interleaved step by step
-            for (size_t k = 0; k < cs.size(); ++k) {
-                prof[k] = cs[k]->prof;
-                cs[k]->prof = false;
-                cs[k]->capture = true;
-            }
-            DirectOps direct;
             for (int s = 0; s < steps; ++s) captured_ring_step(cs, *ring, fflags, direct);
-            for (size_t k = 0; k < cs.size(); ++k) {
-                cs[k]->capture = false;
-                cs[k]->prof = prof[k];
-            }
-        } else
-        for (size_t k = 0; k < cs.size(); ++k) {
-            Ctx &c = *cs[k];
-            if (k) MDX_HIP(hipStreamWaitEvent(c.stream, evs[0], 0));
-            prof[k] = c.prof;
-            c.prof = false;
-            c.capture = true;
-            for (int s = 0; s < steps; ++s) captured_step(c, fflags);
-            c.capture = false;
-            c.prof = prof[k];
-            if (k) {
-                MDX_HIP(hipEventRecord(evs[cs.size() + k], c.stream));
-                MDX_HIP(hipStreamWaitEvent(c0.stream, evs[cs.size() + k], 0));
-            }
+        } else {
+            for (Ctx *c : cs)
+                for (int s = 0; s < steps; ++s) captured_step(*c, fflags);
         }
     } catch (...) {
-        for (size_t k = 0; k < cs.size(); ++k) {
-            cs[k]->capture = false;
-            if (k < prof.size()) cs[k]->prof = prof[k];
-        }
         hipStreamEndCapture(c0.stream, &graph);
         if (graph) hipGraphDestroy(graph);
-        for (auto e : evs) hipEventDestroy(e);
         throw;
     }
     MDX_HIP(hipStreamEndCapture(c0.stream, &graph));
     hipGraphExec_t exec = nullptr;
     const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
     hipGraphDestroy(graph);
-    for (auto e : evs) hipEventDestroy(e);
     MDX_HIP(ie);
     return exec;
 }

@@ -88,8 +88,8 @@ def test_graph_thermostat_turns(orc, gpu_engine_factory):
 @pytest.mark.parametrize("merge", [1, 0])
 def test_batch_equals_single(orc, gpu_engine_factory, merge):
     """Three replicas of different sizes in one graph == each alone, with one
-    launch per kernel across the replicas (merge 1) and with one stream per
-    replica (merge 0)."""
+    launch per kernel across the replicas (merge 1) and with every replica's
+    launches alone (merge 0)."""
     say(f"batched replicas vs single runs (merge {merge})")
     from md_engine_amd import run_batch
 
@@ -118,6 +118,38 @@ def test_batch_equals_single(orc, gpu_engine_factory, merge):
         assert np.array_equal(xb, xs)
         assert np.array_equal(vb, vs)
         assert eb.nlist_stats()["rebuilds"] == es.nlist_stats()["rebuilds"]
+
+
+def test_batch_of_classes_equals_single(orc, gpu_engine_factory):
+    """Replicas that run other kernels than the rest (another charge spread,
+    the library transforms) are classes of their own in the batch's graph; each
+    replica equals its run alone, also on every later call."""
+    say("batch of several classes vs single runs")
+    from md_engine_amd import run_batch
+
+    specs = [(512, 41, None), (512, 42, ("p3m_spread", 0)), (729, 43, None), (512, 44, ("p3m_fft", 0)),
+             (343, 45, ("p3m_fft", 0))]
+    boxes = [systems.tip4p2005_box(m, seed=s, min_sep=1.8) for m, s, _ in specs]
+    vels = [start_velocities(orc, b, seed=s) for b, (_, s, _) in zip(boxes, specs)]
+
+    def make(k):
+        e, flags = water_md_engine(gpu_engine_factory, boxes[k], vels[k], rc=6.5, skin=0.9, sz=(32, 32, 32), order=5,
+                                   e3b=True, dt=2.0)
+        e.option("graph", 1)
+        if specs[k][2]:
+            e.option(*specs[k][2])
+        return e, flags
+
+    batch = [make(k) for k in range(len(specs))]
+    alone = [make(k) for k in range(len(specs))]
+    flags = batch[0][1]
+    for steps in (20, 20, 9):
+        run_batch([e for e, _ in batch], steps, flags)
+        assert not batch[0][0].batch_merged()
+        for (eb, _), (es, _) in zip(batch, alone):
+            es.run(steps, flags)
+            for a, b in zip(eb.get_system(), es.get_system()):
+                assert np.array_equal(a, b)
 
 
 def test_cached_graphs_across_calls(orc, gpu_engine_factory):
