@@ -83,6 +83,25 @@ int guarded_ro(mdx_ctx *ctx, F &&f) {
     }
 }
 
+// An entry point that reads through kernels of its own (packing by id, the
+// list's missing rows): one at a time on a context, on the context's device
+// whatever the calling thread's is.
+struct Reading {
+    std::lock_guard<std::mutex> lock;
+    int was = -1;
+    explicit Reading(Ctx &c) : lock(c.readLock) {
+        int now = c.device;
+        MDX_HIP(hipGetDevice(&now));
+        if (now != c.device) {
+            MDX_HIP(hipSetDevice(c.device));
+            was = now;
+        }
+    }
+    ~Reading() {
+        if (was >= 0) hipSetDevice(was);
+    }
+};
+
 template <class F>
 int guarded(mdx_ctx *ctx, F &&f) {
     if (!ctx) return MDX_ERR_ARG;
@@ -1498,6 +1517,7 @@ int mdx_positions_set(mdx_ctx *ctx, const double *x) {
     return guarded(ctx, [&](Ctx &c) {
         require_system(c);
         MDX_REQUIRE(x, MDX_ERR_ARG, "positions required");
+        Reading reading(c);
         upload(c, c.io, x, 3 * (size_t)c.n);
         unpack_positions(c, c.io);
         MDX_HIP(hipStreamSynchronize(c.stream));
@@ -1508,6 +1528,7 @@ int mdx_positions_set(mdx_ctx *ctx, const double *x) {
 int mdx_system_get(mdx_ctx *ctx, double *x, double *v) {
     return guarded_ro(ctx, [&](Ctx &c) {
         require_system(c);
+        Reading reading(c);
         const size_t m = 3 * (size_t)c.n;
         pack_state(c, x ? c.io : nullptr, v ? c.io + m : nullptr);
         if (x) MDX_HIP(hipMemcpyAsync(x, c.io, sizeof(double) * m, hipMemcpyDeviceToHost, c.stream));
@@ -1645,6 +1666,7 @@ int mdx_nlist_get(mdx_ctx *ctx, int32_t *counts, uint32_t *tagged_ids, int row_c
     return guarded_ro(ctx, [&](Ctx &c) {
         require_system(c);
         MDX_REQUIRE(c.listValid, MDX_ERR_STATE, "no neighbor list built");
+        Reading reading(c);
         nlist_complete(c);
         if (!c.wholeList) {
             c.wholeList = true;
@@ -2031,6 +2053,7 @@ int mdx_forces_get(mdx_ctx *ctx, double *f) {
     return guarded_ro(ctx, [&](Ctx &c) {
         require_system(c);
         MDX_REQUIRE(f, MDX_ERR_ARG, "output required");
+        Reading reading(c);
         pack_forces(c, c.io);
         MDX_HIP(hipMemcpyAsync(f, c.io, sizeof(double) * 3 * (size_t)c.n, hipMemcpyDeviceToHost, c.stream));
         MDX_HIP(hipStreamSynchronize(c.stream));
@@ -2644,6 +2667,7 @@ int mdx_nlist_totals(mdx_ctx *ctx, int64_t *pair_entries, int64_t *mol_entries) 
     return guarded_ro(ctx, [&](Ctx &c) {
         require_system(c);
         MDX_REQUIRE(c.listValid, MDX_ERR_STATE, "no neighbor list built");
+        Reading reading(c);
         nlist_complete(c);
         std::vector<int> cnt(c.n);
         MDX_HIP(hipMemcpyAsync(cnt.data(), c.nlCount, sizeof(int) * c.n, hipMemcpyDeviceToHost, c.stream));

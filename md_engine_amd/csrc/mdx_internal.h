@@ -18,6 +18,7 @@
 #include <cstdint>
 #include <string>
 #include <cmath>
+#include <mutex>
 #include <numeric>
 #include <vector>
 
@@ -481,6 +482,7 @@ struct Ctx {
     int cur = 0;
     int *idToIdx = nullptr;
     double *io = nullptr;                  // 6 n: staging of the boundary's n x 3 arrays
+    std::mutex readLock;                   // held by the entry points that stage in io or complete the list's rows
     float4 *xq = nullptr;
     float4 *meshRec = nullptr;             // per charged site: mesh offsets and point (mesh_record)
     unsigned long long *force = nullptr;   // 3 per atom
