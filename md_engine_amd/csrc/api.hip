@@ -367,7 +367,9 @@ void snapshot_restore(Ctx &c) {
         c.geo = c.snap.geo;
         nlist_setup(c, c.snap.nc);
     }
-    const bool relist = c.snap.listValid && c.nlistConfigured;
+    // A ring's list was built on centroids that are gone (the ring's table
+    // holds later ones): ring_lists builds one from the chunk's first positions.
+    const bool relist = c.snap.listValid && c.nlistConfigured && !c.cenById;
     if (relist) {
         // Build the chunk's starting list again from the positions and box of
         // its build: the records are already in that build's order, so the

@@ -268,3 +268,31 @@ def test_ring_merged_launches_equal_separate(orc, gpu_engine_factory, mode):
     for (xa, va), (xb, vb) in zip(out[0], out[1]):
         assert np.array_equal(xa, xb)
         assert np.array_equal(va, vb)
+
+
+@pytest.mark.parametrize("mode", ["contracted", "per-bead", "bead-lists"])
+def test_ring_replay_with_a_carried_list(orc, gpu_engine_factory, mode):
+    """The first chunk of a second call replayed: the list it was entered with
+    belongs to an earlier call.  A list of each bead's own positions is built
+    again as it was (bit for bit); a centroid list is built from the chunk's
+    first positions, whose rows come in another order (FP32 sums: some 1e-7 A
+    after 64 steps of 0.5 fs)."""
+    say(f"ring replay with a carried list, {mode}")
+    P = 4
+    box = systems.tip4p2005_box(64, seed=33, min_sep=1.8)
+    xs = bead_systems(box, P, 5, spread=0.02)
+    vs = [start_velocities(orc, dict(box, x=x), seed=20 + k) for k, x in enumerate(xs)]
+    wP = ring_omega(P * 298.0, systems.REAL_BOLTZ, systems.REAL_HBAR)
+    out = []
+    for chunk in (0, 1):
+        es, flags = ring_engines(gpu_engine_factory, box, xs, vs, dt=0.5)
+        run_flags = flags | {"contracted": 0, "per-bead": PPPM_PER_BEAD, "bead-lists": RING_BEAD_LISTS}[mode]
+        run_ring(es, 64, run_flags, wP)
+        es[0].option("replay_chunk", chunk)
+        run_ring(es, 64, run_flags, wP)
+        out.append([e.get_system() for e in es])
+        for e in es:
+            e.close()
+    dx = max(np.abs(a[0] - b[0]).max() for a, b in zip(*out))
+    say(f"  max |dx| {dx:.1e}")
+    assert dx == 0.0 if mode == "bead-lists" else dx < 1e-5
