@@ -112,8 +112,8 @@ int mdx_pppm_info(mdx_ctx *ctx, double *alpha, double *rms_error);
  * for tests and benchmarks): spread 2 owner-computes cell blocks, 1 LDS tiles
  * with global atomics, 0 global atomics; gather 2 LDS field tiles, 1 row
  * teams from the per-site mesh records, 0 row teams from the positions; fft
- * 1 the mesh solve in three LDS passes (power-of-two meshes whose planes fit
- * a workgroup), 0 hipFFT with separate field and conversion kernels; -1
+ * 1 the mesh solve in three LDS passes (axes of 32, 64 and 128 points, at
+ * least 64 planes where one holds over 4,096), 0 hipFFT with separate field and conversion kernels; -1
  * before any evaluation.  Any pointer may be NULL. */
 int mdx_pppm_paths(mdx_ctx *ctx, int *spread, int *gather, int *fft);
 /* Error mode (FixChargeEwald::setError + setGridToErrorTolerance,
@@ -365,12 +365,12 @@ int mdx_sync(mdx_ctx *ctx);
  * columns cut the halo points but halve the workgroups: measured slower
  * here; identical forces); "p3m_fft" 1 (default) solves the mesh
  * in three hand-written passes (FFTs in LDS with the charge conversion, the
- * field and the k-space energy and virial fused; power-of-two meshes whose
- * planes fit a workgroup, else hipFFT), 0 hipFFT with separate conversion and
+ * field and the k-space energy and virial fused; axes of 32, 64 and 128
+ * points, at least 64 planes where one holds over 4,096, else hipFFT), 0 hipFFT with separate conversion and
  * field kernels (forces equal to FP32 rounding); "mesh_stream" 1 (default) runs the
  * P3M chain of a captured step on a second stream beside the pair and E3B
- * kernels, 0 on one stream (identical trajectories); "graph" 1 (default)
- * runs mdx_run as captured 8-step graphs, 0 eagerly; "build_mode" 0 or 2
+ * kernels, 0 on one stream (identical trajectories); "graph" 1
+ * runs mdx_run as captured 8-step graphs, 0 (default) eagerly; "build_mode" 0 or 2
  * (both the per-atom team build); "cell_reach_xy" 1..2 and "cell_reach_z"
  * 1..16: cell edges >= rlist / reach per axis (identical lists, finer cells
  * test fewer candidates); "gather_team" 8 or 16 lanes per charged atom in

@@ -232,7 +232,7 @@ void compute(Ctx &c, int flags) {
     // step, 16,384 145 -> 167, 32,768 210 -> 209, 131,072 544 -> 501).
     const bool eagerFork = c.inRun && !c.prof && c.n >= kForkSites;
     const bool fork = mesh && (c.capture || eagerFork) && !c.rec && c.side && c.meshStream;
-    const bool forked = c.forked;  // recorded by this step's rebuild after its copy-back
+    const bool forked = c.forked;  // recorded by this step's rebuild after its sort
     c.forked = false;
     if (fork) {
         if (!forked) MDX_HIP(hipEventRecord(c.evFork, c.stream));
@@ -449,7 +449,7 @@ constexpr int kGraphChunk = 64;
 void captured_step(Ctx &c, int fflags) {
     // all-water systems without a Nose-Hoover chain: the rigid second half
     // sums the molecular virial terms and the thermostat's m v^2 (no separate
-    // passes over the molecules; k_decide clears the m v^2 sum)
+    // passes over the molecules; the step's decisions clear the m v^2 sum)
     c.fuseMolVirial = c.baro.on && all_rigid(c);
     c.fuseThermo = c.thermoOn && all_rigid(c);
     c.fuseCheck = fuses_check(c);
@@ -1046,7 +1046,7 @@ void run_captured(const std::vector<Ctx *> &cs, int nsteps, int flags, const Rin
     }
     // Without a ring, the step graphs stay with the first context after the
     // call: the next call replays them as long as nothing they bake in (the
-    // contexts, their set-up, buffers, cell grid, buffer parity, the force
+    // contexts, their set-up, buffers, cell grid, the force
     // terms) changed.  A ring's bead table is made per call.
     Ctx::GraphCache *cache = ring ? nullptr : &cs[0]->graphs;
     hipGraphExec_t big = nullptr, one = nullptr;
@@ -1056,7 +1056,6 @@ void run_captured(const std::vector<Ctx *> &cs, int nsteps, int flags, const Rin
         big = cache->big;
         one = cache->one;
     }
-    std::vector<int> ringCur;
     auto drop = [&] {
         if (big) hipGraphExecDestroy(big);
         if (one) hipGraphExecDestroy(one);
@@ -1077,7 +1076,6 @@ void run_captured(const std::vector<Ctx *> &cs, int nsteps, int flags, const Rin
             k.push_back(cp->serial);
             k.push_back(cp->apiEpoch);
             k.push_back(cp->layoutEpoch);
-            k.push_back((uint64_t)cp->cur);
         }
         return k;
     };
@@ -1115,12 +1113,6 @@ void run_captured(const std::vector<Ctx *> &cs, int nsteps, int flags, const Rin
                 if (cp != cs[0]) stream_after(cs[0]->stream, c.stream);
             }
             if (ring) {
-                // a bead's buffers may have flipped in the set-up above: a new
-                // table and new graphs
-                std::vector<int> curs;
-                for (Ctx *cp : cs) curs.push_back(cp->cur);
-                if (curs != ringCur) drop();
-                ringCur = curs;
                 ring_table(cs, *ring);
                 if (ringStale) {
                     ring_forces(cs, *ring, fflags);

@@ -479,7 +479,7 @@ struct Ctx {
     float *q[2] = {nullptr, nullptr};
     int *type[2] = {nullptr, nullptr};
     int *id[2] = {nullptr, nullptr};
-    int cur = 0;
+    int cur = 0;                           // the records; a re-sort copies them to the other half and back
     int *idToIdx = nullptr;
     double *io = nullptr;                  // 6 n: staging of the boundary's n x 3 arrays
     std::mutex readLock;                   // held by the entry points that stage in io or complete the list's rows
@@ -528,14 +528,14 @@ struct Ctx {
     // [3] rebuild gate, [4] rebuilds, [5] thermostat gate, [6] turn;
     // [7] bit 0: an atom's candidate stream overflowed the build table, bit 1:
     // a charged site's P3M stencil left the cells next to its own;
-    // [8] barostat gate; [10] last-workgroup ticket of the first half kick
+    // [8] barostat gate; [9] last-workgroup ticket of the second half kick
     int *dFlags = nullptr;
     int *waveMax = nullptr;       // per-wave longest rows: [0, n + 4) pair list, then the molecule list
     int waveMaxN = 0, waveMaxA = 0, waveMaxB = 0;
     bool capture = false;         // a step is being recorded into a graph
     bool rowMaxPending = false;   // a captured build's row maxima go with the next position refresh
     bool refreshed = false;       // ... and refreshed xq, the mesh records, forces and accumulators
-    bool forked = false;          // the captured rebuild recorded the mesh stream's fork after its copy-back
+    bool forked = false;          // the captured rebuild recorded the mesh stream's fork after its sort
     bool baroFused = false;       // the rigid second half of this captured step ran the barostat step
     bool fuseStep = true;         // option "fuse_step": captured steps fold small launches into others
     int graphSteps = 0;           // mdx_run: 1 = captured steps (option "graph")

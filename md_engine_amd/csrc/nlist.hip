@@ -1326,7 +1326,7 @@ void nlist_setup(Ctx &c, const int *cells) {
         c.chunkSum = dalloc<int>(c, 2048);
         MDX_HIP(hipMemsetAsync(c.chunkSum, 0, sizeof(int) * 2048, c.stream));
     }
-    // one wave per atom (k_build_wave) measured fastest for dense water and
+    // one wave per atom (build_wave_body) measured fastest for dense water and
     // LJ alike; mdx_tune revisits the width
     if (!c.buildTeamUser) c.buildTeam = 64;
     const double dens = c.n / (c.geo.L[0] * c.geo.L[1] * c.geo.L[2]);

@@ -1900,9 +1900,11 @@ constexpr int kFftBigPlane = 4096;
 constexpr int kFftAllCols = 1024;
 
 // LDS bytes of passes 1 and 3 of the mesh solve, 0 where the mesh takes the
-// library transforms: every axis must be 32, 64 or 128, and
-// there must be at least 64 planes if they are large (one workgroup each: with
-// fewer most CUs idle through pass 1).  Pass 2 takes kFftMax + kFftWavePts
+// library transforms: every axis must be 32, 64 or 128 (the entry points take
+// nothing shorter), and meshes of fewer than 64 large planes stay with the
+// library, as they did while a plane took three LDS copies: the library path's
+// own test runs 32 x 64 x 128, where the passes measured faster (32 us against
+// 48).  Pass 2 takes kFftMax + kFftWavePts
 // points per wave.
 static size_t lds_fft_shm(const PppmState &P) {
     for (int a = 0; a < 3; ++a) {

@@ -219,8 +219,8 @@ __device__ __forceinline__ void rigid_vv1_body(int blk, int nblk, RigidArgs r, d
 // kick = false: only the velocity constraint and the M placement (start of a run)
 // SUMS: on the steps their gates allow, also (doVir) the molecular virial
 // correction and centre-of-mass M|V|^2 of the final velocities (as
-// k_mol_virial) into acc[ACC_MOL], the barostat's pressure without a pass of
-// its own, and (doTh) the sum of m v^2 over the sites (as k_mv2) into
+// molecular_virial) into acc[ACC_MOL], the barostat's pressure without a pass of
+// its own, and (doTh) the sum of m v^2 over the sites (as mv2_body) into
 // thermo[0] for the velocity rescale.
 // the barostat step for the last workgroup of the rigid second half
 // (ticket = nullptr: none)

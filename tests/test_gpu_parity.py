@@ -306,7 +306,7 @@ def test_mesh_solve_paths(orc, gpu_engine_factory, sz):
     """The mesh solve in three LDS passes (real FFT along z two rows at a time,
     complex FFTs along y and x, the field and the k-space energy and virial
     beside rho_hat, the inverse likewise) against the FP64 oracle's P3M and
-    against the hipFFT path; a mesh whose planes do not fit a workgroup's LDS
+    against the hipFFT path; a mesh of fewer than 64 large planes
     (32 x 64 x 128) takes the hipFFT path."""
     say(f"mesh solve paths, mesh {sz}")
     from md_engine_amd._lib import ENERGY, PPPM, VIRIAL

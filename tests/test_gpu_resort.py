@@ -6,8 +6,10 @@ wrong, through the neighbor list it leaves: rows against the oracle bit for bit.
 * a grid with fewer cells than one chunk, and one with several rounds per chunk
   (a sparse gas over hundreds of thousands of cell slots);
 * exclusion rows longer than a wave's registers;
-* captured steps of free atoms (first half kick, binning and decisions fused)
-  against the separate launches, bit for bit.
+* steps of free atoms (first half kick, check and refresh fused; captured: the
+  decisions in the binning) against the separate launches, bit for bit;
+* what a list read back depends on: parts left out, captured builds that did
+  not run, a box turned on its side.
 """
 import numpy as np
 import pytest
@@ -87,11 +89,13 @@ def test_long_exclusion_rows(orc, gpu_engine_factory):
     e.close()
 
 
+@pytest.mark.parametrize("graph", [0, 1])
 @pytest.mark.parametrize("n", [256, 257, 4000])
-def test_fused_first_half_equals_separate(orc, gpu_engine_factory, n):
-    """Free atoms, captured steps: kick, check, decisions and refresh in one
-    launch give the separate launches' trajectory bit for bit."""
-    say(f"fused first half, {n} atoms")
+def test_fused_first_half_equals_separate(orc, gpu_engine_factory, n, graph):
+    """Free atoms, eager and captured steps: kick, check and refresh in one
+    launch (captured: the decisions in the binning) give the separate
+    launches' trajectory bit for bit."""
+    say(f"fused first half, {n} atoms, graph {graph}")
     from md_engine_amd import systems
 
     x, L, lo = systems.fcc_lj(10, 0.8442)
@@ -105,6 +109,7 @@ def test_fused_first_half_equals_separate(orc, gpu_engine_factory, n):
         e.nlist_config(2.8, 0.3)
         e.integrator_set(0.005, 1.0)
         e.option("fuse_step", fuse)
+        e.option("graph", graph)
         e.run(150, PAIR)
         st = e.nlist_stats()
         out.append((*e.get_system(), st["rebuilds"], st["violations"]))
