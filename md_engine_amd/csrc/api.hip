@@ -262,6 +262,7 @@ void compute(Ctx &c, int flags) {
         if (!c.deferMSpread) flex_spread_m(c);  // every term's M force goes onto O and H before the kick
     }
     c.forceFlags = flags & kForceTerms;
+    c.dilated = false;
 }
 
 void prepare_terms(Ctx &c) {
@@ -305,13 +306,17 @@ void snapshot_save(Ctx &c) {
         MDX_HIP(hipMemcpyAsync(c.snap.posLast, c.posLast, sizeof(double4) * c.n, hipMemcpyDeviceToDevice,
                                c.stream));
         MDX_HIP(hipMemcpyAsync(c.snap.boxLast, c.boxLast, sizeof(BoxDev), hipMemcpyDeviceToDevice, c.stream));
-        // Forces carried into the chunk belong to the positions before the
-        // last step's dilation: the replay takes these, as the chunk did.
+    }
+    // Where a barostat dilated the sites after the last forces, or the mesh part
+    // is a stored one, forces carried into the chunk cannot be computed again:
+    // the replay takes these, as the chunk did.
+    c.snap.forceFlags = -1;
+    if (c.snap.listValid && (c.dilated || (c.pppm.on && c.pppm.interval > 1))) {
         if (!c.snap.force) c.snap.force = dalloc<unsigned long long>(c, 3 * (size_t)c.n);
         MDX_HIP(hipMemcpyAsync(c.snap.force, c.force, sizeof(unsigned long long) * 3 * c.n, hipMemcpyDeviceToDevice,
                                c.stream));
+        c.snap.forceFlags = c.forceFlags;
     }
-    c.snap.forceFlags = c.snap.listValid ? c.forceFlags : -1;
     if (c.box) {
         if (!c.snap.box) c.snap.box = dalloc<BoxDev>(c, 1);
         MDX_HIP(hipMemcpyAsync(c.snap.box, c.box, sizeof(BoxDev), hipMemcpyDeviceToDevice, c.stream));
@@ -384,10 +389,14 @@ void snapshot_restore(Ctx &c) {
         MDX_HIP(hipMemcpyAsync(c.box, c.snap.box, sizeof(BoxDev), hipMemcpyDeviceToDevice, c.stream));
         box_pull(c);
         refresh_xq(c);
+    }
+    c.forceFlags = -1;
+    if (relist && c.snap.forceFlags >= 0) {
         MDX_HIP(hipMemcpyAsync(c.force, c.snap.force, sizeof(unsigned long long) * 3 * c.n, hipMemcpyDeviceToDevice,
                                c.stream));
+        c.forceFlags = c.snap.forceFlags;
+        c.dilated = true;
     }
-    c.forceFlags = relist ? c.snap.forceFlags : -1;
     c.nRebuilds = c.snap.rebuilds;
     bool moved = false;
     for (int d = 0; d < 3; ++d) moved = moved || c.snap.geo.L[d] != c.geo.L[d] || c.snap.geo.lo[d] != c.geo.lo[d];
@@ -1185,6 +1194,7 @@ void run_captured(const std::vector<Ctx *> &cs, int nsteps, int flags, const Rin
                 c.nRebuilds += hs[k][3];
                 if (hs[k][3]) list_built(c);
                 c.turn += len;
+                c.dilated = c.baro.on;
                 // the box grew by a cell: the next chunk takes a finer grid
                 if (c.baro.on && regrid_if_needed(c)) regrid = true;
             }
@@ -2156,6 +2166,7 @@ int mdx_run(mdx_ctx *ctx, int nsteps, int flags) {
                 if (thermo) thermostat_apply(c);
                 if (baro) {
                     baro_step(c, nullptr);
+                    c.dilated = true;
                     if (!boxSafe) {
                         box_pull(c);
                         regrid_if_needed(c);

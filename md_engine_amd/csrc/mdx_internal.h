@@ -534,7 +534,8 @@ struct Ctx {
     int waveMaxN = 0, waveMaxA = 0, waveMaxB = 0;
     bool capture = false;         // a step is being recorded into a graph
     bool rowMaxPending = false;   // a captured build's row maxima go with the next position refresh
-    bool refreshed = false;       // ... and refreshed xq, the mesh records, forces and accumulators
+    bool dilated = false;         // a barostat moved the sites after the forces were computed
+    bool refreshed = false;       // the first half kick refreshed xq, the mesh records, forces and accumulators
     bool forked = false;          // the captured rebuild recorded the mesh stream's fork after its sort
     bool baroFused = false;       // the rigid second half of this captured step ran the barostat step
     bool fuseStep = true;         // option "fuse_step": captured steps fold small launches into others

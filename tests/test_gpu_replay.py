@@ -274,3 +274,38 @@ def test_overflow_of_molecule_rows_is_exact(gpu_engine_factory, graph, ensemble)
     assert out[0][3] == out[1][3]
     for a, b in zip(out[0][:3], out[1][:3]):
         assert np.array_equal(a, b)
+
+
+def test_replay_after_the_barostat_was_switched_off(gpu_engine_factory):
+    """The forces carried into a constant-volume run are still those before
+    the barostat's last dilation."""
+    say("replay after the barostat was switched off")
+    out = []
+    for chunk in (0, 1):
+        e, flags = water(gpu_engine_factory, 343, 33, nh=False)
+        e.barostat(True, 1.0, 100.0, 1, 10.0, 1e-4, mvv_to_eng=systems.REAL_MVV_TO_ENG)
+        e.run(20, flags)
+        e.barostat(False)
+        e.option("replay_chunk", chunk)
+        e.run(40, flags)
+        out.append(e.get_system())
+        e.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+def test_replay_with_a_long_range_interval(gpu_engine_factory):
+    """Between the steps that evaluate the mesh its stored forces are added:
+    a chunk entered in between is replayed from the forces it was entered with."""
+    say("replay with a long-range interval")
+    out = []
+    for chunk in (0, 1):
+        e, flags = water(gpu_engine_factory, 343, 33, nh=False)
+        e.pppm_interval(3)
+        e.run(20, flags)
+        e.option("replay_chunk", chunk)
+        e.run(40, flags)
+        out.append(e.get_system())
+        e.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
