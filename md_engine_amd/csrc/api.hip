@@ -1858,14 +1858,6 @@ int mdx_e3b_set(mdx_ctx *ctx, int nmol, const int32_t *mol_ids, const double par
         require_system(c);
         MDX_REQUIRE(nmol > 0 && mol_ids && params, MDX_ERR_ARG, "molecules and parameters required");
         E3BState &E = c.e3b;
-        if (E.molIds) {
-            dfree(c, E.molIds);
-            dfree(c, E.molAtoms);
-            dfree(c, E.atomMolO);
-            dfree(c, E.nl);
-            dfree(c, E.nlCount);
-            dfree(c, E.tot);
-        }
         std::vector<int4> ids(nmol);
         std::vector<int> seen(c.n, 0);
         for (int m = 0; m < nmol; ++m) {
@@ -1875,6 +1867,14 @@ int mdx_e3b_set(mdx_ctx *ctx, int nmol, const int32_t *mol_ids, const double par
                 MDX_REQUIRE(a >= 0 && a < c.n, MDX_ERR_ARG, "E3B molecule id out of range");
                 MDX_REQUIRE(!seen[a]++, MDX_ERR_ARG, "atom listed in two E3B molecules");
             }
+        }
+        if (E.molIds) {
+            dfree(c, E.molIds);
+            dfree(c, E.molAtoms);
+            dfree(c, E.atomMolO);
+            dfree(c, E.nl);
+            dfree(c, E.nlCount);
+            dfree(c, E.tot);
         }
         E.on = true;
         E.nmol = nmol;
@@ -1918,11 +1918,6 @@ int mdx_rigid_set(mdx_ctx *ctx, int nmol, const int32_t *mol_ids, double m_O, do
         MDX_REQUIRE(m_O > 0 && m_H > 0 && d_OH > 0 && d_HH > 0 && d_HH < 2 * d_OH, MDX_ERR_ARG,
                     "invalid rigid water geometry");
         RigidState &R = c.rigid;
-        if (R.ids) {
-            dfree(c, R.ids);
-            dfree(c, R.atoms);
-            dfree(c, R.member);
-        }
         std::vector<int4> ids(nmol);
         std::vector<int> seen(c.n, 0);
         for (int m = 0; m < nmol; ++m) {
@@ -1939,6 +1934,11 @@ int mdx_rigid_set(mdx_ctx *ctx, int nmol, const int32_t *mol_ids, double m_O, do
                         "ids of a rigid water must be ordered O, H1, H2, M");
             if (p[3] >= 0) MDX_REQUIRE(c.invMassHost[p[3]] == 0.0, MDX_ERR_ARG, "M site must be massless");
             ids[m] = make_int4(p[0], p[1], p[2], p[3]);
+        }
+        if (R.ids) {
+            dfree(c, R.ids);
+            dfree(c, R.atoms);
+            dfree(c, R.member);
         }
         R.on = true;
         R.fresh = true;
@@ -1968,10 +1968,6 @@ int mdx_flexible_water_set(mdx_ctx *ctx, int nmol, const int32_t *mol_ids, doubl
         MDX_REQUIRE(r0 > 0 && theta0 > 0 && theta0 < M_PI && gamma > 0 && gamma <= 1, MDX_ERR_ARG,
                     "invalid flexible water parameters");
         FlexState &F = c.flex;
-        if (F.ids) {
-            dfree(c, F.ids);
-            dfree(c, F.atoms);
-        }
         std::vector<int4> ids(nmol);
         std::vector<int> seen(c.n, 0);
         for (int m = 0; m < nmol; ++m) {
@@ -1986,6 +1982,10 @@ int mdx_flexible_water_set(mdx_ctx *ctx, int nmol, const int32_t *mol_ids, doubl
                 MDX_REQUIRE(c.invMassHost[p[3]] == 0.0, MDX_ERR_ARG, "M site must be massless");
             }
             ids[m] = make_int4(p[0], p[1], p[2], p[3]);
+        }
+        if (F.ids) {
+            dfree(c, F.ids);
+            dfree(c, F.atoms);
         }
         F.on = true;
         F.nmol = nmol;

@@ -204,3 +204,44 @@ def test_nose_hoover_chain_matches_oracle(orc, gpu_engine_factory, graph):
         assert err < 1e-4, (name, err)
     assert st[40] == pytest.approx(so[40], rel=1e-5)
     assert st[41] == pytest.approx(so[41], rel=1e-9)
+
+
+@pytest.mark.parametrize("kind", ["rigid", "flexible"])
+def test_refused_molecules_leave_the_set_up(orc, gpu_engine_factory, kind):
+    """Molecules that a setter refuses (an id out of range, an atom in two
+    molecules) leave the molecules set before as they were."""
+    say(f"refused molecules, {kind}")
+    box = systems.tip4p2005_box(216, seed=21, min_sep=1.8)
+    v = start_velocities(orc, box)
+    mol = box["mol"]
+    far, twice = mol.copy(), mol.copy()
+    far[7, 1] = 4 * 216
+    twice[9] = twice[8]
+    p = systems.QTIP4PF
+    flex = (p["k2"], p["k3"], p["k4"], p["r0"], p["ktheta"], p["theta0"], p["gamma"])
+    out = []
+    for refuse in (False, True):
+        if kind == "flexible":
+            from test_gpu_flex import flex_engine
+
+            e, flags = flex_engine(gpu_engine_factory, box, v)
+        else:
+            e, flags = water_md_engine(gpu_engine_factory, box, v, rc=7.0, skin=1.0, sz=(32, 32, 32), order=5,
+                                       e3b=True, dt=0.5)
+        e.run(3, flags)
+        if refuse:
+            for bad in (far, twice):
+                with pytest.raises(RuntimeError):
+                    if kind == "rigid":
+                        e.rigid_set(bad, G["mO"], G["mH"], G["dOH"], G["dHH"], G["gamma"])
+                    else:
+                        e.flexible_water_set(bad, *flex)
+                if kind == "rigid":
+                    k = 0.23900573614
+                    with pytest.raises(RuntimeError):
+                        e.e3b_set(bad, [453000 * k, 150 * k, -1005 * k, 1880 * k, 4.872, 1.907, 5.0, 5.2])
+        e.run(40, flags)
+        out.append(e.get_system())
+        e.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
